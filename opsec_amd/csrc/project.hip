@@ -2,13 +2,13 @@
 //
 // Replaces the comma band loop (src/comma-scalapack.cpp:228-266): per band
 // p, fill S_p, C = S_p B (pdgemm), P = B^T C (pdgemm), write the packed upper
-// triangle.  Here every band runs in one batched launch per stage (grid.z =
-// band) and S_p is never stored:
-//   stage 1  C_p = T_p B'      T_p[a][b] = Q_p[key(a,b)] generated in the A
-//                              loader, B' = diag(sqrt(Nbar)) B (once per upload)
-//   stage 2  P_p = B'^T C_p    upper-triangle tiles only, written packed
+// triangle.  Here, for several bands per launch:
+//   stage 1  C_p = T_p B'      T_p[a][b] = Q_p[key(a,b)], written a panel of rows
+//                              at a time; B' = diag(sqrt(Nbar)) B (once per upload)
+//   stage 2  P_p = B'^T C_p    one triangle's tiles only, written packed
 //                              (column j holds rows 0..j: the covfile layout).
-// Precisions: FP64 (v_mfma_f64_16x16x4f64), FP32 (v_mfma_f32_16x16x4f32) and
+// Precisions: FP64 (v_mfma_f64_16x16x4f64) and FP32 (v_mfma_f32_16x16x4f32), both
+// on nt_gemm_kernel, and
 // split-BF16x3 (x = hi + lo in bf16, hi*hi + hi*lo + lo*hi on
 // v_mfma_f32_16x16x32_bf16 with FP32 accumulation).
 //
@@ -27,12 +27,13 @@
 
 #include "common.h"
 #include "gemm.h"
+#include "nt_gemm.h"
 
 namespace opsec {
 
 struct ProjState {
     double* d_Bw = nullptr;      // B' = diag(sqrt(Nbar)) B, ncells x nmodes column-major, pitch ldw
-    size_t ldw = 0;              // ncells + 32 (a power-of-two pitch aliases L2 sets and HBM channels)
+    size_t ldw = 0;              // nt_pitch(ncells); columns from ncells on are zero
     size_t cap_Bw = 0;
     void* d_C = nullptr;         // stage-1 products, nb x ncells x nmodes (double or float)
     size_t cap_C = 0;
@@ -80,214 +81,85 @@ struct ProjState {
     size_t cap_trig = 0;
     float* d_W = nullptr;        // inverse-DFT weights, transposed: nbat x n1p (n1p = n1 rounded up to 4)
     size_t cap_W = 0;
+    // FP64 / FP32 projection on nt_gemm_kernel
+    float* d_Bw32 = nullptr;     // B' rounded to FP32, pitch nt_pitch<float>(ncells)
+    size_t cap_Bw32 = 0;
+    bool bw32_valid = false;
+    void* d_T = nullptr;         // a panel of rows of T_p (dense), or That_k rows (Toeplitz)
+    size_t cap_T = 0;
+    NtWork ws;                   // split-K accumulators
     // Toeplitz projection in FP64 / FP32 (same DFT along x, no operand split)
-    bool toep64_valid = false;   // Bg64 and Bhat64 match the uploaded modes
     int* d_gmap64 = nullptr;     // grid index -> cell number (as d_gmap)
     size_t cap_gmap64 = 0;
-    int* d_slab = nullptr;       // slab position r -> (y << 16) | z
-    size_t cap_slab = 0;
     double* d_trig64 = nullptr;  // cos, then sin of 2 pi j / L
     size_t cap_trig64 = 0;
-    double* d_W64 = nullptr;     // inverse-DFT weights W[x][b], n1 x nbat
+    double* d_W64 = nullptr;     // inverse-DFT weights W[b][x], nbat x n1
     size_t cap_W64 = 0;
-    double* d_Bg64 = nullptr;    // B' in grid order: M x Ng (pitch ldg), zero where the grid has no cell
-    size_t cap_Bg64 = 0;
-    double* d_Bhat64 = nullptr;  // DFT of B' along x: nbat x M x G ([b][m][r])
-    size_t cap_Bhat64 = 0;
-    double* d_Yhat64 = nullptr;  // one band's stage-1 products: nbat x M x G
-    size_t cap_Yhat64 = 0;
-    double* d_Y64 = nullptr;     // Y = S_p B' in grid order, up to four bands: M x Ng each (pitch ldg)
-    size_t cap_Y64 = 0;
-    double* d_That64 = nullptr;  // one band's That_k of a shell: (Nphi + 1) x G x G
-    size_t cap_That64 = 0;
+    struct Toep {                // per precision (FP64: 0, FP32: 1)
+        bool valid = false;      // Bg and Bhat match the uploaded modes
+        void* Bg = nullptr;      // B' in grid order: M x Kg (pitch ldg), zero where the grid has no cell
+        size_t cap_Bg = 0;
+        void* Bhat = nullptr;    // DFT of B' along x: nbat x M x Gp ([b][m][r])
+        size_t cap_Bhat = 0;
+        void* Yhat = nullptr;    // stage-1 products of the bands of one launch: nbat x M x Gp each
+        size_t cap_Yhat = 0;
+        void* Y = nullptr;       // Y = S_p B' in grid order, up to four bands: M x Kg each (pitch ldg)
+        size_t cap_Y = 0;
+    } toep[2];
 };
 
-// ---- FP64 / FP32 MFMA GEMM -----------------------------------------------------
+// ---- operands of the FP64 / FP32 projection ---------------------------------------
+//
+// Both stages run on nt_gemm_kernel, whose operands are plain padded rows: the
+// signal-matrix rows T_p are written from the pair table (a panel of them at a
+// time) instead of being generated in the GEMM's operand loader, which left that
+// kernel waiting on table gathers.  Writing and reading a panel costs 16 B per
+// element against 2 M flops.
 
+// out[z][i][c] = Q_f[key(row0 + i, c)], f = funcs[z], i < nrows, c < N; zero for N <= c < Kp.
+// Tile of 8 rows x 512 columns per 256-thread block, two columns per thread; the
+// column coordinates in LDS.
 template <typename T>
-struct Mfma;
-
-template <>
-struct Mfma<double> {
-    typedef d4_t acc_t;
-    __device__ __forceinline__ static acc_t mma(double a, double b, acc_t c) {
-        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+__global__ __launch_bounds__(256) void gen_rows_kernel(const double* __restrict__ Q, size_t qstride,
+                                                       const int* __restrict__ funcs, const int* __restrict__ cellidx,
+                                                       PairKey K, int N, int row0, int nrows, int Kp,
+                                                       T* __restrict__ out, size_t ld, size_t zstride) {
+    __shared__ int cx[512], cy[512], cz[512];
+    const int j0 = blockIdx.x * 512, i0 = blockIdx.y * 8;
+    for (int t = threadIdx.x; t < 512; t += 256) {
+        const int j = min(j0 + t, N - 1);
+        cx[t] = cellidx[3 * j];
+        cy[t] = cellidx[3 * j + 1];
+        cz[t] = cellidx[3 * j + 2];
     }
-};
-
-template <>
-struct Mfma<float> {
-    typedef f4_t acc_t;
-    __device__ __forceinline__ static acc_t mma(float a, float b, acc_t c) {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-    }
-};
-
-// Tile loads: 128 (m or n) x 16 (k) elements, 8 per thread.
-template <typename Src>
-__device__ __forceinline__ void tile_fetch(const Src& s, int i0, int k0, int nI, int nK, double (&r)[8]) {
-    const int t = threadIdx.x;
-    if (Src::k_contig) {
-        int i = i0 + (t >> 1), kb = k0 + (t & 1) * 8;
-        // whole, aligned runs of 8 by 16-byte loads
-        if constexpr (HasLoad8<Src>::value)
-            if (i < nI && kb + 8 <= nK && s.load8(i, kb, r)) return;
+    __syncthreads();
+    const double* q = Q + (size_t)funcs[blockIdx.z] * qstride;
+    T* o = out + (size_t)blockIdx.z * zstride;
+    const int t = 2 * threadIdx.x, j = j0 + t;
+    if (j >= Kp) return;
+    typedef T pair_t __attribute__((ext_vector_type(2)));
 #pragma unroll
-        for (int e = 0; e < 8; e++) r[e] = (i < nI && kb + e < nK) ? s.get(i, kb + e) : 0.0;
-    } else {
-        int k = k0 + (t >> 4), ib = i0 + (t & 15) * 8;
-#pragma unroll
-        for (int e = 0; e < 8; e++) r[e] = (k < nK && ib + e < nI) ? s.get(ib + e, k) : 0.0;
+    for (int r = 0; r < 8; r++) {
+        const int i = i0 + r;
+        if (i >= nrows) break;
+        const int* ca = cellidx + 3 * (size_t)(row0 + i);
+        const int ax = ca[0], ay = ca[1], az = ca[2];
+        pair_t v;
+        v[0] = j < N ? (T)q[K(ax, ay, az, cx[t], cy[t], cz[t])] : (T)0;
+        v[1] = j + 1 < N ? (T)q[K(ax, ay, az, cx[t + 1], cy[t + 1], cz[t + 1])] : (T)0;
+        *(pair_t*)(o + (size_t)i * ld + j) = v;
     }
 }
 
-template <typename Src, typename T>
-__device__ __forceinline__ void tile_store(T (*lds)[GT_M + 4], const double (&r)[8]) {
-    const int t = threadIdx.x;
-    if (Src::k_contig) {
-        int i = t >> 1, kb = (t & 1) * 8;
-#pragma unroll
-        for (int e = 0; e < 8; e++) lds[kb + e][i] = (T)r[e];
-    } else {
-        int k = t >> 4, ib = (t & 15) * 8;
-#pragma unroll
-        for (int e = 0; e < 8; e++) lds[k][ib + e] = (T)r[e];
-    }
-}
-
-// Epilogues
-struct OutColMajor {             // C[n*ld + m]
-    void* p;
-    size_t ld;
-    size_t batch_stride;
-};
-
-struct OutPackedUpper {          // P[n(n+1)/2 + m] for m <= n
-    double* p;
-    size_t batch_stride;
-};
-
-template <typename T, typename SrcA, typename SrcB, typename Out, bool UPPER>
-__global__ __launch_bounds__(GT_THREADS) void gemm_kernel(SrcA A, size_t a_batch, SrcB B, size_t b_batch, Out O,
-                                                          int M, int N, int K) {
-    typedef typename Mfma<T>::acc_t acc_t;
-    __shared__ T As[16][GT_M + 4];
-    __shared__ T Bs[16][GT_N + 4];
-    const int m0 = blockIdx.x * GT_M, n0 = blockIdx.y * GT_N;
-    if (UPPER && m0 > n0 + GT_N - 1) return;   // tile entirely below the diagonal
-    // batch offsets
-    A.p_shift(blockIdx.z, a_batch);
-    B.p_shift(blockIdx.z, b_batch);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
-    acc_t acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = acc_t{0, 0, 0, 0};
-
-    double ra[8], rb[8];
-    tile_fetch(A, m0, 0, M, K, ra);
-    tile_fetch(B, n0, 0, N, K, rb);
-    for (int k0 = 0; k0 < K; k0 += 16) {
-        __syncthreads();
-        tile_store<SrcA, T>(As, ra);
-        tile_store<SrcB, T>(Bs, rb);
-        __syncthreads();
-        if (k0 + 16 < K) {
-            tile_fetch(A, m0, k0 + 16, M, K, ra);
-            tile_fetch(B, n0, k0 + 16, N, K, rb);
-        }
-#pragma unroll
-        for (int kk = 0; kk < 4; kk++) {
-            T af[4], bf[4];
-            const int kr = kk * 4 + (lane >> 4);
-#pragma unroll
-            for (int i = 0; i < 4; i++) af[i] = As[kr][wm + i * 16 + (lane & 15)];
-#pragma unroll
-            for (int j = 0; j < 4; j++) bf[j] = Bs[kr][wn + j * 16 + (lane & 15)];
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc[i][j] = Mfma<T>::mma(af[i], bf[j], acc[i][j]);
-        }
-    }
-    // epilogue
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int n = n0 + wn + j * 16 + (lane & 15);
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int m = m0 + wm + i * 16 + acc_row<T>(lane, r);
-                O.put(blockIdx.z, m, n, M, N, (double)acc[i][j][r]);
-            }
-        }
-}
-
-// Sources with batch shifting (z index = band)
-template <bool SPH>
-struct GA_PairTableT : SrcPairTableT<SPH> {
-    size_t qstride;
-    const int* funcs;
-    __device__ __forceinline__ void p_shift(int z, size_t) { this->Q += (size_t)funcs[z] * qstride; }
-};
-typedef GA_PairTableT<false> GA_PairTable;
-typedef GA_PairTableT<true> GA_PairTableSph;
-struct GA_RowMajor : SrcDenseRowMajor {
-    __device__ __forceinline__ void p_shift(int z, size_t s) { p += (size_t)z * s; }
-};
-struct GB_ColMajor : SrcKColMajor {   // B[k][n] = p[n*ld + k]
-    __device__ __forceinline__ void p_shift(int z, size_t s) { p += (size_t)z * s; }
-};
-struct GA_ColMajorT : SrcKColMajor {  // A = X^T with X column-major: A[m][k] = X[k][m] = p[m*ld + k]
-    __device__ __forceinline__ void p_shift(int z, size_t s) { p += (size_t)z * s; }
-};
-
+// out[i][c] = X[i * ldx + c] for c < cols, zero for cols <= c < ld.
 template <typename T>
-struct PutColMajor {
-    T* p;
-    size_t ld, batch;
-    __device__ __forceinline__ void put(int z, int m, int n, int M, int N, double v) const {
-        if (m < M && n < N) p[(size_t)z * batch + (size_t)n * ld + m] = (T)v;
-    }
-};
-
-struct PutPacked {
-    double* p;
-    size_t batch;
-    __device__ __forceinline__ void put(int z, int m, int n, int M, int N, double v) const {
-        if (m < M && n < N && m <= n) p[(size_t)z * batch + (size_t)n * (n + 1) / 2 + m] = v;
-    }
-};
-
-// Stage-2 source reading the stage-1 product stored as T (double or float).
-template <typename T>
-struct GB_ColMajorT {
-    const T* p;
-    size_t ld;
-    static constexpr bool k_contig = true;
-    __device__ __forceinline__ double get(int n, int k) const { return (double)p[(size_t)n * ld + k]; }
-    __device__ __forceinline__ bool load8(int n, int k, double (&r)[8]) const {
-        const T* q = p + (size_t)n * ld + k;
-        if constexpr (std::is_same<T, double>::value) {
-            return load8_f64(q, r);
-        } else {
-            if ((reinterpret_cast<uintptr_t>(q) & 15) != 0) return false;
-#pragma unroll
-            for (int e = 0; e < 2; e++) {
-                const float4 v = reinterpret_cast<const float4*>(q)[e];
-                r[4 * e] = v.x;
-                r[4 * e + 1] = v.y;
-                r[4 * e + 2] = v.z;
-                r[4 * e + 3] = v.w;
-            }
-            return true;
-        }
-    }
-    __device__ __forceinline__ void p_shift(int z, size_t s) { p += (size_t)z * s; }
-};
+__global__ void pad_rows_kernel(const double* __restrict__ X, size_t ldx, int rows, int cols, T* __restrict__ out,
+                                size_t ld) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= (size_t)rows * ld) return;
+    const size_t r = i / ld, c = i - r * ld;
+    out[i] = c < (size_t)cols ? (T)X[r * ldx + c] : (T)0;
+}
 
 // ---- split-BF16x3 on pre-split planes --------------------------------------------
 //
@@ -939,13 +811,13 @@ __global__ void sum_parts_kernel(const float* __restrict__ part, int nparts, siz
     }
 }
 
-// B' = diag(w) B with w = sqrt(Nbar)
-__global__ void scale_rows_kernel(const double* B, const double* nbar, int N, int M, double* Bw, size_t ldw) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    size_t tot = (size_t)N * M;
-    if (i >= tot) return;
-    const size_t a = i % N, n = i / N;
-    Bw[n * ldw + a] = B[i] * sqrt(nbar[a]);
+// B' = diag(w) B with w = sqrt(Nbar), rows padded with zeros to ldw.
+template <typename T>
+__global__ void scale_rows_kernel(const double* B, const double* nbar, int N, int M, T* Bw, size_t ldw) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= ldw * M) return;
+    const size_t n = i / ldw, a = i - n * ldw;
+    Bw[i] = a < (size_t)N ? (T)(B[n * N + a] * sqrt(nbar[a])) : (T)0;
 }
 
 // ---- Toeplitz projection of box surveys ---------------------------------------------
@@ -1174,36 +1046,42 @@ __global__ __launch_bounds__(256) void idft_kernel(const float* __restrict__ yha
 // ---- Toeplitz projection in FP64 / FP32 -------------------------------------------
 //
 // The same identity without splitting the operands: B' in grid order and its
-// DFT along x in FP64, stage 1 as nbat = 2 n1 batched GEMMs (batch b:
-// That_((b+1)/2) times the b-th transformed block, That generated inside the
-// GEMM's A loader from Qhat), the inverse DFT in FP64, stage 2 as the upper
-// triangle of Bg'^T Y over the grid.  MFMA in FP64 (v_mfma_f64_16x16x4f64) or
-// FP32 (v_mfma_f32_16x16x4f32, operands rounded to FP32 at the LDS store).
+// DFT along x (FP64 sums), stage 1 as nbat = 2 n1 batched GEMMs (batch b: the
+// b-th transformed block of the modes times That_((b+1)/2)), the inverse DFT
+// (FP64 sums), stage 2 as the lower triangle of Y Bg'^T over the grid.  MFMA in
+// FP64 (v_mfma_f64_16x16x4f64) or FP32 (v_mfma_f32_16x16x4f32), operands stored
+// in that type; every row is padded to whole 128-byte k-steps with zeros.
 
-// B' in grid order: Bg[m][g] = B'[m][gmap[g]] (0 where the grid has no cell).
-__global__ void grid_b64_kernel(const double* __restrict__ Bw, size_t ldw, const int* __restrict__ gmap, int Ng, int M,
-                                double* __restrict__ Bg, size_t ldg) {
+// B' in grid order: Bg[m][g] = B'[m][gmap[g]] (0 where the grid has no cell and in the padding).
+template <typename T>
+__global__ void grid_b_kernel(const double* __restrict__ Bw, size_t ldw, const int* __restrict__ gmap, int Ng, int M,
+                              T* __restrict__ Bg, size_t ldg) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)M * Ng) return;
-    const size_t m = i / Ng, g = i - m * Ng;
-    const int a = gmap[g];
-    Bg[m * ldg + g] = a >= 0 ? Bw[m * ldw + a] : 0.0;
+    if (i >= (size_t)M * ldg) return;
+    const size_t m = i / ldg, g = i - m * ldg;
+    const int a = g < (size_t)Ng ? gmap[g] : -1;
+    Bg[i] = a >= 0 ? (T)Bw[m * ldw + a] : (T)0;
 }
 
-// Bhat[b][m][r] = sum_x cos(2 pi x k / L) Bg[m][x G + r] (b = 0 or odd) or
-// -sum_x sin(2 pi x k / L) Bg[m][x G + r] (b even, > 0), k = (b + 1) / 2.
-// Block (r tile, m); each thread keeps the n1 <= 64 grid values of its (m, r)
-// in registers.
+// Bhat[b][m][r] = sum_x cos(2 pi x k / L) B'_x[m][r] (b = 0 or odd) or
+// -sum_x sin(2 pi x k / L) B'_x[m][r] (b even, > 0), k = (b + 1) / 2; zero for
+// G <= r < Gp.  Block (r tile, m); each thread keeps the n1 <= 64 grid values of
+// its (m, r) in registers.
 constexpr int TOEP_MAXX = 64;
-__global__ __launch_bounds__(256) void bhat64_kernel(const double* __restrict__ Bg, size_t ldg, int n1, int G, int M,
-                                                     const double* __restrict__ trig, double* __restrict__ Bhat,
+template <typename T>
+__global__ __launch_bounds__(256) void bhat64_kernel(const double* __restrict__ Bw, size_t ldw,
+                                                     const int* __restrict__ gmap, int n1, int G, int M,
+                                                     const double* __restrict__ trig, T* __restrict__ Bhat, size_t Gp,
                                                      int nbat) {
     const int m = blockIdx.y, r = blockIdx.x * 256 + threadIdx.x;
-    if (r >= G) return;
+    if (r >= (int)Gp) return;
     const int L = 2 * n1;
     double v[TOEP_MAXX];
 #pragma unroll
-    for (int x = 0; x < TOEP_MAXX; x++) v[x] = x < n1 ? Bg[(size_t)m * ldg + (size_t)x * G + r] : 0.0;
+    for (int x = 0; x < TOEP_MAXX; x++) {
+        const int a = (x < n1 && r < G) ? gmap[(size_t)x * G + r] : -1;
+        v[x] = a >= 0 ? Bw[(size_t)m * ldw + a] : 0.0;
+    }
     for (int b = 0; b < nbat; b++) {
         const int k = (b + 1) >> 1;
         const bool imag = b > 0 && !(b & 1);
@@ -1212,35 +1090,38 @@ __global__ __launch_bounds__(256) void bhat64_kernel(const double* __restrict__ 
 #pragma unroll
         for (int x = 0; x < TOEP_MAXX; x++)
             if (x < n1) acc += t[(x * k) % L] * v[x];
-        Bhat[((size_t)b * M + m) * G + r] = imag ? -acc : acc;
+        Bhat[((size_t)b * M + m) * Gp + r] = (T)(imag ? -acc : acc);
     }
 }
 
-// A operand of the FP64 Toeplitz stage 1: That_k[r][c] = Qhat_k(|y_r - y_c| n3
-// + |z_r - z_c|) with k = (batch + 1) / 2; slab[r] = (y << 16) | z.
-struct GA_That {
-    const double* qhat;
-    const int* slab;
-    int G, n3;
-    static constexpr bool k_contig = true;
-    __device__ __forceinline__ void p_shift(int z, size_t) { qhat += (size_t)((z + 1) >> 1) * G; }
-    __device__ __forceinline__ double get(int r, int c) const {
-        const int a = slab[r], b = slab[c];
-        const int dy = abs((a >> 16) - (b >> 16)), dz = abs((a & 0xffff) - (b & 0xffff));
-        return qhat[dy * n3 + dz];
-    }
-};
+// That_k of a box, rows [row0, row0 + nrows): out[k][r - row0][c] =
+// Qhat_k(|y_r - y_c| n3 + |z_r - z_c|), zero for G <= c < Gp; k = blockIdx.z.
+template <typename T>
+__global__ __launch_bounds__(256) void that_rows_kernel(const double* __restrict__ qhat, int G, int n3, int row0,
+                                                        int nrows, T* __restrict__ out, size_t Gp) {
+    const int c = blockIdx.x * 256 + threadIdx.x, r = row0 + blockIdx.y, k = blockIdx.z;
+    if (c >= (int)Gp) return;
+    const int yr = r / n3, zr = r - yr * n3, yc = c / n3, zc = c - yc * n3;
+    const double v = c < G ? qhat[(size_t)k * G + abs(yr - yc) * n3 + abs(zr - zc)] : 0.0;
+    out[((size_t)k * nrows + blockIdx.y) * Gp + c] = (T)v;
+}
 
 // Y[m][x G + r] = sum_b W[b][x] Yhat[b][m][r] for x < n1 (FP64), summed in b
-// order.  Block (r tile, m); W (nbat x n1) in LDS, the n1 <= NMAX sums of a
-// thread in registers; the Yhat values of eight batches are loaded together.
-template <int NMAX>
-__global__ __launch_bounds__(256) void idft64_kernel(const double* __restrict__ Yhat, int nbat, int G, int n1, int M,
-                                                     const double* __restrict__ W, double* __restrict__ Y, size_t ldg) {
+// order; zero for n1 G <= g < Kg.  Block (r tile, m, band); W (nbat x n1) in LDS,
+// the n1 <= NMAX sums of a thread in registers; the Yhat values of eight batches
+// are loaded together.
+template <typename T, int NMAX>
+__global__ __launch_bounds__(256) void idft64_kernel(const T* __restrict__ Yhat, int nbat, int G, size_t Gp, int n1,
+                                                     int M, const double* __restrict__ W, T* __restrict__ Y, size_t ldg,
+                                                     int Kg) {
     extern __shared__ double id64_w[];   // nbat x n1
     const int m = blockIdx.y, r = blockIdx.x * 256 + threadIdx.x;
+    Yhat += (size_t)blockIdx.z * nbat * M * Gp;
+    Y += ((size_t)blockIdx.z * M + m) * ldg;
     for (int i = threadIdx.x; i < nbat * n1; i += 256) id64_w[i] = W[i];
     __syncthreads();
+    if (blockIdx.x == 0)
+        for (int g = n1 * G + threadIdx.x; g < Kg; g += 256) Y[g] = (T)0;
     if (r >= G) return;
     double acc[NMAX];
 #pragma unroll
@@ -1248,7 +1129,7 @@ __global__ __launch_bounds__(256) void idft64_kernel(const double* __restrict__ 
     for (int b0 = 0; b0 < nbat; b0 += 8) {
         double yh[8];
 #pragma unroll
-        for (int u = 0; u < 8; u++) yh[u] = b0 + u < nbat ? Yhat[((size_t)(b0 + u) * M + m) * G + r] : 0.0;
+        for (int u = 0; u < 8; u++) yh[u] = b0 + u < nbat ? (double)Yhat[((size_t)(b0 + u) * M + m) * Gp + r] : 0.0;
 #pragma unroll
         for (int u = 0; u < 8; u++) {
             if (b0 + u >= nbat) break;
@@ -1260,7 +1141,7 @@ __global__ __launch_bounds__(256) void idft64_kernel(const double* __restrict__ 
     }
 #pragma unroll
     for (int x = 0; x < NMAX; x++)
-        if (x < n1) Y[(size_t)m * ldg + (size_t)x * G + r] = acc[x];
+        if (x < n1) Y[(size_t)x * G + r] = (T)acc[x];
 }
 
 // ---- Toeplitz projection of spherical shells (DFT along phi) -----------------------
@@ -1283,19 +1164,19 @@ __global__ __launch_bounds__(256) void idft64_kernel(const double* __restrict__ 
 // C[k][d] (1 at d = 0, else 2 cos(2 pi d k / L)); each thread then forms the Nphi + 1
 // transformed values of its column, That_k = sum_d C[k][d] q[d] in d order, from
 // wave-uniform LDS rows.  NMAX >= Nphi bounds the registers; CB = 128 for NMAX = 64 keeps
-// the block's LDS under 100 KB.  SPLIT: hi / lo BF16 planes
-// [k][Gr][Gp], zero outside G x G (the grid covers Gr x Gp); else FP64 T[k][G][G] (the
-// grid covers G x G).
-template <bool SPLIT, int NMAX>
+// the block's LDS under 100 KB.  T void: hi / lo BF16 planes
+// [k][Gr][Gp], zero outside G x G (the grid covers Gr x Gp); else out[k][h - row0][c]
+// for the grid's rows h = row0 + blockIdx.y, Gr of them, zero for G <= c < Gp.
+template <typename T, int NMAX>
 __global__ __launch_bounds__(256) void that_sph_kernel(const double* __restrict__ Q, int G, int nph,
                                                        const double* __restrict__ trig, __bf16* __restrict__ hi,
-                                                       __bf16* __restrict__ lo, size_t Gr, size_t Gp,
-                                                       double* __restrict__ T) {
+                                                       __bf16* __restrict__ lo, size_t Gr, size_t Gp, int row0,
+                                                       T* __restrict__ out) {
     constexpr int CB = NMAX <= 32 ? 256 : 128;
     extern __shared__ double ts_q[];   // CB x (nph + 1) table entries, then C: (nph + 1) x NMAX
     const int L = 2 * nph, ldq = nph + 1;
     double* sC = ts_q + CB * ldq;
-    const int h = blockIdx.y, c0 = blockIdx.x * CB, t = threadIdx.x;
+    const int h = row0 + blockIdx.y, c0 = blockIdx.x * CB, t = threadIdx.x;
     const int ncol = (h < G && c0 < G) ? min(CB, G - c0) : 0;
     for (int i = t; i < (nph + 1) * NMAX; i += CB) {
         const int k = i / NMAX, d = i - k * NMAX;
@@ -1332,16 +1213,15 @@ __global__ __launch_bounds__(256) void that_sph_kernel(const double* __restrict_
 #pragma unroll
         for (int d = 0; d < NMAX; d++)
             if (d < nph) acc += Ck[d] * q[d];
-        if constexpr (SPLIT) {
-            if ((size_t)c < Gp) {
-                __bf16 x, y;
-                split2((float)acc, x, y);
-                const size_t o = ((size_t)k * Gr + h) * Gp + c;
-                hi[o] = x;
-                lo[o] = y;
-            }
-        } else if (live) {
-            T[((size_t)k * G + h) * G + c] = acc;
+        if ((size_t)c >= Gp) continue;
+        const size_t o = ((size_t)k * Gr + blockIdx.y) * Gp + c;
+        if constexpr (std::is_same<T, void>::value) {
+            __bf16 x, y;
+            split2((float)acc, x, y);
+            hi[o] = x;
+            lo[o] = y;
+        } else {
+            out[o] = (T)acc;
         }
     }
 }
@@ -1351,36 +1231,27 @@ static int that_sph_cb(int nph) { return nph <= 32 ? 256 : 128; }
 static size_t that_sph_lds(int nph) {
     return ((size_t)that_sph_cb(nph) * (nph + 1) + (size_t)(nph + 1) * (nph <= 32 ? 32 : TOEP_MAXX)) * 8;
 }
-template <bool SPLIT>
+template <typename T>
 static int that_sph_attr(opsec_ctx* ctx, int nph) {
-    const void* fn = nph <= 32 ? (const void*)that_sph_kernel<SPLIT, 32> : (const void*)that_sph_kernel<SPLIT, TOEP_MAXX>;
+    const void* fn = nph <= 32 ? (const void*)that_sph_kernel<T, 32> : (const void*)that_sph_kernel<T, TOEP_MAXX>;
     OPSEC_HIP_TRY(ctx, hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)that_sph_lds(nph)));
     return OPSEC_OK;
 }
-template <bool SPLIT>
+// Rows row0 .. row0 + rows - 1 of every That_k of one band.
+template <typename T>
 static void launch_that_sph(opsec_ctx* ctx, const double* Q, int G, int nph, const double* trig, __bf16* hi,
-                            __bf16* lo, size_t Gr, size_t Gp, double* T) {
-    const size_t cb = that_sph_cb(nph), cols = SPLIT ? Gp : (size_t)G;
-    const dim3 grid((unsigned)((cols + cb - 1) / cb), SPLIT ? (unsigned)Gr : (unsigned)G);
+                            __bf16* lo, size_t rows, size_t Gp, int row0, T* out) {
+    const size_t cb = that_sph_cb(nph);
+    const dim3 grid((unsigned)((Gp + cb - 1) / cb), (unsigned)rows);
     if (nph <= 32)
-        hipLaunchKernelGGL((that_sph_kernel<SPLIT, 32>), grid, dim3((unsigned)cb), that_sph_lds(nph), ctx->stream, Q, G,
-                           nph, trig, hi, lo, Gr, Gp, T);
+        hipLaunchKernelGGL((that_sph_kernel<T, 32>), grid, dim3((unsigned)cb), that_sph_lds(nph), ctx->stream, Q, G,
+                           nph, trig, hi, lo, rows, Gp, row0, out);
     else
-        hipLaunchKernelGGL((that_sph_kernel<SPLIT, TOEP_MAXX>), grid, dim3((unsigned)cb), that_sph_lds(nph), ctx->stream,
-                           Q, G, nph, trig, hi, lo, Gr, Gp, T);
+        hipLaunchKernelGGL((that_sph_kernel<T, TOEP_MAXX>), grid, dim3((unsigned)cb), that_sph_lds(nph), ctx->stream,
+                           Q, G, nph, trig, hi, lo, rows, Gp, row0, out);
 }
-
-// A operand of the FP64 / FP32 Toeplitz stage 1 of a shell: batch b reads the dense
-// That_((b + 1) / 2), row-major G x G.
-struct GA_ThatDense : SrcDenseRowMajor {
-    __device__ __forceinline__ void p_shift(int z, size_t s) { p += (size_t)((z + 1) >> 1) * s; }
-};
 
 // ---- host --------------------------------------------------------------------------
-
-static dim3 grid_for(int M, int N, int nb) {
-    return dim3((M + GT_M - 1) / GT_M, (N + GT_N - 1) / GT_N, nb);
-}
 
 static dim3 blocks_for(size_t threads) { return dim3((unsigned)((threads + 255) / 256)); }
 
@@ -1711,7 +1582,7 @@ static int run_project_toeplitz(opsec_ctx* ctx, int nb, const int* funcs) {
     const size_t id_lds = ((size_t)nbat * 128 + (size_t)((n1 + 3) & ~3) * nbat) * 4;
     OPSEC_HIP_TRY(ctx, hipFuncSetAttribute((const void*)idft_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
                                            (int)id_lds));
-    if (tgrid.sph && (rc = that_sph_attr<true>(ctx, n1))) return rc;
+    if (tgrid.sph && (rc = that_sph_attr<void>(ctx, n1))) return rc;
     __bf16* Th = ps->d_That;
     __bf16* Tl = ps->d_That + (size_t)(n1 + 1) * plane_t;
     EpiYhat toY{ps->d_Yhat, M, G, nbat};
@@ -1732,7 +1603,7 @@ static int run_project_toeplitz(opsec_ctx* ctx, int nb, const int* funcs) {
             const double* Qf = ctx->d_Q + (size_t)funcs[z] * ctx->nkeys;
             hipEventRecord(evb[4 * z], ctx->stream);
             if (tgrid.sph) {
-                launch_that_sph<true>(ctx, Qf, G, n1, ps->d_trig, Th, Tl, Gr, Gp, nullptr);
+                launch_that_sph<void>(ctx, Qf, G, n1, ps->d_trig, Th, Tl, Gr, Gp, 0, nullptr);
             } else {
                 hipLaunchKernelGGL(qhat_kernel, dim3((unsigned)(((n1 + 1) * G + 255) / 256)), dim3(256), 0,
                                    ctx->stream, Qf, n1, G, ps->d_trig, ps->d_Qhat);
@@ -1797,12 +1668,41 @@ static int run_project_toeplitz(opsec_ctx* ctx, int nb, const int* funcs) {
     return OPSEC_OK;
 }
 
-// Toeplitz projection without operand splitting: FP64 (prec FP64) or FP32
-// (prec FP32) MFMA, FP64 DFTs.  Per band: Qhat (FP64 DFT of the table along
-// x), the batched stage-1 GEMMs into Yhat, the inverse DFT into Y (grid
-// order), the upper-triangle stage-2 GEMM into the packed result.
-static int run_project_toeplitz64(opsec_ctx* ctx, int nb, const int* funcs, int prec) {
+// ---- FP64 / FP32 projection (host) ----------------------------------------------------
+
+// Bytes of generated operand rows (T_p panels, That_k rows) and of stage-1
+// products in frequency that one launch works on: large enough that a launch
+// has many rounds of tiles (2 GiB of T_p rows at 32^3: 8192 rows x 4000 modes,
+// four rounds of 512 tiles), small next to the stage-1 products themselves.
+constexpr size_t NT_PANEL_BYTES = (size_t)2 << 30;
+
+// Rows of a panel of `row_bytes` each within NT_PANEL_BYTES: all of them, or a
+// multiple of the tile (at most 32768: the generators' grid).
+static int panel_rows(int rows, size_t row_bytes) {
+    const size_t fit = NT_PANEL_BYTES / row_bytes / NT_BN * NT_BN;
+    return (int)std::min<size_t>(rows, std::max<size_t>(NT_BN, std::min<size_t>(fit, 32768)));
+}
+
+// Stage 2 of g bands: P_p = B'^T C_p, packed, from X (M rows of K, pitch ld) and
+// the bands' products C (M rows each, band stride cstride).  The lower tiles of
+// C_p B'^T hold column m of the packed upper triangle as row m, so a tile's rows
+// are contiguous in the output.
+template <typename T>
+static int stage2_nt(opsec_ctx* ctx, NtWork& ws, const T* X, size_t ld, const T* C, size_t cstride, int g, int M, int K,
+                     double* P) {
+    NtArgs<T> A{C, ld, 0, cstride, M, X, ld, 0, 0, M, (int)(nt_kpad<T>(K) / nt_bk<T>()), 1, g};
+    return launch_nt_gemm<T>(ctx, ws, A, NtPacked{P, (size_t)packed_size(M)});
+}
+
+// Toeplitz projection without operand splitting: FP64 or FP32 MFMA, FP64 DFTs.
+// Per band: That (from the FP64 DFT of the table), the batched stage-1 GEMMs
+// into Yhat, the inverse DFT into Y (grid order); stage 2 for up to
+// TOEP64_GROUP bands per launch.  Small surveys run stage 1 for several bands
+// per launch as well.
+template <typename T>
+static int run_project_toeplitz_nt(opsec_ctx* ctx, int nb, const int* funcs, int prec) {
     ProjState* ps = ctx->proj;
+    ProjState::Toep& tp = ps->toep[std::is_same<T, float>::value];
     const SurveyDev& sv = ctx->sv;
     const int M = ctx->nmodes;
     const ToepGrid tgrid = toep_grid(sv);
@@ -1811,26 +1711,24 @@ static int run_project_toeplitz64(opsec_ctx* ctx, int nb, const int* funcs, int 
     if ((rc = toep_check(ctx, tgrid))) return rc;
     if (!tgrid.sph && (sv.n2 >= 65536 || sv.n3 >= 65536))
         return set_error(ctx, OPSEC_EINVAL, "Toeplitz projection: Ny, Nz < 65536");
-    const size_t ldg = (size_t)Ng + 32;   // pitch of the grid-order operands (not a power of two)
-    // stage 2 runs once per group of up to TOEP64_GROUP bands (grid.z = band): the upper
-    // tiles of one band alone fill the CUs unevenly (528 at 4000 modes: 2.06 rounds of 256)
+    const size_t Gp = nt_pitch<T>(G), ldg = nt_pitch<T>(Ng);
+    const int Kg = (int)nt_kpad<T>(Ng);
     const int grp = std::min(nb, TOEP64_GROUP);
-    const size_t ystride = (size_t)M * ldg;
-    if ((rc = dev_realloc(ctx, (void**)&ps->d_Yhat64, &ps->cap_Yhat64, (size_t)nbat * M * G * 8))) return rc;
-    if ((rc = dev_realloc(ctx, (void**)&ps->d_Y64, &ps->cap_Y64, (size_t)grp * ystride * 8))) return rc;
-    if (tgrid.sph) {
-        if ((rc = dev_realloc(ctx, (void**)&ps->d_That64, &ps->cap_That64, (size_t)(n1 + 1) * G * G * 8))) return rc;
-    } else if ((rc = dev_realloc(ctx, (void**)&ps->d_Qhat, &ps->cap_Qhat, (size_t)(n1 + 1) * G * 8))) {
-        return rc;
-    }
+    const size_t ystride = (size_t)M * ldg, hstride = (size_t)nbat * M * Gp;
+    // rows of That_k (all k) per launch; bands per stage-1 launch when all rows fit
+    const size_t trow = (size_t)(n1 + 1) * Gp * sizeof(T);
+    const int trows = panel_rows(G, trow);
+    const int sub = trows < G ? 1
+                              : (int)std::max<size_t>(1, std::min<size_t>(grp, NT_PANEL_BYTES / (trow * G + hstride * sizeof(T))));
+    const size_t tstride = (size_t)(n1 + 1) * trows * Gp;
+    if ((rc = dev_realloc(ctx, &tp.Yhat, &tp.cap_Yhat, (size_t)sub * hstride * sizeof(T)))) return rc;
+    if ((rc = dev_realloc(ctx, &tp.Y, &tp.cap_Y, (size_t)grp * ystride * sizeof(T)))) return rc;
+    if ((rc = dev_realloc(ctx, &ps->d_T, &ps->cap_T, (size_t)sub * tstride * sizeof(T)))) return rc;
+    if (!tgrid.sph && (rc = dev_realloc(ctx, (void**)&ps->d_Qhat, &ps->cap_Qhat, (size_t)(n1 + 1) * G * 8))) return rc;
     if ((rc = dev_realloc(ctx, &ps->d_P, &ps->cap_P, (size_t)nb * packed_size(M) * 8))) return rc;
-    if (!ps->toep64_valid) {
+    if (!tp.valid) {
         std::vector<int> gmap;
         if ((rc = toep_gmap(ctx, Ng, gmap))) return rc;
-        // slab position -> (y << 16) | z (box only)
-        std::vector<int> slab((size_t)G, 0);
-        if (!tgrid.sph)
-            for (int r = 0; r < G; r++) slab[r] = ((r / sv.n3) << 16) | (r % sv.n3);
         std::vector<double> trig;
         trig_table(L, trig);
         // inverse weights W[b][x]: (c_k / L) cos and -(c_k / L) sin, c_0 = c_n1 = 1, else 2
@@ -1843,114 +1741,85 @@ static int run_project_toeplitz64(opsec_ctx* ctx, int nb, const int* funcs, int 
                 W[(size_t)b * n1 + x] = imag ? -ck * trig[L + j] / L : ck * trig[j] / L;
             }
         if ((rc = dev_realloc(ctx, (void**)&ps->d_gmap64, &ps->cap_gmap64, (size_t)Ng * 4))) return rc;
-        if ((rc = dev_realloc(ctx, (void**)&ps->d_slab, &ps->cap_slab, (size_t)G * 4))) return rc;
         if ((rc = dev_realloc(ctx, (void**)&ps->d_trig64, &ps->cap_trig64, trig.size() * 8))) return rc;
         if ((rc = dev_realloc(ctx, (void**)&ps->d_W64, &ps->cap_W64, W.size() * 8))) return rc;
-        if ((rc = dev_realloc(ctx, (void**)&ps->d_Bg64, &ps->cap_Bg64, (size_t)M * ldg * 8))) return rc;
-        if ((rc = dev_realloc(ctx, (void**)&ps->d_Bhat64, &ps->cap_Bhat64, (size_t)nbat * M * G * 8))) return rc;
+        if ((rc = dev_realloc(ctx, &tp.Bg, &tp.cap_Bg, ystride * sizeof(T)))) return rc;
+        if ((rc = dev_realloc(ctx, &tp.Bhat, &tp.cap_Bhat, hstride * sizeof(T)))) return rc;
         OPSEC_HIP_TRY(ctx, stream_copy(ctx, ps->d_gmap64, gmap.data(), gmap.size() * 4, hipMemcpyHostToDevice));
-        OPSEC_HIP_TRY(ctx, stream_copy(ctx, ps->d_slab, slab.data(), slab.size() * 4, hipMemcpyHostToDevice));
         OPSEC_HIP_TRY(ctx, stream_copy(ctx, ps->d_trig64, trig.data(), trig.size() * 8, hipMemcpyHostToDevice));
         OPSEC_HIP_TRY(ctx, stream_copy(ctx, ps->d_W64, W.data(), W.size() * 8, hipMemcpyHostToDevice));
-        const size_t tot = (size_t)M * Ng;
-        hipLaunchKernelGGL(grid_b64_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, ctx->stream, ps->d_Bw,
-                           ps->ldw, ps->d_gmap64, Ng, M, ps->d_Bg64, ldg);
-        hipLaunchKernelGGL(bhat64_kernel, dim3((unsigned)((G + 255) / 256), (unsigned)M), dim3(256), 0, ctx->stream,
-                           ps->d_Bg64, ldg, n1, G, M, ps->d_trig64, ps->d_Bhat64, nbat);
+        hipLaunchKernelGGL(grid_b_kernel<T>, blocks_for(ystride), dim3(256), 0, ctx->stream, ps->d_Bw, ps->ldw,
+                           ps->d_gmap64, Ng, M, (T*)tp.Bg, ldg);
+        hipLaunchKernelGGL(bhat64_kernel<T>, dim3((unsigned)((Gp + 255) / 256), (unsigned)M), dim3(256), 0, ctx->stream,
+                           ps->d_Bw, ps->ldw, ps->d_gmap64, n1, G, M, ps->d_trig64, (T*)tp.Bhat, Gp, nbat);
         OPSEC_HIP_TRY(ctx, hipGetLastError());
-        ps->toep64_valid = true;
+        tp.valid = true;
     }
     const size_t id_lds = (size_t)nbat * n1 * 8;
-    OPSEC_HIP_TRY(ctx, hipFuncSetAttribute(n1 <= 32 ? (const void*)idft64_kernel<32> : (const void*)idft64_kernel<TOEP_MAXX>,
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)id_lds));
-    if (tgrid.sph && (rc = that_sph_attr<false>(ctx, n1))) return rc;
-    const int ngroups = (nb + grp - 1) / grp;
-    // events per band: start, That / Qhat generated, stage 1 and inverse DFT; per group: stage 2
-    std::vector<hipEvent_t> ev(3 * (size_t)nb + ngroups);
+    const auto idft = n1 <= 32 ? idft64_kernel<T, 32> : idft64_kernel<T, TOEP_MAXX>;
+    OPSEC_HIP_TRY(ctx, hipFuncSetAttribute((const void*)idft, hipFuncAttributeMaxDynamicSharedMemorySize, (int)id_lds));
+    if (tgrid.sph && (rc = that_sph_attr<T>(ctx, n1))) return rc;
+    const int ngroups = (nb + grp - 1) / grp, nsub = (nb + sub - 1) / sub + ngroups;
+    // events: per stage-1 launch its start and end, That generated; per group: stage 2
+    std::vector<hipEvent_t> ev(3 * (size_t)nsub + 2 * (size_t)ngroups);
     for (auto& e : ev) OPSEC_HIP_TRY(ctx, hipEventCreate(&e));
-    hipEvent_t* evb = ev.data();
-    hipEvent_t* evg = ev.data() + 3 * (size_t)nb;
+    hipEvent_t* evg = ev.data() + 3 * (size_t)nsub;
     const size_t np = (size_t)packed_size(M);
-    GA_That A;
-    A.qhat = ps->d_Qhat;
-    A.slab = ps->d_slab;
-    A.G = G;
-    A.n3 = sv.n3;
-    GA_ThatDense As;
-    As.p = ps->d_That64;
-    As.ld = G;
-    GB_ColMajor Bop;   // batch b: Bhat[b] (B[k = r][n = m] = p[m G + r])
-    Bop.p = ps->d_Bhat64;
-    Bop.ld = G;
-    PutColMajor<double> toYhat{ps->d_Yhat64, (size_t)G, (size_t)M * G};
-    GA_ColMajorT A2;   // Bg'^T: A2[m][g] = Bg[m ldg + g]
-    A2.p = ps->d_Bg64;
-    A2.ld = ldg;
-    GB_ColMajorT<double> B2{ps->d_Y64, ldg};
-    const dim3 g1 = grid_for(G, M, nbat);
+    T* Tp = (T*)ps->d_T;
+    int si = 0;
     for (int z0 = 0, gi = 0; z0 < nb; z0 += grp, gi++) {
         const int g = std::min(grp, nb - z0);
-        for (int q = 0; q < g; q++) {
-            const int z = z0 + q;
-            const double* Qf = ctx->d_Q + (size_t)funcs[z] * ctx->nkeys;
-            hipEventRecord(evb[3 * z], ctx->stream);
-            if (tgrid.sph)
-                launch_that_sph<false>(ctx, Qf, G, n1, ps->d_trig64, nullptr, nullptr, 0, 0, ps->d_That64);
-            else
-                hipLaunchKernelGGL(qhat_kernel, dim3((unsigned)(((n1 + 1) * G + 255) / 256)), dim3(256), 0,
-                                   ctx->stream, Qf, n1, G, ps->d_trig64, ps->d_Qhat);
-            hipEventRecord(evb[3 * z + 1], ctx->stream);
-            const size_t tplane = (size_t)G * G;
-            if (tgrid.sph && prec == OPSEC_PREC_FP64)
-                hipLaunchKernelGGL((gemm_kernel<double, GA_ThatDense, GB_ColMajor, PutColMajor<double>, false>), g1,
-                                   dim3(GT_THREADS), 0, ctx->stream, As, tplane, Bop, (size_t)M * G, toYhat, G, M, G);
-            else if (tgrid.sph)
-                hipLaunchKernelGGL((gemm_kernel<float, GA_ThatDense, GB_ColMajor, PutColMajor<double>, false>), g1,
-                                   dim3(GT_THREADS), 0, ctx->stream, As, tplane, Bop, (size_t)M * G, toYhat, G, M, G);
-            else if (prec == OPSEC_PREC_FP64)
-                hipLaunchKernelGGL((gemm_kernel<double, GA_That, GB_ColMajor, PutColMajor<double>, false>), g1,
-                                   dim3(GT_THREADS), 0, ctx->stream, A, 0, Bop, (size_t)M * G, toYhat, G, M, G);
-            else
-                hipLaunchKernelGGL((gemm_kernel<float, GA_That, GB_ColMajor, PutColMajor<double>, false>), g1,
-                                   dim3(GT_THREADS), 0, ctx->stream, A, 0, Bop, (size_t)M * G, toYhat, G, M, G);
-            if (n1 <= 32)
-                hipLaunchKernelGGL(idft64_kernel<32>, dim3((unsigned)((G + 255) / 256), (unsigned)M), dim3(256), id_lds,
-                                   ctx->stream, ps->d_Yhat64, nbat, G, n1, M, ps->d_W64,
-                                   ps->d_Y64 + (size_t)q * ystride, ldg);
-            else
-                hipLaunchKernelGGL(idft64_kernel<TOEP_MAXX>, dim3((unsigned)((G + 255) / 256), (unsigned)M), dim3(256),
-                                   id_lds, ctx->stream, ps->d_Yhat64, nbat, G, n1, M, ps->d_W64,
-                                   ps->d_Y64 + (size_t)q * ystride, ldg);
-            hipEventRecord(evb[3 * z + 2], ctx->stream);
+        for (int q0 = 0; q0 < g; q0 += sub, si++) {
+            const int ns = std::min(sub, g - q0);
+            hipEventRecord(ev[3 * si], ctx->stream);
+            for (int r0 = 0; r0 < G; r0 += trows) {
+                const int nr = std::min(trows, G - r0);
+                const size_t tz = (size_t)(n1 + 1) * nr * Gp;   // one band's That_k rows
+                for (int q = 0; q < ns; q++) {
+                    const double* Qf = ctx->d_Q + (size_t)funcs[z0 + q0 + q] * ctx->nkeys;
+                    if (tgrid.sph) {
+                        launch_that_sph<T>(ctx, Qf, G, n1, ps->d_trig64, nullptr, nullptr, nr, Gp, r0, Tp + q * tz);
+                        continue;
+                    }
+                    if (r0 == 0)
+                        hipLaunchKernelGGL(qhat_kernel, dim3((unsigned)(((n1 + 1) * G + 255) / 256)), dim3(256), 0,
+                                           ctx->stream, Qf, n1, G, ps->d_trig64, ps->d_Qhat);
+                    hipLaunchKernelGGL(that_rows_kernel<T>, dim3((unsigned)((Gp + 255) / 256), (unsigned)nr, n1 + 1),
+                                       dim3(256), 0, ctx->stream, ps->d_Qhat, G, sv.n3, r0, nr, Tp + q * tz, Gp);
+                }
+                if (r0 == 0) hipEventRecord(ev[3 * si + 1], ctx->stream);
+                // batch b of band q: Yhat[b] (M x G) = Bhat[b] That_((b+1)/2), columns r0 .. r0 + nr - 1
+                NtArgs<T> A{(const T*)tp.Bhat, Gp, (size_t)M * Gp, 0, M, Tp, Gp, (size_t)nr * Gp, tz, nr,
+                            (int)(nt_kpad<T>(G) / nt_bk<T>()), nbat, nbat * ns};
+                if (!rc) rc = launch_nt_gemm<T>(ctx, ps->ws, A, NtRows<T>{(T*)tp.Yhat + r0, Gp, (size_t)M * Gp, hstride, nr});
+            }
+            hipLaunchKernelGGL(idft, dim3((unsigned)((G + 255) / 256), (unsigned)M, (unsigned)ns), dim3(256), id_lds,
+                               ctx->stream, (const T*)tp.Yhat, nbat, G, Gp, n1, M, ps->d_W64,
+                               (T*)tp.Y + (size_t)q0 * ystride, ldg, Kg);
+            hipEventRecord(ev[3 * si + 2], ctx->stream);
         }
-        // stage 2 of the group's bands in one launch: batch q = band z0 + q
-        PutPacked outP{(double*)ps->d_P + (size_t)z0 * np, np};
-        const dim3 g2 = grid_for(M, M, g);
-        if (prec == OPSEC_PREC_FP64)
-            hipLaunchKernelGGL((gemm_kernel<double, GA_ColMajorT, GB_ColMajorT<double>, PutPacked, true>), g2,
-                               dim3(GT_THREADS), 0, ctx->stream, A2, 0, B2, ystride, outP, M, M, Ng);
-        else
-            hipLaunchKernelGGL((gemm_kernel<float, GA_ColMajorT, GB_ColMajorT<double>, PutPacked, true>), g2,
-                               dim3(GT_THREADS), 0, ctx->stream, A2, 0, B2, ystride, outP, M, M, Ng);
-        hipEventRecord(evg[gi], ctx->stream);
+        hipEventRecord(evg[2 * gi], ctx->stream);
+        if (!rc)
+            rc = stage2_nt<T>(ctx, ps->ws, (const T*)tp.Bg, ldg, (const T*)tp.Y, ystride, g, M, Ng,
+                              (double*)ps->d_P + (size_t)z0 * np);
+        hipEventRecord(evg[2 * gi + 1], ctx->stream);
     }
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) rc = set_error(ctx, OPSEC_EHIP, "projection launch: %s", hipGetErrorString(e));
-    hipError_t es = hipEventSynchronize(evg[ngroups - 1]);
+    if (!rc && e != hipSuccess) rc = set_error(ctx, OPSEC_EHIP, "projection launch: %s", hipGetErrorString(e));
+    hipError_t es = hipStreamSynchronize(ctx->stream);
     if (!rc && es != hipSuccess) rc = set_error(ctx, OPSEC_EHIP, "projection: %s", hipGetErrorString(es));
     float tg = 0, t1 = 0, t2 = 0;
     if (!rc) {
-        for (int z = 0; z < nb; z++) {
+        for (int i = 0; i < si; i++) {
             float a, b;
-            hipEventElapsedTime(&a, evb[3 * z], evb[3 * z + 1]);
-            hipEventElapsedTime(&b, evb[3 * z + 1], evb[3 * z + 2]);
+            hipEventElapsedTime(&a, ev[3 * i], ev[3 * i + 1]);
+            hipEventElapsedTime(&b, ev[3 * i + 1], ev[3 * i + 2]);
             tg += a;
             t1 += b;
         }
         for (int gi = 0; gi < ngroups; gi++) {
-            const int zl = std::min(nb, (gi + 1) * grp) - 1;   // last band of the group
             float c;
-            hipEventElapsedTime(&c, evb[3 * zl + 2], evg[gi]);
+            hipEventElapsedTime(&c, evg[2 * gi], evg[2 * gi + 1]);
             t2 += c;
         }
     }
@@ -1959,7 +1828,7 @@ static int run_project_toeplitz64(opsec_ctx* ctx, int nb, const int* funcs, int 
     ps->last_ms_gen = tg;
     ps->last_ms_gemm1 = t1;     // stage-1 GEMMs and the inverse DFT
     ps->last_ms_gemm2 = t2;
-    ps->last_launches = nb;
+    ps->last_launches = si;
     ps->last_launches2 = ngroups;
     ps->last_ms_stage1 = tg + t1;
     ps->last_ms_stage2 = t2;
@@ -1968,89 +1837,61 @@ static int run_project_toeplitz64(opsec_ctx* ctx, int nb, const int* funcs, int 
     return OPSEC_OK;
 }
 
-// Stage 1 + stage 2 for nb functions (device pair tables), results to d_P.
 // Dense FP64 / FP32 projection of the bands funcs[0..nb) in groups: stage 1
-// (all bands of a group in one launch, grid.z = band) keeps the group's
-// products C_p = T_p B' (N x M each), so a group holds at most
-// DENSE_GROUP_BYTES of them (all 40 bands of the 32^3 box fit; the 50 bands
-// of the 65536-cell shell at 6000 modes take seven groups).
+// keeps the group's products C_p = T_p B' (N x M each), so a group holds at most
+// DENSE_GROUP_BYTES of them (all 40 bands of the 32^3 box fit; the 50 bands of
+// the 65536-cell shell at 6000 modes take seven groups).  Within a group stage 1
+// takes the rows of T_p in panels of NT_PANEL_BYTES (several bands per launch
+// where their whole T_p fit).  T_p is symmetric: C_p's row m (mode m, cells
+// contiguous) is row m of B' times the rows of T_p.
 constexpr size_t DENSE_GROUP_BYTES = (size_t)48 << 30;
 
-static int run_project(opsec_ctx* ctx, int nb, const int* d_funcs, const int* funcs, int prec) {
-    if (prec == OPSEC_PREC_BF16X3 && ctx->projection == OPSEC_PROJ_TOEPLITZ) return run_project_toeplitz(ctx, nb, funcs);
-    if (ctx->projection == OPSEC_PROJ_TOEPLITZ) return run_project_toeplitz64(ctx, nb, funcs, prec);
-    if (prec == OPSEC_PREC_BF16X3) return run_project_bf16x3(ctx, nb, funcs);
+template <typename T>
+static int run_project_dense_nt(opsec_ctx* ctx, int nb, const int* d_funcs, const T* Bw, size_t ldw, int prec) {
     ProjState* ps = ctx->proj;
     const int N = ctx->ncells, M = ctx->nmodes;
-    const size_t esize = (prec == OPSEC_PREC_FP64) ? 8 : 4;
-    const size_t ldc = ps->ldw;   // stage-1 products use the same padded pitch as B'
-    const size_t per_band = ldc * M * esize;
-    const int grp = (int)std::max<size_t>(1, std::min<size_t>(nb, DENSE_GROUP_BYTES / per_band));
+    const size_t per_band = ldw * M;   // stage-1 products use the same padded pitch as B'
+    const int grp = (int)std::max<size_t>(1, std::min<size_t>(nb, DENSE_GROUP_BYTES / (per_band * sizeof(T))));
+    const int Kp = (int)nt_kpad<T>(N), rows = panel_rows(N, ldw * sizeof(T));
+    const size_t tband = (size_t)rows * ldw;
+    const int sub = rows < N ? 1 : (int)std::max<size_t>(1, std::min<size_t>(grp, NT_PANEL_BYTES / (tband * sizeof(T))));
     int rc;
-    if ((rc = dev_realloc(ctx, &ps->d_C, &ps->cap_C, (size_t)grp * per_band))) return rc;
+    if ((rc = dev_realloc(ctx, &ps->d_C, &ps->cap_C, (size_t)grp * per_band * sizeof(T)))) return rc;
+    if ((rc = dev_realloc(ctx, &ps->d_T, &ps->cap_T, (size_t)sub * tband * sizeof(T)))) return rc;
     if ((rc = dev_realloc(ctx, &ps->d_P, &ps->cap_P, (size_t)nb * packed_size(M) * 8))) return rc;
-    const bool sph = ctx->sv.coordsys == OPSEC_COORD_SPHERICAL;
-    GA_PairTable A;
-    A.Q = ctx->d_Q;
-    A.cellidx = ctx->d_cellidx;
-    A.Ny = ctx->sv.n2;
-    A.Nz = ctx->sv.n3;
-    A.narcs = ctx->sv.n1 * ctx->sv.n2;
-    A.qstride = ctx->nkeys;
-    GA_PairTableSph As;
-    As.Q = A.Q;
-    As.cellidx = A.cellidx;
-    As.Ny = A.Ny;
-    As.Nz = A.Nz;
-    As.narcs = A.narcs;
-    As.qstride = A.qstride;
-    GB_ColMajor Bop;
-    Bop.p = ps->d_Bw;
-    Bop.ld = ps->ldw;
-    GA_ColMajorT A2;
-    A2.p = ps->d_Bw;
-    A2.ld = ps->ldw;
     const size_t np = (size_t)packed_size(M);
     const int ngroups = (nb + grp - 1) / grp;
     std::vector<hipEvent_t> ev(2 * (size_t)ngroups + 1);
     for (auto& e : ev) OPSEC_HIP_TRY(ctx, hipEventCreate(&e));
     hipEventRecord(ev[0], ctx->stream);
+    T* Tp = (T*)ps->d_T;
     for (int gi = 0; gi < ngroups; gi++) {
         const int z0 = gi * grp, g = std::min(grp, nb - z0);
-        A.funcs = d_funcs + z0;
-        As.funcs = d_funcs + z0;
-        dim3 g1 = grid_for(N, M, g), g2 = grid_for(M, M, g);
-        PutPacked outP{(double*)ps->d_P + (size_t)z0 * np, np};
-        if (prec == OPSEC_PREC_FP64) {
-            PutColMajor<double> outC{(double*)ps->d_C, ldc, ldc * M};
-            if (sph)
-                hipLaunchKernelGGL((gemm_kernel<double, GA_PairTableSph, GB_ColMajor, PutColMajor<double>, false>), g1,
-                                   dim3(GT_THREADS), 0, ctx->stream, As, 0, Bop, 0, outC, N, M, N);
-            else
-                hipLaunchKernelGGL((gemm_kernel<double, GA_PairTable, GB_ColMajor, PutColMajor<double>, false>), g1,
-                                   dim3(GT_THREADS), 0, ctx->stream, A, 0, Bop, 0, outC, N, M, N);
-            hipEventRecord(ev[2 * gi + 1], ctx->stream);
-            GB_ColMajorT<double> B2{(const double*)ps->d_C, ldc};
-            hipLaunchKernelGGL((gemm_kernel<double, GA_ColMajorT, GB_ColMajorT<double>, PutPacked, true>), g2,
-                               dim3(GT_THREADS), 0, ctx->stream, A2, 0, B2, ldc * M, outP, M, M, N);
-        } else {
-            PutColMajor<float> outC{(float*)ps->d_C, ldc, ldc * M};
-            if (sph)
-                hipLaunchKernelGGL((gemm_kernel<float, GA_PairTableSph, GB_ColMajor, PutColMajor<float>, false>), g1,
-                                   dim3(GT_THREADS), 0, ctx->stream, As, 0, Bop, 0, outC, N, M, N);
-            else
-                hipLaunchKernelGGL((gemm_kernel<float, GA_PairTable, GB_ColMajor, PutColMajor<float>, false>), g1,
-                                   dim3(GT_THREADS), 0, ctx->stream, A, 0, Bop, 0, outC, N, M, N);
-            hipEventRecord(ev[2 * gi + 1], ctx->stream);
-            GB_ColMajorT<float> B2{(const float*)ps->d_C, ldc};
-            hipLaunchKernelGGL((gemm_kernel<float, GA_ColMajorT, GB_ColMajorT<float>, PutPacked, true>), g2,
-                               dim3(GT_THREADS), 0, ctx->stream, A2, 0, B2, ldc * M, outP, M, M, N);
+        for (int q0 = 0; q0 < g; q0 += sub) {
+            const int ns = std::min(sub, g - q0);
+            for (int r0 = 0; r0 < N; r0 += rows) {
+                const int nr = std::min(rows, N - r0);
+                hipLaunchKernelGGL(gen_rows_kernel<T>, dim3((unsigned)((Kp + 511) / 512), (unsigned)((nr + 7) / 8), ns),
+                                   dim3(256), 0, ctx->stream, ctx->d_Q, (size_t)ctx->nkeys, d_funcs + z0 + q0,
+                                   ctx->d_cellidx, pair_key_of(ctx->sv), N, r0, nr, Kp, Tp, ldw, tband);
+                NtArgs<T> A{Bw, ldw, 0, 0, M, Tp, ldw, 0, tband, nr, Kp / nt_bk<T>(), 1, ns};
+                // the last panel's tiles also write the padding columns of C (from clamped rows: finite,
+                // and they meet the zero padding of B' in stage 2)
+                if (!rc)
+                    rc = launch_nt_gemm<T>(ctx, ps->ws, A,
+                                           NtRows<T>{(T*)ps->d_C + (size_t)q0 * per_band + r0, ldw, 0, per_band,
+                                                     r0 + nr < N ? nr : Kp - r0});
+            }
         }
+        hipEventRecord(ev[2 * gi + 1], ctx->stream);
+        if (!rc)
+            rc = stage2_nt<T>(ctx, ps->ws, Bw, ldw, (const T*)ps->d_C, per_band, g, M, N,
+                              (double*)ps->d_P + (size_t)z0 * np);
         hipEventRecord(ev[2 * gi + 2], ctx->stream);
     }
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess) rc = set_error(ctx, OPSEC_EHIP, "projection launch: %s", hipGetErrorString(e));
-    hipError_t es = hipEventSynchronize(ev[2 * ngroups]);
+    if (!rc && e != hipSuccess) rc = set_error(ctx, OPSEC_EHIP, "projection launch: %s", hipGetErrorString(e));
+    hipError_t es = hipStreamSynchronize(ctx->stream);
     if (!rc && es != hipSuccess) rc = set_error(ctx, OPSEC_EHIP, "projection: %s", hipGetErrorString(es));
     float t1 = 0, t2 = 0;
     if (!rc)
@@ -2070,13 +1911,62 @@ static int run_project(opsec_ctx* ctx, int nb, const int* d_funcs, const int* fu
     return OPSEC_OK;
 }
 
+// Stage 1 + stage 2 for nb functions (device pair tables), results to d_P.
+static int run_project(opsec_ctx* ctx, int nb, const int* d_funcs, const int* funcs, int prec) {
+    ProjState* ps = ctx->proj;
+    if (ctx->projection == OPSEC_PROJ_TOEPLITZ) {
+        if (prec == OPSEC_PREC_BF16X3) return run_project_toeplitz(ctx, nb, funcs);
+        if (prec == OPSEC_PREC_FP32) return run_project_toeplitz_nt<float>(ctx, nb, funcs, prec);
+        return run_project_toeplitz_nt<double>(ctx, nb, funcs, prec);
+    }
+    if (prec == OPSEC_PREC_BF16X3) return run_project_bf16x3(ctx, nb, funcs);
+    if (prec == OPSEC_PREC_FP64) return run_project_dense_nt<double>(ctx, nb, d_funcs, ps->d_Bw, ps->ldw, prec);
+    const size_t ld32 = nt_pitch<float>(ctx->ncells);
+    if (!ps->bw32_valid) {
+        int rc;
+        if ((rc = dev_realloc(ctx, (void**)&ps->d_Bw32, &ps->cap_Bw32, ld32 * ctx->nmodes * 4))) return rc;
+        hipLaunchKernelGGL(scale_rows_kernel<float>, blocks_for(ld32 * ctx->nmodes), dim3(256), 0, ctx->stream,
+                           ctx->d_B, ctx->d_nbar, ctx->ncells, ctx->nmodes, ps->d_Bw32, ld32);
+        OPSEC_HIP_TRY(ctx, hipGetLastError());
+        ps->bw32_valid = true;
+    }
+    return run_project_dense_nt<float>(ctx, nb, d_funcs, ps->d_Bw32, ld32, prec);
+}
+
+// P = B S B^T (packed) of a device matrix S (N x N row-major) and modes B (M x N).
+template <typename T>
+static int project_host_nt(opsec_ctx* ctx, int N, const double* dS, int M, const double* dB, double* dP) {
+    const size_t ld = nt_pitch<T>(N);
+    const int Kp = (int)nt_kpad<T>(N);
+    struct Work : NtWork {
+        ~Work() { dev_free(&p); }
+    } ws;
+    T *X = nullptr, *Bp = nullptr, *Cp = nullptr;
+    DevScratch tmp;
+    OPSEC_HIP_TRY(ctx, tmp.alloc(&X, ld * N * sizeof(T)));
+    OPSEC_HIP_TRY(ctx, tmp.alloc(&Bp, ld * M * sizeof(T)));
+    OPSEC_HIP_TRY(ctx, tmp.alloc(&Cp, ld * M * sizeof(T)));
+    hipLaunchKernelGGL(pad_rows_kernel<T>, blocks_for(ld * N), dim3(256), 0, ctx->stream, dS, (size_t)N, N, N, X, ld);
+    hipLaunchKernelGGL(pad_rows_kernel<T>, blocks_for(ld * M), dim3(256), 0, ctx->stream, dB, (size_t)N, M, N, Bp, ld);
+    // C[m][a] = sum_b S[a][b] B[m][b]
+    NtArgs<T> A1{Bp, ld, 0, 0, M, X, ld, 0, 0, N, Kp / nt_bk<T>(), 1, 1};
+    int rc = launch_nt_gemm<T>(ctx, ws, A1, NtRows<T>{Cp, ld, 0, 0, Kp});
+    // P[i][j] = sum_a B[i][a] C[j][a], i <= j
+    if (!rc) rc = stage2_nt<T>(ctx, ws, Bp, ld, Cp, 0, 1, M, N, dP);
+    if (rc) return rc;
+    OPSEC_HIP_TRY(ctx, hipGetLastError());
+    OPSEC_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    return OPSEC_OK;
+}
+
 // A new cell set invalidates the uploaded modes and everything derived from them.
 void invalidate_modes(opsec_ctx* ctx) {
     ctx->nmodes = 0;
     if (!ctx->proj) return;
     ctx->proj->bp_valid = false;
+    ctx->proj->bw32_valid = false;
     ctx->proj->toep_valid = false;
-    ctx->proj->toep64_valid = false;
+    for (auto& t : ctx->proj->toep) t.valid = false;
     ctx->proj->nb = 0;
 }
 
@@ -2101,14 +1991,17 @@ void free_proj(opsec_ctx* ctx) {
     dev_free((void**)&ctx->proj->d_trig);
     dev_free((void**)&ctx->proj->d_W);
     dev_free((void**)&ctx->proj->d_gmap64);
-    dev_free((void**)&ctx->proj->d_slab);
     dev_free((void**)&ctx->proj->d_trig64);
     dev_free((void**)&ctx->proj->d_W64);
-    dev_free((void**)&ctx->proj->d_Bg64);
-    dev_free((void**)&ctx->proj->d_Bhat64);
-    dev_free((void**)&ctx->proj->d_Yhat64);
-    dev_free((void**)&ctx->proj->d_Y64);
-    dev_free((void**)&ctx->proj->d_That64);
+    for (auto& t : ctx->proj->toep) {
+        dev_free(&t.Bg);
+        dev_free(&t.Bhat);
+        dev_free(&t.Yhat);
+        dev_free(&t.Y);
+    }
+    dev_free((void**)&ctx->proj->d_Bw32);
+    dev_free(&ctx->proj->d_T);
+    dev_free(&ctx->proj->ws.p);
     delete ctx->proj;
     ctx->proj = nullptr;
 }
@@ -2133,18 +2026,18 @@ int opsec_modes_upload(opsec_ctx* ctx, const double* B, int ncells, int nmodes) 
     dev_free((void**)&ctx->d_B);
     size_t capB = 0;
     if ((rc = dev_realloc(ctx, (void**)&ctx->d_B, &capB, bytes))) return rc;
-    ps->ldw = (size_t)ncells + 32;
+    ps->ldw = nt_pitch<double>(ncells);
     if ((rc = dev_realloc(ctx, (void**)&ps->d_Bw, &ps->cap_Bw, ps->ldw * nmodes * 8))) return rc;
     OPSEC_HIP_TRY(ctx, hipMemcpyAsync(ctx->d_B, B, bytes, hipMemcpyHostToDevice, ctx->stream));
-    size_t tot = (size_t)ncells * nmodes;
-    hipLaunchKernelGGL(scale_rows_kernel, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, ctx->stream, ctx->d_B,
+    hipLaunchKernelGGL(scale_rows_kernel<double>, blocks_for(ps->ldw * nmodes), dim3(256), 0, ctx->stream, ctx->d_B,
                        ctx->d_nbar, ncells, nmodes, ps->d_Bw, ps->ldw);
     OPSEC_HIP_TRY(ctx, hipGetLastError());
     OPSEC_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     ctx->nmodes = nmodes;
     ps->bp_valid = false;
+    ps->bw32_valid = false;
     ps->toep_valid = false;
-    ps->toep64_valid = false;
+    for (auto& t : ps->toep) t.valid = false;
     return OPSEC_OK;
 }
 
@@ -2273,40 +2166,16 @@ int opsec_project_dense(opsec_ctx* ctx, int n, const double* S, int nmodes, cons
     OPSEC_HIP_TRY(ctx, hipSetDevice(ctx->device));
     const int N = n, M = nmodes;
     double *dS = nullptr, *dB = nullptr, *dP = nullptr;
-    void* dC = nullptr;
-    size_t esize = prec == OPSEC_PREC_FP64 ? 8 : 4;
     DevScratch tmp;
     OPSEC_HIP_TRY(ctx, tmp.alloc(&dS, (size_t)N * N * 8));
     OPSEC_HIP_TRY(ctx, tmp.alloc(&dB, (size_t)N * M * 8));
-    OPSEC_HIP_TRY(ctx, tmp.alloc(&dC, (size_t)N * M * esize));
     OPSEC_HIP_TRY(ctx, tmp.alloc(&dP, (size_t)packed_size(M) * 8));
     OPSEC_HIP_TRY(ctx, hipMemcpyAsync(dS, S, (size_t)N * N * 8, hipMemcpyHostToDevice, ctx->stream));
     OPSEC_HIP_TRY(ctx, hipMemcpyAsync(dB, B, (size_t)N * M * 8, hipMemcpyHostToDevice, ctx->stream));
-    GA_RowMajor A;
-    A.p = dS;
-    A.ld = N;
-    GB_ColMajor Bop;
-    Bop.p = dB;
-    Bop.ld = N;
-    GA_ColMajorT A2;
-    A2.p = dB;
-    A2.ld = N;
-    PutPacked outP{dP, (size_t)packed_size(M)};
-    dim3 g1 = grid_for(N, M, 1), g2 = grid_for(M, M, 1);
-    if (prec == OPSEC_PREC_FP64) {
-        PutColMajor<double> outC{(double*)dC, (size_t)N, 0};
-        hipLaunchKernelGGL((gemm_kernel<double, GA_RowMajor, GB_ColMajor, PutColMajor<double>, false>), g1,
-                           dim3(GT_THREADS), 0, ctx->stream, A, 0, Bop, 0, outC, N, M, N);
-        GB_ColMajorT<double> B2{(const double*)dC, (size_t)N};
-        hipLaunchKernelGGL((gemm_kernel<double, GA_ColMajorT, GB_ColMajorT<double>, PutPacked, true>), g2,
-                           dim3(GT_THREADS), 0, ctx->stream, A2, 0, B2, 0, outP, M, M, N);
-    } else if (prec == OPSEC_PREC_FP32) {
-        PutColMajor<float> outC{(float*)dC, (size_t)N, 0};
-        hipLaunchKernelGGL((gemm_kernel<float, GA_RowMajor, GB_ColMajor, PutColMajor<float>, false>), g1,
-                           dim3(GT_THREADS), 0, ctx->stream, A, 0, Bop, 0, outC, N, M, N);
-        GB_ColMajorT<float> B2{(const float*)dC, (size_t)N};
-        hipLaunchKernelGGL((gemm_kernel<float, GA_ColMajorT, GB_ColMajorT<float>, PutPacked, true>), g2,
-                           dim3(GT_THREADS), 0, ctx->stream, A2, 0, B2, 0, outP, M, M, N);
+    if (prec != OPSEC_PREC_BF16X3) {
+        int rc = prec == OPSEC_PREC_FP64 ? project_host_nt<double>(ctx, N, dS, M, dB, dP)
+                                         : project_host_nt<float>(ctx, N, dS, M, dB, dP);
+        if (rc) return rc;
     } else {
         const size_t Kp = round_up(N, 256), Mp = round_up(M, 256), Pp = plane_pitch(Kp);
         __bf16 *Sp = nullptr, *Bp = nullptr, *Cp = nullptr;

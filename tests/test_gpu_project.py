@@ -37,6 +37,50 @@ def test_project_dense_fp64(ctx, n, m):
     np.testing.assert_allclose(got, ref, rtol=1e-11, atol=1e-11 * np.abs(ref).max())
 
 
+# one tile and less, one row or k-step over a tile, a K range long enough to be
+# split over the CUs, and more than one tile each way
+@pytest.mark.parametrize("n,m", [(1, 1), (15, 15), (16, 3), (17, 17), (33, 32), (128, 1), (129, 128), (255, 129),
+                                 (1025, 130), (2050, 257)])
+def test_project_dense_tile_edges(ctx, n, m):
+    """The projection GEMM at the edges of its tiles and k-steps, FP64 and FP32:
+    an entry sums n^2 products of order-one terms, so its rounding error is a few
+    eps sqrt(n) of the largest entry (bound: 16 eps sqrt(n) + the operands' own
+    rounding, 4 eps)."""
+    S = rand_sym(n, n + m)
+    B = np.random.default_rng(m).normal(size=(m, n))
+    P = B @ S @ B.T
+    ref = np.array([P[i, j] for j in range(m) for i in range(j + 1)])
+    for prec, eps in ((lib.OPSEC_PREC_FP64, 2.0 ** -53), (lib.OPSEC_PREC_FP32, 2.0 ** -24)):
+        got = ctx.project_dense(S, B, prec)
+        tol = (16 * np.sqrt(n) + 4) * eps * max(np.abs(ref).max(), n)
+        assert np.abs(got - ref).max() <= tol, (prec, np.abs(got - ref).max(), tol)
+
+
+def test_toeplitz_fp64_long_slabs_vs_dense(ctx):
+    """A flat box (4 x 96 x 96, one band): its slab matrices exceed one launch's
+    2 GiB and its T_p takes several panels, so both projections work on row
+    ranges; they agree to rounding."""
+    cells = synth.box_cells(96, 0.0, 960.0)
+    cells = cells[cells["d1"] < 4].copy()
+    cells["a"] = np.arange(len(cells))
+    sv = lib.survey_box(96, 0.0, 960.0, L=1e9)
+    sv.n1, sv.max1 = 4, 40.0
+    lo, hi = synth.linear_bands(1, 0.02, 0.03)
+    ctx.model_real(GOLD["pk_k"], GOLD["pk_P"], lo, hi, lib.OPSEC_XI_CLOSED)
+    ctx.cells_upload(cells, sv)
+    ctx.pair_tables([1], ctx.quad(lib.OPSEC_QUAD_GAUSS, nodes=4, near=1))
+    B = np.random.default_rng(5).normal(size=(24, len(cells)))
+    ctx.modes_upload(B)
+    ref = ctx.project([1], lib.OPSEC_PREC_FP64)[0]
+    try:
+        ctx.set_projection(lib.OPSEC_PROJ_TOEPLITZ)
+        got = ctx.project([1], lib.OPSEC_PREC_FP64)[0]
+    finally:
+        ctx.set_projection(lib.OPSEC_PROJ_DENSE)
+    assert np.abs(ref).max() > 0
+    assert np.abs(got - ref).max() <= 1e-12 * np.abs(ref).max()
+
+
 @pytest.mark.parametrize("prec,tol", [(lib.OPSEC_PREC_FP32, 2e-5), (lib.OPSEC_PREC_BF16X3, 5e-5)])
 def test_project_dense_mixed(ctx, prec, tol):
     n, m = 400, 96
