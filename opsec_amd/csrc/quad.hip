@@ -9,12 +9,12 @@
 // atomicMin per (row, col).
 //
 // Methods:
-//  GM     one wavefront per integral: the Genz-Malik degree-7/5 embedded rule
+//  GM     one workgroup (or thread) per integral: the Genz-Malik degree-7/5 embedded rule
 //         (Genz & Malik 1980, 149 nodes in 6-D) with h-adaptive bisection of
 //         the worst regions, max-error binary heap and Gladwell's batch
 //         selection, run with the reference's arguments (epsrel lands in the
 //         absolute slot, epsabs in the relative slot: src/sig.cpp:427-430 vs
-//         src/cubature.h:70-73).  The 149 values are summed by one lane in the
+//         src/cubature.h:70-73).  The 149 values are summed in the
 //         reference's node order so that equal xi values give equal sums.
 //  GAUSS  exact tent-kernel reduction of the 6-D cube-pair mean to 3-D:
 //           Q = int xi(|mi(D + s)|) prod_i T(s_i) ds,  T(s) = (1-|s|/h)/h,
@@ -63,6 +63,9 @@ struct GMJobs {
         J.f = funcs[t];
         return J;
     }
+    // the same without a copy: job j's record, its function
+    __device__ __forceinline__ const GMJob* at(int j) const { return funcs ? p + j % npairs : p + j; }
+    __device__ __forceinline__ int func(int j) const { return funcs ? funcs[j / npairs] : p[j].f; }
 };
 
 struct GaussJob {
@@ -86,8 +89,9 @@ struct TentRule {
     double w[64];          // weights, sum 1
 };
 
-// ---- GM: one wavefront per integral ----------------------------------------
+// ---- GM: the adaptive driver's region pools ------------------------------------
 
+// Region store of an integral in a thread's private memory (gm_thread_kernel).
 struct GMSlot {
     double* c;       // 6 x R centres
     double* hw;      // 6 x R half-widths
@@ -99,20 +103,12 @@ struct GMSlot {
     int* list;       // R
 };
 
-__device__ __forceinline__ GMSlot gm_slot(double* dpool, int* ipool, int slot, int R) {
-    GMSlot s;
-    double* d = dpool + (size_t)slot * 15 * R;
-    int* q = ipool + (size_t)slot * 3 * R;
-    s.c = d;
-    s.hw = d + 6 * R;
-    s.val = d + 12 * R;
-    s.err = d + 13 * R;
-    s.hkey = d + 14 * R;
-    s.split = q;
-    s.heap = q + R;
-    s.list = q + 2 * R;
-    return s;
-}
+// Region pool of an integral in HBM (gm_kernel): a 128-byte record per region
+// (6 centres, 6 half-widths, value, split axis), so that one 16-lane access moves
+// a region, then the heap's keys and indices and the current batch's list.
+constexpr int GM_REC = 16;
+enum { GM_REC_VAL = 12, GM_REC_SPLIT = 13 };
+constexpr size_t GM_SLOT_DOUBLES = GM_REC + 1, GM_SLOT_INTS = 2;   // per region
 
 __device__ __forceinline__ double gm_integrand(const XiModelDev& m, const XiDesc& xd, const GMJob& J,
                                                const GMParams& P, const double* u) {
@@ -239,7 +235,8 @@ struct SphIdx {
 // Table entries of region (c, hw) of job J (src/sig.cpp:436-462 mapping:
 // lo/hi = {r1^3, r2^3, mu1, mu2, phi1, phi2}); entry e of SPH_TAB, with the
 // phi values it needs formed on the spot.
-__device__ __forceinline__ double sph_entry(const GMJob& J, const double* c, const double* hw, int e) {
+template <typename Bounds>
+__device__ __forceinline__ double sph_entry(const Bounds& J, const double* c, const double* hw, int e) {
     auto w = [&](int d, int v) {
         const double u = gm_axis_value(c[d], hw[d], v);
         return (1 - u) * J.lo[d] + u * J.hi[d];
@@ -305,87 +302,19 @@ __device__ __forceinline__ void gm_region_sum(const double* vals, const double* 
     err = fabs(res5th - result);
 }
 
-constexpr int GM_SUB = 16;   // regions evaluated together by one wavefront
-
-// Evaluate the regions list[0..n): GM_SUB at a time, the lanes share out their
-// GM_SUB x 149 nodes, then lane t forms the rule of region t.
-__device__ void gm_eval_regions(const XiModelDev& m, const XiDesc& xd, const GMJob& J, const GMParams& P,
-                                GMSlot& S, int R, const int* list, int n, double (*vals)[GM_NPTS],
-                                double (*tab)[SPH_TAB]) {
-    const int lane = threadIdx.x;
-    const bool sph = P.coordsys != OPSEC_COORD_CARTESIAN;
-    for (int t0 = 0; t0 < n; t0 += GM_SUB) {
-        const int nt = min(GM_SUB, n - t0);
-        if (sph) {   // the regions' tables, then the nodes from them
-            for (int i = lane; i < nt * SPH_TAB; i += blockDim.x) {
-                const int t = i / SPH_TAB, e = i - t * SPH_TAB;
-                const int ri = list[t0 + t];
-                double c[6], hw[6];
-                for (int d = 0; d < 6; d++) {
-                    c[d] = S.c[d * R + ri];
-                    hw[d] = S.hw[d * R + ri];
-                }
-                tab[t][e] = sph_entry(J, c, hw, e);
-            }
-            __syncthreads();
-            for (int i = lane; i < nt * GM_NPTS; i += blockDim.x) {
-                const int t = i / GM_NPTS, p = i - t * GM_NPTS;
-                vals[t][p] = sph_node_value(m, xd, tab[t], p);
-            }
-        } else {
-            for (int i = lane; i < nt * GM_NPTS; i += blockDim.x) {
-                const int t = i / GM_NPTS, p = i - t * GM_NPTS;
-                const int ri = list[t0 + t];
-                double c[6], hw[6], u[6];
-                for (int d = 0; d < 6; d++) {
-                    c[d] = S.c[d * R + ri];
-                    hw[d] = S.hw[d * R + ri];
-                }
-                gm_node(p, c, hw, u);
-                vals[t][p] = gm_integrand(m, xd, J, P, u);
-            }
-        }
-        __syncthreads();
-        if (lane < nt) {
-            const int ri = list[t0 + lane];
-            double hw[6];
-            for (int d = 0; d < 6; d++) hw[d] = S.hw[d * R + ri];
-            double result, err;
-            int split;
-            gm_region_sum(vals[lane], hw, result, err, split);
-            S.val[ri] = result;
-            S.err[ri] = err;
-            S.split[ri] = split;
-        }
-        __syncthreads();
-    }
-}
-
-// Binary max-heap on region errors (Cormen-Leiserson-Rivest), lane 0 only.
-// Storage of the region heap: position p holds region idx(p) with key(p) =
-// its error, keys beside the indices so a sift level costs independent loads.
-// Positions below nl sit in LDS (the top levels, which every pop walks), the
-// rest in the slot's arrays.
+// Binary max-heap on region errors (Cormen-Leiserson-Rivest) of one thread:
+// position p holds region idx(p) with key(p) = its error.
 struct HeapStore {
     double* gk;
     int* gi;
-    double* lk;
-    int* li;
-    int nl;
-    __device__ __forceinline__ double key(int p) const { return p < nl ? lk[p] : gk[p]; }
-    __device__ __forceinline__ int idx(int p) const { return p < nl ? li[p] : gi[p]; }
+    __device__ __forceinline__ double key(int p) const { return gk[p]; }
+    __device__ __forceinline__ int idx(int p) const { return gi[p]; }
     __device__ __forceinline__ void set(int p, double k, int i) const {
-        if (p < nl) {
-            lk[p] = k;
-            li[p] = i;
-        } else {
-            gk[p] = k;
-            gi[p] = i;
-        }
+        gk[p] = k;
+        gi[p] = i;
     }
 };
 
-// Binary max-heap on region errors (Cormen-Leiserson-Rivest), one lane.
 __device__ void heap_push(const GMSlot& S, const HeapStore& H, int& n, int ri, double& tv, double& te) {
     tv += S.val[ri];
     te += S.err[ri];
@@ -432,123 +361,558 @@ __device__ __forceinline__ bool gm_converged(double val, double err, const GMPar
     return err <= P.absTol || rel <= P.relTol;
 }
 
-// One wavefront per integral; jobs idx[0..njobs) (all jobs when idx is null)
-// are taken from a counter.
-// NT threads per integral: 64 in the first pass; in the rerun of the deep
-// integrals, whose split batches are short and follow one another, up to 512
-// when there are few of them, so the nodes of a batch are spread over more
-// lanes while all of them stay resident.
-// NL > 0: the first NL heap positions in LDS.  A register limit of 256 per
-// wave (two waves per SIMD by registers; the LDS of the 64-thread variant holds
-// five per CU): 11 % faster on the shell's prior than 262 registers.
-template <int NT, int NL>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void gm_kernel(XiModelDev m, GMJobs jobs, const int* idx, int njobs,
-                                                int* counter, double* dpool, int* ipool, GMParams P, double* Q,
-                                                size_t qstride, double* Qerr, int* jobfail,
-                                                unsigned long long* nevals) {
-    __shared__ double vals[GM_SUB][GM_NPTS];
-    __shared__ double sphtab[GM_SUB][SPH_TAB];
-    __shared__ double lkey[NL > 0 ? NL : 1];
-    __shared__ int lidx[NL > 0 ? NL : 1];
-    __shared__ int sh_job, sh_nR, sh_done;
-    const int lane = threadIdx.x;
+// ---- GM: one workgroup per integral ----------------------------------------------
+//
+// The driver's chain per split -- pop the worst region, cut it, evaluate the two
+// halves, push them -- is sequential, so an integral's time is the chain's latency
+// (a self pair of the 12^3 box: 36 700 splits).  Wave 0 runs the chain with all its
+// lanes; every value, comparison and sum is the serial driver's, in its order.
+
+// Lane `l`'s value of x in every lane (l uniform).
+__device__ __forceinline__ double lane_f64(double x, int l) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
+    const unsigned lo = __builtin_amdgcn_readlane((unsigned)b, l), hi = __builtin_amdgcn_readlane((unsigned)(b >> 32), l);
+    return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+}
+__device__ __forceinline__ int lane_i32(int x, int l) { return __builtin_amdgcn_readlane(x, l); }
+// Value of the neighbouring lane (lane ^ 1).
+__device__ __forceinline__ double pair_f64(double x) {
+    const unsigned long long b = __builtin_bit_cast(unsigned long long, x);
+    const unsigned lo = __builtin_amdgcn_mov_dpp((unsigned)b, 0xB1, 0xF, 0xF, true);
+    const unsigned hi = __builtin_amdgcn_mov_dpp((unsigned)(b >> 32), 0xB1, 0xF, 0xF, true);
+    return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+}
+// Workgroup barrier for data in LDS: unlike __syncthreads it does not wait for
+// this wave's outstanding stores to the pool, which only wave 0 reads.
+__device__ __forceinline__ void lds_barrier() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+// Order of one wave's own accesses across its lanes (they issue in order).
+__device__ __forceinline__ void wave_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
+
+// Max-heap of region errors worked by one wavefront: the same array, element for
+// element, as the serial sift of HeapStore's heap_push / heap_pop.  Positions below
+// nl sit in LDS, the rest in the slot's arrays.
+struct WaveHeap {
+    double* gk;
+    int* gi;
+    double* lk;
+    int* li;
+    int nl;
+    __device__ __forceinline__ double key(int p) const { return p < nl ? lk[p] : gk[p]; }
+    __device__ __forceinline__ int idx(int p) const { return p < nl ? li[p] : gi[p]; }
+    __device__ __forceinline__ void set(int p, double k, int i) const {
+        if (p < nl) {
+            lk[p] = k;
+            li[p] = i;
+        } else {
+            gk[p] = k;
+            gi[p] = i;
+        }
+    }
+    // Sift up from position n: lane l holds the l-th ancestor; those below the first
+    // one that is not smaller move down one step, all at once.
+    __device__ __forceinline__ void push(int lane, int& n, double k, int ri) const {
+        const unsigned q = (unsigned)n + 1;
+        n++;
+        const unsigned a = lane < 31 ? q >> (lane + 1) : 0u;   // ancestor's position + 1
+        const bool have = a >= 1;
+        double pk = 0.0;
+        int pi = 0;
+        if (have) {
+            pk = key((int)a - 1);
+            pi = idx((int)a - 1);
+        }
+        const int f = __builtin_ctzll(__ballot(!have || k <= pk));
+        wave_order();
+        if (lane < f) set((int)(q >> lane) - 1, pk, pi);
+        if (lane == 0) set((int)(q >> f) - 1, k, ri);
+        wave_order();
+    }
+    // The element at the end of the heap, loaded ahead of the pop that moves it.
+    struct Last {
+        double k = 0;
+        int i = 0, pos = -1;
+    };
+    __device__ __forceinline__ void fetch_last(int n, Last& e) const {
+        e.pos = n - 1;
+        if (n > 0) {
+            e.k = key(n - 1);
+            e.i = idx(n - 1);
+        }
+    }
+    // Remove the root; returns its region, its key in *rk.  The last element sifts
+    // down the path of larger children, five levels (62 positions, one per lane) at a
+    // time: each lane tests whether it beats its sibling and the sifted key, a lane is
+    // on the path if it and its ancestors in the chunk (mask anc) do, and every
+    // element on the path moves up one level at once.
+    __device__ __forceinline__ int pop(int lane, unsigned long long anc, int& n, double* rk, Last& e) const {
+        const int ret = idx(0);
+        *rk = key(0);
+        if (e.pos != n - 1) fetch_last(n, e);
+        const int m = --n;
+        const double ki = e.k;
+        const int ii = e.i;
+        const int lev = 31 - __builtin_clz(lane + 2), off = lane + 2 - (1 << lev);
+        int i = 0;
+        for (;;) {
+            const int pos = ((i + 1) << lev) - 1 + off;
+            const bool have = lane < 62 && pos < m;
+            double kk = 0.0;
+            int id = 0;
+            if (have) {
+                kk = key(pos);
+                id = idx(pos);
+            }
+            const double ks = pair_f64(kk);
+            // the right child only if it exists and is larger
+            const bool beats = (lane & 1) ? ks < kk : !(pos + 1 < m && kk < ks);
+            const unsigned long long W = __ballot(have && beats && !(kk <= ki));
+            const bool on = (W & anc) == anc;
+            const unsigned long long path = __ballot(on);
+            wave_order();
+            if (on) set((pos - 1) >> 1, kk, id);
+            if (path == 0) break;
+            const int last = 63 - __builtin_clzll(path);
+            i = lane_i32(pos, last);
+            if (last < 30) break;   // the path ended above the chunk's last level
+        }
+        if (lane == 0) set(i, ki, ii);
+        wave_order();
+        fetch_last(n, e);
+        return ret;
+    }
+};
+// Lanes of this lane's position and its ancestors within a five-level chunk (level
+// l starts at lane 2^l - 2; lane c's children are 2 c + 2 and 2 c + 3); lanes 62 and
+// 63 hold no position and can never match.
+__device__ __forceinline__ unsigned long long heap_chunk_ancestors(int lane) {
+    if (lane >= 62) return ~0ull;
+    unsigned long long a = 0;
+    for (int c = lane;; c = (c - 2) >> 1) {
+        a |= 1ull << c;
+        if (c < 2) break;
+    }
+    return a;
+}
+
+// QSpline table of the current function in LDS.
+struct XiLds {
+    double y[QS_N];
+    double u[QS_N2];
+};
+
+// xi_eval with a table function's nodes in LDS, the same bits.  Below 200 the
+// nodes are i h, h = 200 / 512 = 0.390625 exactly, so lookup_index's interval is
+// floor(r / h), and the division by x2 - x1 = h is the correctly rounded quotient
+// from the reciprocal and one remainder step (Markstein: q + rem / h rounded once;
+// a quotient by 25/64 is never near a midpoint).
+__device__ __forceinline__ double xi_eval_lds(const XiModelDev& m, const XiDesc& d, const XiLds* t, double r) {
+    if (d.kind == XI_TABLE) {
+        if (r >= 0 && r < QS_X1) {
+            constexpr double h = 0.390625, rh = 2.56;
+            int i = (int)(r * rh);
+            i -= r < i * h ? 1 : 0;
+            i += r >= (i + 1) * h ? 1 : 0;
+            const double y1 = t->y[i], y2 = t->y[i + 1];
+            const double a = __dmul_rn(y2 - y1, r - i * h);
+            double q = a * rh;
+            if (fabs(q) > 1e-280 && fabs(q) < 1e280) q = __builtin_fma(__builtin_fma(-q, h, a), rh, q);
+            else q = __ddiv_rn(a, h);
+            return y1 + q;
+        }
+        if (r >= 0 && r < m.x2) return linear_spline(log(r), QS_N2, t->u, t->y + QS_N1);
+    }
+    return xi_eval(m, d, r);
+}
+
+// Entries of a region's coordinate table: 42 for a box (six axes x the seven values
+// of gm_axis_value, mapped to the cell), SPH_TAB for a shell (sph_entry).
+constexpr int BOX_TAB = 42;
+template <typename Bounds>
+__device__ __forceinline__ double box_entry(const Bounds& B, const double* g, int e) {
+    const int d = e / 7;
+    const double u = gm_axis_value(g[d], g[6 + d], e - 7 * d);
+    return (1 - u) * B.lo[d] + u * B.hi[d];
+}
+
+// xi at the node with value indices vi (3 bits per axis).
+__device__ __forceinline__ double gm_node_value(const XiModelDev& m, const XiDesc& xd, const XiLds* xt, const double* T,
+                                                unsigned vi, bool sph, double L) {
+    const int v0 = vi & 7, v1 = (vi >> 3) & 7, v2 = (vi >> 6) & 7, v3 = (vi >> 9) & 7, v4 = (vi >> 12) & 7,
+              v5 = (vi >> 15) & 7;
+    if (!sph)
+        return xi_eval_lds(m, xd, xt,
+                           box_r(T[v0], T[7 + v1], T[14 + v2], T[21 + v3], T[28 + v4], T[35 + v5], L));
+    const double r1 = T[SphIdx::R1 + v0], r2 = T[SphIdx::R2 + v1];
+    const double cosg = T[SphIdx::SQ + sph_cmb(v2, v3)] * T[SphIdx::CS + sph_cmb(v4, v5)] +
+                        T[SphIdx::M1 + v2] * T[SphIdx::M2 + v3];
+    return xi_eval_lds(m, xd, xt, sqrt(fmax(r1 * r1 + r2 * r2 - 2 * r1 * r2 * cosg, 0.0)));
+}
+
+// One of the four chains of region t's rule, in gm_region_sum's order: the 60 values
+// of sum4 (role 0), the 64 of sum5 (1), the axis sums and split axis (2), the volume (3).
+__device__ __forceinline__ void gm_role_sum(const double* v, const double* g, int role, double (*part)[5], int t) {
+    const double ratio = (GM_L2 * GM_L2) / (GM_L4 * GM_L4);
+    if (role < 2) {
+        const double* x = v + (role ? 85 : 25);
+        double acc = 0;
+#pragma unroll 20
+        for (int k = 0; k < 60; k++) acc += x[k];
+        if (role)
+#pragma unroll
+            for (int k = 60; k < 64; k++) acc += x[k];
+        part[t][role] = acc;
+    } else if (role == 2) {
+        const double val0 = v[0];
+        double sum2 = 0, sum3 = 0, maxdiff = 0;
+        int split = 0;
+#pragma unroll
+        for (int k = 0; k < 6; k++) {
+            const double v0 = v[1 + 4 * k], v1 = v[2 + 4 * k], v2 = v[3 + 4 * k], v3 = v[4 + 4 * k];
+            sum2 += v0 + v1;
+            sum3 += v2 + v3;
+            const double diff = 0.0 + fabs(v0 + v1 - 2 * val0 - ratio * (v2 + v3 - 2 * val0));
+            if (diff > maxdiff) {
+                maxdiff = diff;
+                split = k;
+            }
+        }
+        part[t][2] = sum2;
+        part[t][3] = sum3;
+        part[t][4] = (double)split;
+    }
+}
+// The rule of a region from its chains (part) and its value at the centre.
+__device__ __forceinline__ void gm_combine(const double* part, double val0, const double* g, double& result, double& err) {
+    const double w1 = (double)(12824 - 9120 * 6 + 400 * 36) / 19683.0;
+    const double w2 = 980. / 6561.;
+    const double w3 = (double)(1820 - 400 * 6) / 19683.0;
+    const double w4 = 200. / 19683.;
+    const double w5 = 6859.0 / 19683.0 / 64.0;
+    const double e1 = (double)(729 - 950 * 6 + 50 * 36) / 729.0;
+    const double e2 = 245. / 486.;
+    const double e3 = (double)(265 - 100 * 6) / 1458.0;
+    const double e4 = 25. / 729.;
+    const double sum4 = part[0], sum5 = part[1], sum2 = part[2], sum3 = part[3];
+    double vol = 1;
+    for (int d = 0; d < 6; d++) vol *= 2 * g[6 + d];
+    result = vol * (w1 * val0 + w2 * sum2 + w3 * sum3 + w4 * sum4 + w5 * sum5);
+    const double res5th = vol * (e1 * val0 + e2 * sum2 + e3 * sum3 + e4 * sum4);
+    err = fabs(res5th - result);
+}
+
+// gm_converged without its division where the quotient is clearly above the
+// relative tolerance.
+__device__ __forceinline__ bool gm_converged_quick(double val, double err, const GMParams& P) {
+    if (err > P.absTol && fabs(err) > 2 * P.relTol * fabs(val)) return false;
+    return gm_converged(val, err, P);
+}
+
+// NT threads per integral; jobs idx[0..njobs) (all jobs when idx is null) are taken
+// from a counter.  Wave 0 runs the driver: it pops and cuts the batch's regions into
+// LDS (the first SUB) and the pool, and later pushes their results.  The worker waves
+// (all of them with one wave) evaluate the batch SUB regions at a time: coordinate
+// tables (14 cbrt, 17 sqrt and 17 cos of a shell's region, one thread per entry),
+// nodes (one thread per node), the rules' chains (one wave per chain); meanwhile wave
+// 0 pushes the previous chunk.  The pool in HBM holds a record per region and the
+// heap below its first NL positions; the record of a popped region is loaded under
+// the next pop, and the next root's under the batch's evaluation.
+//
+// Bound by wave 0's chain of dependent heap accesses: a 12^3 box's self pair (36 675
+// splits in 38 batches) takes 2.2 us per split (83 ms), 10.4 us with one lane running the
+// heap, the geometry in twelve arrays and the node values formed from the unit cube
+// (380 ms).
+template <int NT, int NL, int SUB>
+__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void gm_kernel(
+    XiModelDev m, GMJobs jobs, const int* idx, int njobs, int* counter, double* dpool, int* ipool, GMParams P, double* Q,
+    size_t qstride, double* Qerr, int* jobfail, unsigned long long* nevals) {
+    constexpr bool SOLO = NT == 64;
+    constexpr int W0 = SOLO ? 0 : 64, NW = NT - W0;                      // the workers: threads W0 .. NT - 1
+    constexpr int RS = NW >= GM_NPTS ? NW / GM_NPTS : 1;                 // regions per sweep over the nodes
+    constexpr int NP = NW >= GM_NPTS ? 1 : (GM_NPTS + NW - 1) / NW;      // nodes of a region per thread
+    constexpr int CH = SUB * GM_NPTS / 2;                                // heap entries summed at once
+    static_assert(SUB % 2 == 0 && SUB <= 16, "batches are region pairs; four lanes each in one wave");
+    __shared__ double vals[SUB][GM_NPTS];
+    __shared__ double tab[SUB][SPH_TAB];
+    __shared__ double geo[2][SUB][GM_REC];   // records of two chunks
+    __shared__ double part[2][SUB][5];       // rule chains of two chunks, and their centre values
+    __shared__ double cval[2][SUB];
+    __shared__ int list[2][SUB];
+    __shared__ double lkey[NL];
+    __shared__ int lidx[NL];
+    __shared__ XiLds xt;
+    __shared__ struct {
+        double lo[6], hi[6];
+    } B;   // the integral's bounds
+    __shared__ int sh_job, sh_nR, sh_done, sh_nheap;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool driver = wave == 0, worker = SOLO || wave > 0;
     const int R = P.rmax;
-    GMSlot S = gm_slot(dpool, ipool, blockIdx.x, R);
-    const HeapStore H{S.hkey, S.heap, lkey, lidx, NL < R ? NL : R};
+    const bool sph = P.coordsys != OPSEC_COORD_CARTESIAN;
+    const int te = sph ? SPH_TAB : BOX_TAB;
+    double* rec = dpool + (size_t)blockIdx.x * GM_SLOT_DOUBLES * R;
+    int* glist = ipool + (size_t)blockIdx.x * GM_SLOT_INTS * R + R;
+    const WaveHeap H{rec + (size_t)GM_REC * R, ipool + (size_t)blockIdx.x * GM_SLOT_INTS * R, lkey, lidx, NL < R ? NL : R};
+    const unsigned long long anc = heap_chunk_ancestors(lane);
+    // this worker's nodes: region slot tr of a sweep, nodes p0 + q NW
+    const int wt = tid - W0, tr = NW >= GM_NPTS ? wt / GM_NPTS : 0, p0 = wt - tr * GM_NPTS;
+    unsigned vis[NP];
+    for (int q = 0; q < NP; q++) {
+        int vi[6];
+        gm_node_vi(max(0, min(p0 + q * NW, GM_NPTS - 1)), vi);
+        vis[q] = vi[0] | vi[1] << 3 | vi[2] << 6 | vi[3] << 9 | vi[4] << 12 | vi[5] << 15;
+    }
+    int xt_table = -1;
     for (;;) {
-        if (lane == 0) sh_job = atomicAdd(counter, 1);
+        if (tid == 0) sh_job = atomicAdd(counter, 1);
         __syncthreads();
         const int jl = sh_job;
-        __syncthreads();
         if (jl >= njobs) break;
         const int jb = idx ? idx[jl] : jl;
-        const GMJob J = jobs.get(jb);
-        const XiDesc xd = m.desc[J.f];
-        // region 0 = [0,1]^6
-        if (lane < 6) {
-            S.c[lane * R] = 0.5;
-            S.hw[lane * R] = 0.5;
+        const int f = jobs.func(jb), key = jobs.at(jb)->key;
+        const XiDesc xd = m.desc[f];
+        if (tid < 6) {
+            B.lo[tid] = jobs.at(jb)->lo[tid];
+            B.hi[tid] = jobs.at(jb)->hi[tid];
         }
-        if (lane == 0) S.list[0] = 0;
-        __syncthreads();
-        gm_eval_regions(m, xd, J, P, S, R, S.list, 1, vals, sphtab);
-        // lane-0 state (heap size, totals, evaluation count)
-        int nheap = 0, nregions = 1;
-        double tv = 0, te = 0;
+        if (xd.kind == XI_TABLE && xd.table != xt_table) {
+            for (int i = tid; i < QS_N; i += NT) xt.y[i] = m.y[(size_t)xd.table * QS_N + i];
+            for (int i = tid; i < QS_N2; i += NT) xt.u[i] = m.ugrid[i];
+            xt_table = xd.table;
+        }
+        // the driver's state: heap size and last element, regions used, totals,
+        // evaluations, the prefetched record of the heap's root; gb: the buffer of the
+        // batch's first chunk (all waves)
+        int nheap = 0, nregions = 1, gb = 0, preidx = -1, status = 0;
+        WaveHeap::Last last;
+        double tv = 0, te_sum = 0, pre = 0;
         unsigned numEval = GM_NPTS;
-        if (lane == 0) heap_push(S, H, nheap, 0, tv, te);
-        int status = 0;
-        for (;;) {
-            if (lane == 0) {
-                int done = 0, nR = 0;
-                if (!(numEval < P.maxEval || !P.maxEval)) done = 1;
-                else if (gm_converged(tv, te, P)) done = 1;
-                else {
-                    double eev = tv, eee = te;
-                    do {
-                        if (nregions + 1 > R) {   // pool exhausted
-                            done = 2;
-                            break;
-                        }
-                        int ri = heap_pop(S, H, nheap, tv, te);
-                        eee -= S.err[ri];
-                        // cut along the split dimension (src/cubature.c:210-224)
-                        int d = S.split[ri];
-                        int r2 = nregions++;
-                        // the region's geometry through registers: all 12 loads
-                        // first, so they overlap, then the stores
-                        double cc[6], hh[6];
-#pragma unroll
-                        for (int k = 0; k < 6; k++) {
-                            cc[k] = S.c[k * R + ri];
-                            hh[k] = S.hw[k * R + ri];
-                        }
-                        const double h = hh[d] * 0.5;
-#pragma unroll
-                        for (int k = 0; k < 6; k++) {
-                            S.c[k * R + r2] = k == d ? cc[k] + h : cc[k];
-                            S.hw[k * R + r2] = k == d ? h : hh[k];
-                        }
-                        S.hw[d * R + ri] = h;
-                        S.c[d * R + ri] = cc[d] - h;
-                        numEval += GM_NPTS * 2;
-                        S.list[nR++] = ri;
-                        S.list[nR++] = r2;
-                        if (gm_converged(eev, eee, P)) break;
-                    } while (nheap > 0 && (numEval < P.maxEval || !P.maxEval));
-                }
-                sh_nR = nR;
-                sh_done = done;
+        if (driver) {   // region 0 = [0,1]^6
+            if (lane < 12) {
+                geo[0][0][lane] = 0.5;
+                rec[lane] = 0.5;
             }
-            __syncthreads();
-            int nR = sh_nR, done = sh_done;
-            __syncthreads();
+            if (lane == 0) {
+                list[0][0] = 0;
+                sh_nR = 1;
+                sh_done = 0;
+            }
+        }
+        for (;;) {
+            lds_barrier();   // the batch's first chunk is in geo[gb], list[gb]
+            const int n = __builtin_amdgcn_readfirstlane(sh_nR), done = __builtin_amdgcn_readfirstlane(sh_done);
             if (done) {   // 2: region pool exhausted, the host reruns this job with a larger pool
                 status = done;
                 break;
             }
-            __threadfence_block();
-            gm_eval_regions(m, xd, J, P, S, R, S.list, nR, vals, sphtab);
-            if (lane == 0)
-                for (int t = 0; t < nR; t++) heap_push(S, H, nheap, S.list[t], tv, te);
-        }
-        if (lane == 0) {
-            if (status == 2) {
-                jobfail[jb] = 1;
-            } else {
-                double val = 0, err = 0;
-                for (int i = 0; i < nheap; i++) {
-                    val += S.val[H.idx(i)];
-                    err += S.err[H.idx(i)];
+            // results of chunk c (buffer b, nt regions): formed by the driver, then pushed
+            double rv = 0, re = 0;
+            int rl = 0;   // the chunk's regions, one per lane (list is refilled meanwhile)
+            auto combine = [&](int b, int nt) {
+                const int t = min(lane, nt - 1);
+                rl = list[b][t];
+                gm_combine(part[b][t], cval[b][t], geo[b][t], rv, re);
+                if (lane < nt) {
+                    double* r = rec + (size_t)rl * GM_REC;
+                    geo[b][t][GM_REC_VAL] = r[GM_REC_VAL] = rv;
+                    geo[b][t][GM_REC_SPLIT] = r[GM_REC_SPLIT] = part[b][t][4];
                 }
-                Q[(size_t)J.f * qstride + J.key] = val;
-                if (Qerr) Qerr[(size_t)J.f * qstride + J.key] = err;
-                jobfail[jb] = 0;
-                atomicAdd(nevals, (unsigned long long)numEval);
+            };
+            auto push = [&](int i0, int i1) {
+                for (int t = i0; t < i1; t++) {
+                    const double ke = lane_f64(re, t);
+                    tv += lane_f64(rv, t);
+                    te_sum += ke;
+                    H.push(lane, nheap, ke, lane_i32(rl, t));
+                }
+            };
+            const int nch = (n + SUB - 1) / SUB;
+            for (int c = 0; c < nch; c++) {
+                const int b = (gb + c) & 1, nt = min(SUB, n - c * SUB);
+                // with several waves the driver pushes chunk c - 1 (a full one) in three steps
+                const bool behind = !SOLO && driver && c > 0;
+                if (behind) {
+                    combine(b ^ 1, SUB);
+                    push(0, SUB / 3);
+                }
+                if (worker)
+                    for (int i = wt; i < nt * te; i += NW) {
+                        const int t = i / te, e = i - t * te;
+                        const double* g = geo[b][t];
+                        tab[t][e] = sph ? sph_entry(B, g, g + 6, e) : box_entry(B, g, e);
+                    }
+                lds_barrier();
+                if (behind) push(SUB / 3, 2 * SUB / 3);
+                if (worker && tr < RS)
+                    for (int t = tr; t < nt; t += RS)
+#pragma unroll
+                        for (int q = 0; q < NP; q++)
+                            if (p0 + q * NW < GM_NPTS)
+                                vals[t][p0 + q * NW] = gm_node_value(m, xd, &xt, tab[t], vis[q], sph, P.L);
+                lds_barrier();
+                if (behind) push(2 * SUB / 3, SUB);
+                // the rules' chains: a wave each, or four lanes per region with one wave
+                const int role = SOLO ? lane & 3 : wave - 1, t = SOLO ? lane >> 2 : lane;
+                if (worker && role < 3 && t < nt) {
+                    gm_role_sum(vals[t], geo[b][t], role, part[b], t);
+                    if (role == 0) cval[b][t] = vals[t][0];
+                }
+                if (SOLO) {
+                    wave_order();
+                    combine(b, nt);
+                    push(0, nt);
+                }
+                // the next chunk's regions from the pool, sixteen lanes per record
+                if ((SOLO || wave == (NT > 256 ? 4 : 1)) && c + 1 < nch) {
+                    const int n1 = min(SUB, n - (c + 1) * SUB), e = lane & 15;
+                    int ri[SUB / 4 + 1];
+                    double v[SUB / 4 + 1];
+#pragma unroll
+                    for (int u = 0; 4 * u < SUB; u++) {
+                        const int t1 = 4 * u + (lane >> 4);
+                        ri[u] = t1 < n1 ? glist[(c + 1) * SUB + t1] : 0;
+                    }
+#pragma unroll
+                    for (int u = 0; 4 * u < SUB; u++) v[u] = rec[(size_t)ri[u] * GM_REC + e];
+#pragma unroll
+                    for (int u = 0; 4 * u < SUB; u++) {
+                        const int t1 = 4 * u + (lane >> 4);
+                        if (t1 < n1) {
+                            if (e < 12) geo[b ^ 1][t1][e] = v[u];
+                            else if (e == 12) list[b ^ 1][t1] = ri[u];
+                        }
+                    }
+                }
+                lds_barrier();
+            }
+            const int bl = (gb + nch - 1) & 1, ntl = n - (nch - 1) * SUB;   // the last chunk
+            gb = bl ^ 1;                                                   // the next batch's first buffer
+            if (!driver) continue;
+            if (!SOLO) {
+                combine(bl, ntl);
+                push(0, ntl);
+            }
+            // the driver's decision and the next batch
+            int dn = 0, nb = 0;
+            const int lastn = nch == 1 ? n : 0;   // records still in geo[bl]
+            if (!(numEval < P.maxEval || !P.maxEval)) dn = 1;
+            else if (gm_converged(tv, te_sum, P)) dn = 1;
+            else {
+                const double eev = tv;
+                double eee = te_sum;
+                // cut region ri (record v, one element per lane) along its split dimension
+                // (src/cubature.c:210-224): lane k < 6 holds centre k, lane 6 + k half-width k
+                auto cut = [&](double v, int ri, int r2, int at) {
+                    tv -= lane_f64(v, GM_REC_VAL);
+                    const int d = __builtin_amdgcn_readfirstlane((int)lane_f64(v, GM_REC_SPLIT));
+                    const double h = lane_f64(v, 6 + d) * 0.5;
+                    const double va = lane == d ? v - h : lane == 6 + d ? h : v;
+                    const double vb = lane == d ? v + h : lane == 6 + d ? h : v;
+                    if (lane < 12) {
+                        rec[(size_t)ri * GM_REC + lane] = va;
+                        rec[(size_t)r2 * GM_REC + lane] = vb;
+                        if (at < SUB) {
+                            geo[gb][at][lane] = va;
+                            geo[gb][at + 1][lane] = vb;
+                        }
+                    }
+                    if (lane < 2) {
+                        const int r = lane ? r2 : ri;
+                        glist[at + lane] = r;
+                        if (at < SUB) list[gb][at + lane] = r;
+                    }
+                };
+                double vp = 0;
+                int rp = -1, rp2 = 0;   // the popped region not cut yet: its record is on its way
+                H.fetch_last(nheap, last);
+                do {
+                    if (nregions + 1 > R) {   // pool exhausted
+                        dn = 2;
+                        break;
+                    }
+                    double rk;
+                    const int ri = __builtin_amdgcn_readfirstlane(H.pop(lane, anc, nheap, &rk, last));
+                    if (rp >= 0) cut(vp, rp, rp2, nb - 2);
+                    // the region's record: just evaluated, prefetched, or from the pool
+                    const unsigned long long hit = __ballot(lane < lastn && list[bl][lane & (SUB - 1)] == ri);
+                    if (hit) vp = geo[bl][__builtin_ctzll(hit)][lane & (GM_REC - 1)];
+                    else if (ri == preidx) vp = pre;
+                    else vp = rec[(size_t)ri * GM_REC + (lane & (GM_REC - 1))];
+                    rp = ri;
+                    rp2 = nregions++;
+                    te_sum -= rk;
+                    eee -= rk;
+                    nb += 2;
+                    numEval += GM_NPTS * 2;
+                    if (gm_converged_quick(eev, eee, P)) break;
+                } while (nheap > 0 && (numEval < P.maxEval || !P.maxEval));
+                if (rp >= 0) cut(vp, rp, rp2, nb - 2);
+                preidx = -1;
+                if (nheap > 0) {
+                    preidx = __builtin_amdgcn_readfirstlane(H.idx(0));
+                    pre = rec[(size_t)preidx * GM_REC + (lane & (GM_REC - 1))];
+                }
+                // a long batch: another wave reads the records from the pool
+                if (nb > SUB) __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            }
+            if (lane == 0) {
+                sh_nR = nb;
+                sh_done = dn;
+                sh_nheap = nheap;
             }
         }
+        // the totals over the heap in its order, CH entries at a time
+        __syncthreads();
+        if (status == 2) {
+            if (tid == 0) jobfail[jb] = 1;
+            __syncthreads();
+            continue;
+        }
+        const int nh = sh_nheap;
+        double* buf = &vals[0][0];
+        double acc = 0;
+        for (int b0 = 0; b0 < nh; b0 += CH) {
+            const int nc = min(CH, nh - b0);
+            for (int i = tid; i < nc; i += NT) {
+                buf[i] = rec[(size_t)H.idx(b0 + i) * GM_REC + GM_REC_VAL];
+                buf[CH + i] = H.key(b0 + i);
+            }
+            __syncthreads();
+            if (tid < 2) {   // thread 0: the values, thread 1: the errors
+                const double* x = buf + tid * CH;
+                int i = 0;
+                for (; i + 16 <= nc; i += 16)
+#pragma unroll
+                    for (int e = 0; e < 16; e++) acc += x[i + e];
+                for (; i < nc; i++) acc += x[i];
+            }
+            __syncthreads();
+        }
+        if (tid == 0) {
+            Q[(size_t)f * qstride + key] = acc;
+            jobfail[jb] = 0;
+            atomicAdd(nevals, (unsigned long long)numEval);
+        }
+        if (tid == 1 && Qerr) Qerr[(size_t)f * qstride + key] = acc;
         __syncthreads();
     }
+}
+
+// Few deep integrals get a workgroup of eight waves each, many one wave each (the
+// 65 536-cell shell's prior, 4 x 10^3 capped integrals among 1.3 x 10^8: 2.4 s, 4.7 s
+// before).
+static void launch_gm(opsec_ctx* ctx, hipStream_t s, int slots, const XiModelDev& mv, const GMJobs& jobs, const int* idx,
+                      int n, int* counter, double* dpool, int* ipool, const GMParams& P, double* dQ, size_t nkeys,
+                      double* dQerr, int* fail, unsigned long long* nev) {
+    const dim3 g((unsigned)slots);
+    if (n <= 2 * ctx->num_cus)
+        hipLaunchKernelGGL((gm_kernel<512, 8191, 16>), g, dim3(512), 0, s, mv, jobs, idx, n, counter, dpool, ipool, P, dQ,
+                           nkeys, dQerr, fail, nev);
+    else if (n <= 4 * ctx->num_cus)
+        hipLaunchKernelGGL((gm_kernel<256, 2047, 16>), g, dim3(256), 0, s, mv, jobs, idx, n, counter, dpool, ipool, P, dQ,
+                           nkeys, dQerr, fail, nev);
+    else
+        hipLaunchKernelGGL((gm_kernel<64, 1023, 8>), g, dim3(64), 0, s, mv, jobs, idx, n, counter, dpool, ipool, P, dQ,
+                           nkeys, dQerr, fail, nev);
 }
 
 // The rerun's jobs: job j (template j % npairs, function funcs[j / npairs]) of
@@ -858,7 +1222,7 @@ __global__ __launch_bounds__(256) void gm_thread_kernel(XiModelDev m, GMJobs job
         S.heap = ireg + GM_TR;
         S.list = ireg + 2 * GM_TR;
         const int R = GM_TR;
-        const HeapStore H{S.hkey, S.heap, nullptr, nullptr, 0};
+        const HeapStore H{S.hkey, S.heap};
         for (int d = 0; d < 6; d++) {
             S.c[d * R] = 0.5;
             S.hw[d * R] = 0.5;
@@ -1168,6 +1532,11 @@ struct GMScratch {
     Scratch sj, sd, si, sc, sf, sp, st, sx, sa, se;
 };
 static std::mutex g_gm_stats_mutex;
+// Integrals per CU that still split after their first region, up to which they go
+// straight to gm_kernel; more go through gm_thread_kernel first, whose one launch
+// lasts as long as 16 regions of 149 nodes in one thread (2.7 ms on a box, 13 ms on
+// a shell) however few there are.
+constexpr int GM_WAVE_PENDING = 16;
 // Shell tables: the deep sweep beside the shallow one on a second stream (1, the
 // default) or after it (0).
 static int g_gm_overlap = 1;
@@ -1242,7 +1611,7 @@ static int run_gm_device(opsec_ctx* ctx, int nf, const int* funcs, const GMJob* 
             // as many wavefronts as half the free device memory holds pools for
             size_t fre = 0, tot = 0;
             if (hipMemGetInfo(&fre, &tot) != hipSuccess) fre = (size_t)16 << 30;
-            const size_t per_slot = (size_t)P.rmax * (15 * 8 + 3 * 4);
+            const size_t per_slot = (size_t)P.rmax * (GM_SLOT_DOUBLES * 8 + GM_SLOT_INTS * 4);
             const size_t budget = std::max<size_t>((size_t)1 << 30, fre / 2);
             nslots = std::min(njobs, ctx->num_cus * 8);
             nslots = (int)std::max<size_t>(1, std::min<size_t>(nslots, budget / per_slot));
@@ -1251,8 +1620,8 @@ static int run_gm_device(opsec_ctx* ctx, int nf, const int* funcs, const GMJob* 
         }
         int rc;
         if (pass == 1 && (rc = dev_realloc(ctx, &sj.p, &sj.cap, sizeof(GMJob) * njobs))) return rc;
-        if ((rc = dev_realloc(ctx, &sd.p, &sd.cap, sizeof(double) * 15 * (size_t)P.rmax * nslots))) return rc;
-        if ((rc = dev_realloc(ctx, &si.p, &si.cap, sizeof(int) * 3 * (size_t)P.rmax * nslots))) return rc;
+        if ((rc = dev_realloc(ctx, &sd.p, &sd.cap, sizeof(double) * GM_SLOT_DOUBLES * (size_t)P.rmax * nslots))) return rc;
+        if ((rc = dev_realloc(ctx, &si.p, &si.cap, sizeof(int) * GM_SLOT_INTS * (size_t)P.rmax * nslots))) return rc;
         if ((rc = dev_realloc(ctx, &sc.p, &sc.cap, 64))) return rc;
         if ((rc = dev_realloc(ctx, &sf.p, &sf.cap, sizeof(int) * njobs))) return rc;
         if ((rc = dev_realloc(ctx, &sp.p, &sp.cap, sizeof(int) * njobs))) return rc;
@@ -1266,6 +1635,7 @@ static int run_gm_device(opsec_ctx* ctx, int nf, const int* funcs, const GMJob* 
         const int* d_idx = nullptr;
         int nrun = njobs;
         GMJobs jobs{(const GMJob*)sj.p, nullptr, 0};   // the rerun's gathered jobs
+        int* d_failed_list = (int*)sp.p;               // not the list the jobs are read from
         if (pass == 0) {
             if ((rc = dev_realloc(ctx, &st.p, &st.cap, sizeof(int) * nf))) return rc;
             int* dfun = (int*)st.p;
@@ -1287,8 +1657,12 @@ static int run_gm_device(opsec_ctx* ctx, int nf, const int* funcs, const GMJob* 
                 int npend = 0;
                 OPSEC_HIP_TRY(ctx, hipMemcpyAsync(&npend, d_npend, 4, hipMemcpyDeviceToHost, stm));
                 OPSEC_HIP_TRY(ctx, hipStreamSynchronize(stm));
-                nrun = 0;
-                if (npend > 0) {
+                nrun = npend;
+                d_idx = (const int*)sx.p;
+                if (npend > GM_WAVE_PENDING * ctx->num_cus) {
+                    nrun = 0;
+                    d_idx = (const int*)sp.p;
+                    d_failed_list = (int*)sx.p;
                     hipLaunchKernelGGL(gm_thread_kernel, dim3((unsigned)((npend + 255) / 256)), dim3(256), 0,
                                        stm, mv, jobs, (const int*)sx.p, npend, P, dQ, nkeys,
                                        dQerr, (int*)sf.p, (int*)sp.p, d_ndeep, d_nev);
@@ -1296,35 +1670,20 @@ static int run_gm_device(opsec_ctx* ctx, int nf, const int* funcs, const GMJob* 
                     OPSEC_HIP_TRY(ctx, hipMemcpyAsync(&nrun, d_ndeep, 4, hipMemcpyDeviceToHost, stm));
                     OPSEC_HIP_TRY(ctx, hipStreamSynchronize(stm));
                 }
-                d_idx = (const int*)sp.p;
             }
         } else {
             OPSEC_HIP_TRY(ctx, hipMemcpyAsync(sj.p, sa.p, sizeof(GMJob) * njobs, hipMemcpyDeviceToDevice, stm));
         }
         if (nrun > 0) {
-            if (pass == 0)
-                hipLaunchKernelGGL((gm_kernel<64, 0>), dim3(std::min(nslots, nrun)), dim3(64), 0, stm, mv,
-                                   jobs, d_idx, nrun, d_counter, (double*)sd.p, (int*)si.p, P, dQ,
-                                   nkeys, dQerr, (int*)sf.p, d_nev);
-            else if (nrun <= 2 * ctx->num_cus)   // few deep integrals: 8 waves each
-                hipLaunchKernelGGL((gm_kernel<512, 8192>), dim3(std::min(nslots, nrun)), dim3(512), 0, stm, mv,
-                                   jobs, d_idx, nrun, d_counter, (double*)sd.p, (int*)si.p, P, dQ,
-                                   nkeys, dQerr, (int*)sf.p, d_nev);
-            else if (nrun <= 4 * ctx->num_cus)
-                hipLaunchKernelGGL((gm_kernel<256, 1024>), dim3(std::min(nslots, nrun)), dim3(256), 0, stm, mv,
-                                   jobs, d_idx, nrun, d_counter, (double*)sd.p, (int*)si.p, P, dQ,
-                                   nkeys, dQerr, (int*)sf.p, d_nev);
-            else   // many: one wave each
-                hipLaunchKernelGGL((gm_kernel<64, 0>), dim3(std::min(nslots, nrun)), dim3(64), 0, stm, mv,
-                                   jobs, d_idx, nrun, d_counter, (double*)sd.p, (int*)si.p, P, dQ,
-                                   nkeys, dQerr, (int*)sf.p, d_nev);
+            launch_gm(ctx, stm, std::min(nslots, nrun), mv, jobs, d_idx, nrun, d_counter, (double*)sd.p, (int*)si.p, P,
+                      dQ, nkeys, dQerr, (int*)sf.p, d_nev);
             OPSEC_HIP_TRY(ctx, hipGetLastError());
         }
         // jobs whose region pool ran out, listed on the device
         int nfail = 0;
         if (nrun > 0) {
             hipLaunchKernelGGL(list_failed_kernel, dim3((unsigned)((nrun + 255) / 256)), dim3(256), 0, stm,
-                               (const int*)sf.p, d_idx, nrun, (int*)sx.p, d_nfail);
+                               (const int*)sf.p, d_idx, nrun, d_failed_list, d_nfail);
             OPSEC_HIP_TRY(ctx, hipGetLastError());
         }
         unsigned long long nev = 0;
@@ -1336,7 +1695,7 @@ static int run_gm_device(opsec_ctx* ctx, int nf, const int* funcs, const GMJob* 
             return set_error(ctx, OPSEC_ECONV, "adaptive cubature exceeded %d regions", P.rmax);
         std::vector<int> failed(nfail);
         if (nfail > 0) {
-            OPSEC_HIP_TRY(ctx, hipMemcpyAsync(failed.data(), sx.p, sizeof(int) * nfail, hipMemcpyDeviceToHost,
+            OPSEC_HIP_TRY(ctx, hipMemcpyAsync(failed.data(), d_failed_list, sizeof(int) * nfail, hipMemcpyDeviceToHost,
                                               stm));
             OPSEC_HIP_TRY(ctx, hipStreamSynchronize(stm));
         }

@@ -214,3 +214,49 @@ def test_spherical_sig_block_vs_oracle(ctx):
                                      O.ptr(cols), len(cols), O.ptr(ref), lld, q.epsrel, q.epsabs, q.maxeval) == 0
         np.testing.assert_allclose(got[:, :len(cols)], ref[:, :len(cols)], rtol=1e-12,
                                    atol=1e-13 * np.abs(ref).max(), err_msg=kind)
+
+
+# pending counts that take each kernel of the adaptive driver: eight waves per integral (124 keys),
+# four (728), one (1330), and the one-thread pass before it (4912)
+@pytest.mark.parametrize("n", [5, 9, 11, 17])
+def test_gm_integral_independent_of_its_kernel(ctx, n):
+    """An adaptive integral has the same bits whichever kernel finishes it: the pair tables of
+    n^3 keys (a tolerance under which nearly all of them split) against single integrals, which
+    run on eight waves, and against the oracle for the self pair."""
+    w = 25.0
+    cells = synth.box_cells(n, 0.0, w * n)
+    sv = lib.survey_box(n, 0.0, w * n, L=1e9)
+    lo, hi = synth.linear_bands(1, 0.05, 0.25)
+    ctx.model_real(GOLD["pk_k"], GOLD["pk_P"], lo, hi, lib.OPSEC_XI_TABLE)
+    ctx.cells_upload(cells, sv)
+    q = ctx.quad(lib.OPSEC_QUAD_GM, epsrel=1e-11, epsabs=1e-11, maxeval=20000)
+    ctx.pair_tables([1], q)
+    nodes = ctx.pair_stats()["nodes"]
+    T = ctx.pair_table(1)
+    print(f"{n}^3 keys: {nodes / 149 / n ** 3:.1f} regions per integral", flush=True)
+    assert nodes > 2 * 149 * n ** 3
+    rng = np.random.default_rng(n)
+    for key in [0, 1, n * n * n - 1] + list(rng.choice(n ** 3, 9, replace=False)):
+        got, _ = ctx.pair_integral(cells[0], cells[key], 1, sv, q)
+        assert got == T[key], (key, got, T[key])
+
+
+def test_gm_deep_heap_levels(ctx):
+    """A self pair whose heap outgrows the positions kept on chip (more than 8191 regions) and
+    whose batches hold many chunks of regions, with a region pool of its own: the driver's value
+    and error estimate against the oracle's serial driver, to rounding."""
+    cells = synth.box_cells(4, 0.0, 400.0 / 3)
+    sv = lib.survey_box(4, 0.0, 400.0 / 3, L=1e9)
+    lo, hi = synth.linear_bands(1, 0.02, 0.1)
+    ctx.model_real(GOLD["pk_k"], GOLD["pk_P"], lo, hi, lib.OPSEC_XI_TABLE)
+    q = ctx.quad(lib.OPSEC_QUAD_GM, maxeval=4000000)
+    got, err = ctx.pair_integral(cells[0], cells[0], 0, sv, q)
+    r768, tabs = O.oracle_tables(GOLD["pk_k"], GOLD["pk_P"], lo, hi)
+    xi = O.XiHandle(0, r768, tabs[0])
+    S = np.zeros((1, 1))
+    r = np.array([0], np.int32)
+    O.oracle().orc_sig_block(C.byref(xi.s), cells.ctypes.data, len(cells), 4, 4, 4, 1e9, O.ptr(r), 1, O.ptr(r), 1,
+                             O.ptr(S), 1, 0, q.epsrel, q.epsabs, q.maxeval, 0, 0)
+    ref = S[0, 0] / cells["Nbar"][0]
+    print("deep self pair", got, "error estimate", err, flush=True)
+    assert abs(got - ref) <= 1e-12 * abs(ref)
