@@ -762,7 +762,7 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void gm
                     push(0, nt);
                 }
                 // the next chunk's regions from the pool, sixteen lanes per record
-                if ((SOLO || wave == (NT > 256 ? 4 : 1)) && c + 1 < nch) {
+                if ((SOLO || wave == 4) && c + 1 < nch) {
                     const int n1 = min(SUB, n - (c + 1) * SUB), e = lane & 15;
                     int ri[SUB / 4 + 1];
                     double v[SUB / 4 + 1];
@@ -897,18 +897,17 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(2))) void gm
     }
 }
 
-// Few deep integrals get a workgroup of eight waves each, many one wave each (the
-// 65 536-cell shell's prior, 4 x 10^3 capped integrals among 1.3 x 10^8: 2.4 s, 4.7 s
-// before).
+// Up to eight deep integrals per CU get a workgroup of eight waves each (one resident
+// per CU by its LDS), more one wave each.  Priors of shells, tables in ms: 8x8x8 129,
+// 16x16x16 199, 32x16x16 336; with the line at two per CU and four waves up to four
+// per CU 133, 198, 466; 64x32x32 (one wave each) 2.35 s, 2.45 s with eight (the
+// one-lane driver: 525, 635, 1083 ms and 4.7 s).
 static void launch_gm(opsec_ctx* ctx, hipStream_t s, int slots, const XiModelDev& mv, const GMJobs& jobs, const int* idx,
                       int n, int* counter, double* dpool, int* ipool, const GMParams& P, double* dQ, size_t nkeys,
                       double* dQerr, int* fail, unsigned long long* nev) {
     const dim3 g((unsigned)slots);
-    if (n <= 2 * ctx->num_cus)
+    if (n <= 8 * ctx->num_cus)
         hipLaunchKernelGGL((gm_kernel<512, 8191, 16>), g, dim3(512), 0, s, mv, jobs, idx, n, counter, dpool, ipool, P, dQ,
-                           nkeys, dQerr, fail, nev);
-    else if (n <= 4 * ctx->num_cus)
-        hipLaunchKernelGGL((gm_kernel<256, 2047, 16>), g, dim3(256), 0, s, mv, jobs, idx, n, counter, dpool, ipool, P, dQ,
                            nkeys, dQerr, fail, nev);
     else
         hipLaunchKernelGGL((gm_kernel<64, 1023, 8>), g, dim3(64), 0, s, mv, jobs, idx, n, counter, dpool, ipool, P, dQ,
@@ -1537,6 +1536,10 @@ static std::mutex g_gm_stats_mutex;
 // lasts as long as 16 regions of 149 nodes in one thread (2.7 ms on a box, 13 ms on
 // a shell) however few there are.
 constexpr int GM_WAVE_PENDING = 16;
+// Regions of pass 0's pools: their heap then sits in LDS whole (gm_kernel's NL), and
+// the integrals that need more soon get a workgroup of their own instead of holding
+// one wave for 4096 regions (8x8x8 shell's prior: pass 0 28 ms with 4096, 6.8 with 1024).
+constexpr int GM_POOL = 1024;
 // Shell tables: the deep sweep beside the shallow one on a second stream (1, the
 // default) or after it (0).
 static int g_gm_overlap = 1;
@@ -1571,9 +1574,10 @@ static int run_gm_device(opsec_ctx* ctx, int nf, const int* funcs, const GMJob* 
     P.coordsys = ctx->sv.coordsys;
     P.L = ctx->sv.L;
     // Pass 0: every job's first region (one thread per job), then the jobs
-    // that need splits with a 4096-region pool per wavefront slot.  Pass 1:
-    // jobs that exhausted it, with pools that hold every region the
-    // evaluation cap allows (maxeval / 149 + 2), on fewer slots.
+    // that need splits with a GM_POOL-region pool per workgroup, or, when there is
+    // at most one per CU, with pools that hold every region the evaluation cap
+    // allows (maxeval / 149 + 2).  Pass 1: jobs that exhausted their pool, with
+    // whole-cap pools.
     const size_t njobs_all = npairs * (size_t)nf;
     if (njobs_all > (size_t)INT32_MAX) return set_error(ctx, OPSEC_EINVAL, "too many pair integrals in one call");
     // A shell's sweep of closed-form bands takes its first regions from
@@ -1604,24 +1608,8 @@ static int run_gm_device(opsec_ctx* ctx, int nf, const int* funcs, const GMJob* 
     for (int pass = 0; pass < 2; pass++) {
         const int njobs = pass == 0 ? (int)njobs_all : nagain;
         if (njobs == 0) break;
-        long long cap_regions = P.maxEval ? (long long)P.maxEval / GM_NPTS + 2 : (1LL << 20);
-        P.rmax = pass == 0 ? 4096 : (int)std::min<long long>(cap_regions, 1LL << 22);
-        int nslots = pass == 0 ? std::min(njobs, ctx->num_cus * 8) : std::min(njobs, 64);
-        if (pass == 1) {
-            // as many wavefronts as half the free device memory holds pools for
-            size_t fre = 0, tot = 0;
-            if (hipMemGetInfo(&fre, &tot) != hipSuccess) fre = (size_t)16 << 30;
-            const size_t per_slot = (size_t)P.rmax * (GM_SLOT_DOUBLES * 8 + GM_SLOT_INTS * 4);
-            const size_t budget = std::max<size_t>((size_t)1 << 30, fre / 2);
-            nslots = std::min(njobs, ctx->num_cus * 8);
-            nslots = (int)std::max<size_t>(1, std::min<size_t>(nslots, budget / per_slot));
-            const int cap = g_gm_deep_slots > 0 ? g_gm_deep_slots : deep_cap;
-            if (cap > 0) nslots = std::min(nslots, cap);
-        }
         int rc;
         if (pass == 1 && (rc = dev_realloc(ctx, &sj.p, &sj.cap, sizeof(GMJob) * njobs))) return rc;
-        if ((rc = dev_realloc(ctx, &sd.p, &sd.cap, sizeof(double) * GM_SLOT_DOUBLES * (size_t)P.rmax * nslots))) return rc;
-        if ((rc = dev_realloc(ctx, &si.p, &si.cap, sizeof(int) * GM_SLOT_INTS * (size_t)P.rmax * nslots))) return rc;
         if ((rc = dev_realloc(ctx, &sc.p, &sc.cap, 64))) return rc;
         if ((rc = dev_realloc(ctx, &sf.p, &sf.cap, sizeof(int) * njobs))) return rc;
         if ((rc = dev_realloc(ctx, &sp.p, &sp.cap, sizeof(int) * njobs))) return rc;
@@ -1675,7 +1663,25 @@ static int run_gm_device(opsec_ctx* ctx, int nf, const int* funcs, const GMJob* 
             OPSEC_HIP_TRY(ctx, hipMemcpyAsync(sj.p, sa.p, sizeof(GMJob) * njobs, hipMemcpyDeviceToDevice, stm));
         }
         if (nrun > 0) {
-            launch_gm(ctx, stm, std::min(nslots, nrun), mv, jobs, d_idx, nrun, d_counter, (double*)sd.p, (int*)si.p, P,
+            const long long cap_regions = P.maxEval ? (long long)P.maxEval / GM_NPTS + 2 : (1LL << 20);
+            const bool deep = pass == 1 || nrun <= ctx->num_cus;
+            P.rmax = deep ? (int)std::min<long long>(cap_regions, 1LL << 22) : GM_POOL;
+            const size_t per_slot = (size_t)P.rmax * (GM_SLOT_DOUBLES * 8 + GM_SLOT_INTS * 4);
+            int nslots = std::min(nrun, ctx->num_cus * 8);
+            if (deep) {
+                // as many workgroups as half the free device memory (and what this sweep
+                // already holds) has pools for
+                size_t fre = 0, tot = 0;
+                if (hipMemGetInfo(&fre, &tot) != hipSuccess) fre = (size_t)16 << 30;
+                const size_t budget = std::max<size_t>(sd.cap + si.cap, std::max<size_t>((size_t)1 << 30, fre / 2));
+                nslots = (int)std::max<size_t>(1, std::min<size_t>(nslots, budget / per_slot));
+                const int cap = g_gm_deep_slots > 0 ? g_gm_deep_slots : deep_cap;
+                if (cap > 0) nslots = std::min(nslots, cap);
+            }
+            if ((rc = dev_realloc(ctx, &sd.p, &sd.cap, sizeof(double) * GM_SLOT_DOUBLES * (size_t)P.rmax * nslots)))
+                return rc;
+            if ((rc = dev_realloc(ctx, &si.p, &si.cap, sizeof(int) * GM_SLOT_INTS * (size_t)P.rmax * nslots))) return rc;
+            launch_gm(ctx, stm, nslots, mv, jobs, d_idx, nrun, d_counter, (double*)sd.p, (int*)si.p, P,
                       dQ, nkeys, dQerr, (int*)sf.p, d_nev);
             OPSEC_HIP_TRY(ctx, hipGetLastError());
         }
