@@ -101,14 +101,20 @@ __device__ __forceinline__ int64_t lower_bound_u32(const uint32_t* __restrict__ 
     return lo;
 }
 
-// counts[b] += w over bin b's galaxies, one by one in catalogue order.
+// counts[b] += w over bin b's galaxies, one by one in catalogue order.  Bins of
+// more than LONG_BIN galaxies are listed for fold_long_kernel instead.
+constexpr int LONG_BIN = 1024;
 __global__ void fold_bins_kernel(const uint32_t* __restrict__ key, const float* __restrict__ w, int64_t n,
-                                 int nbins, double* __restrict__ counts) {
+                                 int nbins, double* __restrict__ counts, int* __restrict__ longs) {
     int b = blockIdx.x * blockDim.x + threadIdx.x;
     if (b >= nbins) return;
     int64_t lo = lower_bound_u32(key, n, (uint32_t)b);
     int64_t hi = lower_bound_u32(key, n, (uint32_t)b + 1);
     if (lo == hi) return;
+    if (hi - lo > LONG_BIN) {
+        longs[1 + atomicAdd(longs, 1)] = b;
+        return;
+    }
     double s = counts[b];
     int64_t i = lo;
     for (; i + 8 <= hi; i += 8) {
@@ -120,6 +126,155 @@ __global__ void fold_bins_kernel(const uint32_t* __restrict__ key, const float* 
     }
     for (; i < hi; i++) s += (double)w[i];
     counts[b] = s;
+}
+
+// The same fold of a long bin (the galaxies outside the survey above all), one
+// workgroup per bin, with the bits of the serial loop.  While the sum stays
+// within one binade, s = k u with u = ulp(s) and k an integer in [2^52, 2^53),
+// adding w >= 0 rounds k + w/u to the nearest integer, ties to even: k grows by
+// an integer that depends on k only where w/u is a half-integer, and then only
+// on its parity.  So an addition is a map (parity -> increment), such maps
+// compose associatively, and a block of FOLD_BLOCK weights is composed by all
+// threads at once; the sums within it only grow, so if the last is below 2^53
+// all were.  Where that fails (the sum leaves the binade, a weight is negative or
+// not finite, the sum is not positive and normal), the waves before the failing
+// one are kept, that wave's weights are added one by one from LDS, and the next
+// block starts behind them.
+// Bound by the composition's latency per block: 5 x 10^5 galaxies of one bin take
+// 425 us, 9.8 ms by one thread (a dependent FP64 addition and its load each).
+constexpr int FOLD_THREADS = 512, FOLD_PER = 4, FOLD_BLOCK = FOLD_THREADS * FOLD_PER;
+constexpr int FOLD_WAVES = FOLD_THREADS / 64, FOLD_WAVE = 64 * FOLD_PER;
+struct FoldMap {
+    long long c0, c1;   // increment of an even, of an odd k
+    // this addition (or block) first, then b
+    __device__ __forceinline__ void then(const FoldMap& b) {
+        c0 += (c0 & 1) ? b.c1 : b.c0;
+        c1 += (c1 & 1) ? b.c0 : b.c1;   // an odd k moved by an odd step is even
+    }
+};
+// The map of the lane O further on in its row of 16 (zero past the row's end).
+template <int O>
+__device__ __forceinline__ FoldMap row_next(const FoldMap& f) {
+    auto mv = [](long long x) {
+        const unsigned lo = __builtin_amdgcn_mov_dpp((unsigned)x, 0x100 | O, 0xF, 0xF, true);
+        const unsigned hi = __builtin_amdgcn_mov_dpp((unsigned)((unsigned long long)x >> 32), 0x100 | O, 0xF, 0xF, true);
+        return (long long)((unsigned long long)hi << 32 | lo);
+    };
+    return FoldMap{mv(f.c0), mv(f.c1)};
+}
+__global__ __launch_bounds__(FOLD_THREADS) void fold_long_kernel(const uint32_t* __restrict__ key,
+                                                                 const float* __restrict__ w, int64_t n,
+                                                                 double* __restrict__ counts,
+                                                                 const int* __restrict__ longs) {
+    __shared__ FoldMap part[2][FOLD_WAVES * 4];   // one per row of 16 lanes
+    __shared__ int bad[2][FOLD_WAVES];
+    __shared__ float buf[FOLD_WAVE];
+    __shared__ double sh_s;
+    if ((int)blockIdx.x >= longs[0]) return;
+    const int b = longs[1 + blockIdx.x], t = threadIdx.x, lane = t & 63, wave = t >> 6;
+    const int64_t lo = lower_bound_u32(key, n, (uint32_t)b), hi = lower_bound_u32(key, n, (uint32_t)b + 1);
+    double s = counts[b];
+    float nx[FOLD_PER];
+    auto load = [&](int64_t at) {
+#pragma unroll
+        for (int j = 0; j < FOLD_PER; j++) {
+            const int64_t i = at + FOLD_PER * t + j;
+            nx[j] = i < hi ? w[i] : 0.0f;   // adding 0 to a positive sum changes nothing
+        }
+    };
+    load(lo);
+    int ph = 0;
+    for (int64_t at = lo; at < hi; ph ^= 1) {
+        float v[FOLD_PER];
+#pragma unroll
+        for (int j = 0; j < FOLD_PER; j++) v[j] = nx[j];
+        if (at + FOLD_BLOCK < hi) load(at + FOLD_BLOCK);
+        const unsigned long long bits = __double_as_longlong(s);
+        const int e = (int)(bits >> 52) - 1023;          // s in [2^e, 2^(e+1)) when it is positive and normal
+        const bool normal = e > -800 && e < 800;         // (a negative sum has the sign in e: above 800)
+        const long long k = (long long)((bits & 0xfffffffffffffull) | 0x10000000000000ull);
+        FoldMap f{0, 0};
+        bool ok = normal;
+#pragma unroll
+        for (int j = 0; j < FOLD_PER; j++) {
+            const double q = ldexp((double)v[j], 52 - e);   // w / u, exact
+            ok = ok && q >= 0.0 && q < 9007199254740992.0;
+            const double r = rint(q), d = q - r;
+            FoldMap g;
+            g.c0 = g.c1 = (long long)(ok ? r : 0.0);
+            if (fabs(d) == 0.5) {   // tie: to the even neighbour of k + w/u
+                const long long l = (long long)(ok ? q - 0.5 : 0.0);
+                g.c0 = l + (l & 1);
+                g.c1 = l + (~l & 1);
+            }
+            f.then(g);
+        }
+        f.then(row_next<1>(f));
+        f.then(row_next<2>(f));
+        f.then(row_next<4>(f));
+        f.then(row_next<8>(f));
+        const bool wave_bad = __ballot(!ok) != 0;
+        if ((lane & 15) == 0) part[ph][wave * 4 + (lane >> 4)] = f;
+        if (lane == 0) bad[ph][wave] = wave_bad;
+        __syncthreads();
+        // the whole block: its 32 rows, one per lane, composed like the lanes were
+        {
+            FoldMap F = lane < 4 * FOLD_WAVES ? part[ph][lane] : FoldMap{0, 0};
+            const bool any = __ballot(lane < FOLD_WAVES && bad[ph][lane & (FOLD_WAVES - 1)]) != 0;
+            F.then(row_next<1>(F));
+            F.then(row_next<2>(F));
+            F.then(row_next<4>(F));
+            F.then(row_next<8>(F));
+            long long kw = k;
+#pragma unroll
+            for (int i = 0; i < 4 * FOLD_WAVES; i += 16) {
+                const long long c0 = __shfl(F.c0, i), c1 = __shfl(F.c1, i);
+                kw += (kw & 1) ? c1 : c0;
+            }
+            if (!any && kw < 9007199254740992ll) {
+                s = ldexp((double)kw, e - 52);
+                at += FOLD_BLOCK;
+                continue;
+            }
+        }
+        // the sum after each wave's weights, up to the first wave that fails
+        long long k1 = k;
+        int good = 0;
+        for (; good < FOLD_WAVES - 1; good++) {   // the last one if no earlier
+            long long kw = k1;
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const FoldMap& F = part[ph][good * 4 + i];
+                kw += (kw & 1) ? F.c1 : F.c0;
+            }
+            if (bad[ph][good] || kw >= 9007199254740992ll) break;
+            k1 = kw;
+        }
+        if (good > 0) s = ldexp((double)k1, e - 52);
+        if (wave == good)
+#pragma unroll
+            for (int j = 0; j < FOLD_PER; j++) buf[FOLD_PER * lane + j] = v[j];
+        __syncthreads();
+        at += good * FOLD_WAVE;
+        if (t == 0 && at < hi) {
+            const int m = (int)(hi - at < FOLD_WAVE ? hi - at : FOLD_WAVE);
+            int i = 0;
+            for (; i + 16 <= m; i += 16) {
+                float x[16];
+#pragma unroll
+                for (int j = 0; j < 16; j++) x[j] = buf[i + j];
+#pragma unroll
+                for (int j = 0; j < 16; j++) s += (double)x[j];
+            }
+            for (; i < m; i++) s += (double)buf[i];
+        }
+        at += FOLD_WAVE;
+        load(at);
+        if (t == 0) sh_s = s;
+        __syncthreads();
+        s = sh_s;
+    }
+    if (t == 0) counts[b] = s;
 }
 
 // x_a = (N_a - Nbar_a)/sqrt(Nbar_a)  (src/dot.cpp:130-134)
@@ -240,8 +395,16 @@ int opsec_count_galaxies(opsec_ctx* ctx, const opsec_galaxy* gals, int64_t ngals
         size_t tmp = d->cap_tmp;
         OPSEC_HIP_TRY(ctx, rocprim::radix_sort_pairs(d->d_tmp, tmp, d->d_key[0], d->d_key[1], d->d_w[0], d->d_w[1],
                                                      (size_t)n, 0u, end_bit, ctx->stream));
+        // at most n / LONG_BIN bins are long: their number, then their list, in the sort's
+        // first key buffer (free again)
+        int* longs = (int*)d->d_key[0];
+        const int nlong = (int)std::min<int64_t>(nbins, n / (LONG_BIN + 1));
+        hipLaunchKernelGGL(fill_int_kernel, dim3(1), dim3(64), 0, ctx->stream, longs, 1, 0);
         hipLaunchKernelGGL(fold_bins_kernel, dim3(blocks_for(nbins, 256)), dim3(256), 0, ctx->stream, d->d_key[1],
-                           d->d_w[1], n, nbins, d->d_counts);
+                           d->d_w[1], n, nbins, d->d_counts, longs);
+        if (nlong > 0)
+            hipLaunchKernelGGL(fold_long_kernel, dim3(nlong), dim3(FOLD_THREADS), 0, ctx->stream, d->d_key[1], d->d_w[1],
+                               n, d->d_counts, longs);
         OPSEC_HIP_TRY(ctx, hipGetLastError());
     }
     OPSEC_HIP_TRY(ctx, hipMemcpyAsync(counts, d->d_counts, (size_t)nbins * 8, hipMemcpyDeviceToHost, ctx->stream));

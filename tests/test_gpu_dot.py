@@ -83,6 +83,46 @@ def test_counts_spherical(ctx):
     assert ref[-1] > 0
 
 
+# a bin of one galaxy more than the short path takes, ragged and whole blocks of the long one, and many
+@pytest.mark.parametrize("ngal", [1024, 1025, 2048, 5003, 300001])
+@pytest.mark.parametrize("kind", ["wide", "unit", "ties", "negative", "special"])
+def test_counts_long_bins_bit_exact(ctx, ngal, kind):
+    """Long bins (every galaxy in one cell, or outside) have the bits of the one-by-one sum in
+    catalogue order: weights over six decades, ones, half-ulp ties of the running sum (from a
+    large starting count), mixed signs, and zeros, subnormals and infinities."""
+    cells = synth.box_cells(2, 0.0, 2.0)
+    sv = lib.survey_box(2, 0.0, 2.0)
+    ctx.cells_upload(cells, sv)
+    rng = np.random.default_rng(ngal)
+    g = np.zeros(ngal, dtype=lib.GALAXY_DTYPE)
+    g["x1"] = np.where(rng.random(ngal) < 0.3, 5.0, 0.5)   # 30 % outside, the rest in cell 0
+    g["x2"], g["x3"] = 0.5, 0.5
+    start = np.zeros(9)
+    if kind == "wide":
+        w = 10.0 ** rng.uniform(-3, 3, ngal)
+    elif kind == "unit":
+        w = np.ones(ngal)
+    elif kind == "ties":
+        start[:] = 2.0 ** 53 - 2.0 * rng.integers(1, 400, 9)   # ulp 1 below 2^53, 2 above
+        w = rng.integers(0, 5, ngal) * 0.5
+    elif kind == "negative":
+        w = rng.normal(size=ngal)
+    else:
+        w = np.where(rng.random(ngal) < 0.5, 1e-41, 0.0)
+        w[ngal // 2:] = np.where(rng.random(ngal - ngal // 2) < 0.001, 3e38, 1.5)
+        w[-1] = np.inf
+    g["w"] = w
+    got = ctx.count_galaxies(g, counts=start.copy())
+    # the oracle's loop, one by one
+    ref = start.copy()
+    for b, sel in ((0, g["x1"] == 0.5), (8, g["x1"] == 5.0)):
+        acc = ref[b]
+        for v in g["w"][sel].astype(np.float64):
+            acc += v
+        ref[b] = acc
+    assert np.array_equal(_bits(got), _bits(ref)), (got[[0, 8]], ref[[0, 8]])
+
+
 @pytest.mark.parametrize("n,M,ngal", [(6, 40, 30000), (32, 2000, 2000000)])
 def test_pixel_values_vs_oracle(ctx, n, M, ngal):
     """x bit-exact (IEEE subtract, sqrt and divide); y = B^T x within 1e-13 of
