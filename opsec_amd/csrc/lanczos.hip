@@ -77,29 +77,33 @@ __global__ __launch_bounds__(GT_THREADS) void lgemm_kernel(SrcA A, SrcB B, Out O
     for (int i = 0; i < 4; i++)
         for (int j = 0; j < 4; j++) acc[i][j] = d4_t{0, 0, 0, 0};
     const int t = threadIdx.x;
+    // the next step's operand elements are loaded under the current step's MFMAs
+    double ra[8], rb[8];
+    const int ia = SrcA::k_contig ? t >> 1 : (t & 15) * 8, ka = SrcA::k_contig ? (t & 1) * 8 : t >> 4;
+    const int ib = t >> 1, kb = (t & 1) * 8;
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const int m = m0 + ia + (SrcA::k_contig ? 0 : e), ke = k0 + ka + (SrcA::k_contig ? e : 0);
+            ra[e] = (m < M && ke < kz1) ? A.get(m, ke) : 0.0;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            const int n = n0 + ib, k = k0 + kb + e;
+            rb[e] = (n < N && k < kz1) ? B.get(n, k) : 0.0;
+        }
+    };
+    if (kz0 < kz1) fetch(kz0);
     for (int k0 = kz0; k0 < kz1; k0 += 16) {
         __syncthreads();
-        if (SrcA::k_contig) {
-            int i = t >> 1, kb = (t & 1) * 8;
-            for (int e = 0; e < 8; e++) {
-                int m = m0 + i, k = k0 + kb + e;
-                As[kb + e][i] = (m < M && k < kz1) ? A.get(m, k) : 0.0;
-            }
-        } else {
-            int k = t >> 4, ib = (t & 15) * 8;
-            for (int e = 0; e < 8; e++) {
-                int m = m0 + ib + e, kk = k0 + k;
-                As[k][ib + e] = (m < M && kk < kz1) ? A.get(m, kk) : 0.0;
-            }
-        }
-        {
-            int i = t >> 1, kb = (t & 1) * 8;
-            for (int e = 0; e < 8; e++) {
-                int n = n0 + i, k = k0 + kb + e;
-                Bs[kb + e][i] = (n < N && k < kz1) ? B.get(n, k) : 0.0;
-            }
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            if (SrcA::k_contig) As[ka + e][ia] = ra[e];
+            else As[ka][ia + e] = ra[e];
+            Bs[kb + e][ib] = rb[e];
         }
         __syncthreads();
+        if (k0 + 16 < kz1) fetch(k0 + 16);
         for (int kk = 0; kk < 4; kk++) {
             double af[4], bf[4];
             const int kr = kk * 4 + (lane >> 4);
@@ -179,7 +183,7 @@ struct Dev {
         // split-K fills the CUs when the output has few tiles; the partials
         // (splits x p x q <= 2 CUs x 128 x 128 doubles) are summed in order
         int splits = std::max(1, std::min(64, (2 * ctx->num_cus) / std::max(1, gx * gy)));
-        splits = std::min(splits, std::max(1, N / 512));
+        splits = std::min(splits, std::max(1, N / 128));
         hipLaunchKernelGGL((lgemm_kernel<LA_KCol, LA_KCol, LPut<0>>), dim3(gx, gy, splits), dim3(GT_THREADS), 0, s, A,
                            B, LPut<0>{H, (size_t)p}, p, q, N, parts);
         if (splits > 1)
@@ -238,145 +242,205 @@ struct Dev {
 
 // ---- Householder tridiagonalisation of a dense symmetric K x K (col-major) --
 
-// One workgroup: Householder vector of column k (rows k+1..K-1), in place.
-__global__ __launch_bounds__(1024) void hh_vector_kernel(double* A, int K, int k, double* tau, double* e) {
-    __shared__ double red[1024];
-    __shared__ double sh_scale, sh_tau, sh_beta;
-    const int m = K - k - 1;
-    double* x = A + (size_t)k * K + (k + 1);
-    double s = 0;
-    for (int i = 1 + threadIdx.x; i < m; i += blockDim.x) s += x[i] * x[i];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+constexpr int TR_NB = 32;   // columns per panel
+
+// Three launches per column k (panel column i; it was eight, each a few us whatever
+// its size).  The scalars between them (the column's norm, p . v) are left as one
+// partial per workgroup, which every workgroup of the next launch adds in order.
+// Within a panel the rank-2 updates of its reflectors are kept as the columns of V
+// (reflectors) and W (update vectors), K x nb column-major, meaningful from each
+// column's first row; the trailing matrix is updated once per panel.
+//   hh_col   w of column k - 1; column k with the deferred updates; its norm
+//   hh_symv  the reflector v of column k, A22 v in column chunks, W^T v and V^T v
+//   hh_comb  p = A22 v with the deferred updates' share; p . v
+// Bound by the launches and the latency of the scalars between them while A22 fits the
+// caches, by reading A22 beyond: a 1607 x 1607 reduction takes 24 ms (59 with eight
+// launches per column), the four reductions up to 9216 of a 32^3 box's 3000 modes 1.23 s
+// (2.04).
+
+constexpr int HH_T = 256;    // threads: four waves
+constexpr int HH_R = 64;     // rows per workgroup of hh_col and hh_comb: a wave's lanes, the
+                             // panel's columns shared out over the four waves
+
+// Sum over the wave, in every lane: rows of 16 by DPP, then their four sums.
+__device__ __forceinline__ double wave_total(double x) {
+    auto next = [](double v, auto ctrl) {
+        const unsigned long long u = __builtin_bit_cast(unsigned long long, v);
+        const unsigned lo = __builtin_amdgcn_mov_dpp((unsigned)u, decltype(ctrl)::value, 0xF, 0xF, true);
+        const unsigned hi = __builtin_amdgcn_mov_dpp((unsigned)(u >> 32), decltype(ctrl)::value, 0xF, 0xF, true);
+        return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+    };
+    x += next(x, std::integral_constant<int, 0x101>());   // row_shl: lane + 1, + 2, + 4, + 8 of the row
+    x += next(x, std::integral_constant<int, 0x102>());
+    x += next(x, std::integral_constant<int, 0x104>());
+    x += next(x, std::integral_constant<int, 0x108>());
+    auto row = [&](int l) {
+        const unsigned long long u = __builtin_bit_cast(unsigned long long, x);
+        const unsigned lo = __builtin_amdgcn_readlane((unsigned)u, l), hi = __builtin_amdgcn_readlane((unsigned)(u >> 32), l);
+        return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
+    };
+    return (row(0) + row(16)) + (row(32) + row(48));
+}
+// Sum of x[0..n) in a fixed order, each wave by itself.
+__device__ __forceinline__ double hh_total(const double* __restrict__ x, int n) {
+    double acc = 0.0;
+    for (int i = threadIdx.x & 63; i < n; i += 64) acc += x[i];
+    return wave_total(acc);
+}
+
+// w = tau p - (tau/2)(tau p . v) v of column k (panel column i), stored to W; p is
+// indexed from row k + 1, pv holds npv partials of p . v.
+__global__ __launch_bounds__(HH_T) void hh_w_kernel(int K, int k, int i, const double* __restrict__ V,
+                                                    double* __restrict__ W, const double* __restrict__ tau,
+                                                    const double* __restrict__ p, const double* __restrict__ pv, int npv) {
+    const double t = tau[k], kap = 0.5 * t * (t * hh_total(pv, npv));
+    const int r = k + 1 + blockIdx.x * HH_T + threadIdx.x;
+    if (r < K) W[(size_t)i * K + r] = t * p[r - k - 1] - kap * V[(size_t)i * K + r];
+}
+
+// Column k (rows k .. K-1): w of the panel's previous column (as hh_w_kernel), then
+// A(r, k) -= sum_{j < i} V(r, j) W(k, j) + W(r, j) V(k, j); the partial norms of rows
+// k + 2 .. K - 1 to norms[blockIdx.x].
+__global__ __launch_bounds__(HH_T) void hh_col_kernel(double* __restrict__ A, int K, int k, int i,
+                                                      const double* __restrict__ V, double* __restrict__ W,
+                                                      const double* __restrict__ tau, const double* __restrict__ p,
+                                                      const double* __restrict__ pv, int npv,
+                                                      double* __restrict__ norms) {
+    __shared__ double red[3][HH_R];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = k + blockIdx.x * HH_R + lane;
+    double a = 0.0;
+    if (i > 0) {
+        const double tk = tau[k - 1], kap = 0.5 * tk * (tk * hh_total(pv, npv));
+        // this wave's earlier columns j = wave, wave + 4, ... of the panel
+        double acc = 0.0;
+        if (r < K)
+#pragma unroll
+            for (int q = 0; q < TR_NB / 4; q++) {
+                const int j = wave + 4 * q;
+                if (j < i - 1)
+                    acc += V[(size_t)j * K + r] * W[(size_t)j * K + k] + W[(size_t)j * K + r] * V[(size_t)j * K + k];
+            }
+        if (wave > 0) red[wave - 1][lane] = acc;
         __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        double sigma = red[0], alpha = x[0];
-        if (sigma == 0.0) {
-            sh_tau = 0.0;
-            sh_beta = alpha;
-            sh_scale = 0.0;
-        } else {
-            double nrm = sqrt(alpha * alpha + sigma);
-            double beta = alpha <= 0 ? nrm : -nrm;
-            sh_tau = (beta - alpha) / beta;
-            sh_scale = 1.0 / (alpha - beta);
-            sh_beta = beta;
+        if (wave == 0 && r < K) {
+            const double vr = V[(size_t)(i - 1) * K + r], wr = tk * p[r - k] - kap * vr;
+            const double vk = V[(size_t)(i - 1) * K + k], wk = tk * p[0] - kap * vk;
+            W[(size_t)(i - 1) * K + r] = wr;
+            acc = ((acc + red[0][lane]) + (red[1][lane] + red[2][lane])) + (vr * wk + wr * vk);
+            a = A[(size_t)k * K + r] - acc;
+            A[(size_t)k * K + r] = a;
         }
-        tau[k] = sh_tau;
-        e[k] = sh_beta;
+    } else if (wave == 0 && r < K) {
+        a = A[(size_t)k * K + r];
     }
-    __syncthreads();
-    double sc = sh_scale;
-    for (int i = 1 + threadIdx.x; i < m; i += blockDim.x) x[i] *= sc;
-    if (threadIdx.x == 0) x[0] = 1.0;
+    if (wave == 0) {
+        const double s = wave_total(r >= k + 2 && r < K ? a * a : 0.0);
+        if (lane == 0) norms[blockIdx.x] = s;
+    }
 }
 
-// part[c][i] = sum_{j in chunk c} A22[i][j] v[j]   (A22 = A[k+1:, k+1:], v = A[k+1:, k]);
-// chunk c = blockIdx.y covers columns 256 c .. 256 c + 255
-__global__ __launch_bounds__(256) void hh_symv_kernel(const double* A, int K, int k, double* part) {
-    __shared__ double vs[256];
-    const int m = K - k - 1;
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    const int j0 = blockIdx.y * 256;
-    const double* v = A + (size_t)k * K + (k + 1);
-    vs[threadIdx.x] = (j0 + threadIdx.x < m) ? v[j0 + threadIdx.x] : 0.0;
-    __syncthreads();
-    if (i >= m) return;
-    double acc = 0;
-    const int jn = min(256, m - j0);
-    const double* col = A + (size_t)(k + 1 + j0) * K + (k + 1) + i;
-    for (int jj = 0; jj < jn; jj++) acc += col[(size_t)jj * K] * vs[jj];
-    part[(size_t)blockIdx.y * m + i] = acc;
+// The reflector of column k from its entries (below the diagonal in A) and the
+// partial norms: v = (1, scale a_2, ...), H = I - tau v v^T maps the column to beta e_1.
+struct HHRefl {
+    double tau, beta, scale;
+};
+__device__ __forceinline__ HHRefl hh_reflector(const double* __restrict__ x, const double* __restrict__ norms, int nn) {
+    const double sigma = hh_total(norms, nn), alpha = x[0];
+    if (sigma == 0.0) return HHRefl{0.0, alpha, 0.0};
+    const double nrm = sqrt(alpha * alpha + sigma), beta = alpha <= 0 ? nrm : -nrm;
+    return HHRefl{(beta - alpha) / beta, beta, 1.0 / (alpha - beta)};
 }
 
-// p[i] = sum_c part[c][i], chunks in order
-__global__ __launch_bounds__(256) void hh_symv_sum_kernel(const double* __restrict__ part, int nc, int m,
-                                                          double* __restrict__ p) {
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= m) return;
-    double acc = 0.0;
-    for (int c = 0; c < nc; c++) acc += part[(size_t)c * m + i];
-    p[i] = acc;
-}
-
-// w = tau p - (tau/2)(tau p . v) v  (one workgroup)
-__global__ __launch_bounds__(1024) void hh_w_kernel(const double* A, int K, int k, const double* tau, double* p) {
-    __shared__ double red[1024];
-    const int m = K - k - 1;
-    const double* v = A + (size_t)k * K + (k + 1);
-    const double t = tau[k];
-    double s = 0;
-    for (int i = threadIdx.x; i < m; i += blockDim.x) s += t * p[i] * v[i];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = blockDim.x / 2; w > 0; w >>= 1) {
-        if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+// Workgroups [0, nr nc): part[c][r] = sum over columns j of chunk c (cw <= 256 of them)
+// of A22[r][j] v[j], 256 rows each; then 2 i workgroups: ab[j] = W(:, j) . v, ab[i + j] =
+// V(:, j) . v; then nr workgroups: v to V(:, i), tau and beta.  A22 = A[k+1:, k+1:].
+__global__ __launch_bounds__(HH_T) void hh_symv_kernel(const double* __restrict__ A, int K, int k, int i,
+                                                       double* __restrict__ V, const double* __restrict__ W,
+                                                       const double* __restrict__ norms, int nn, int nr, int nc, int cw,
+                                                       double* __restrict__ part, double* __restrict__ ab,
+                                                       double* __restrict__ tau, double* __restrict__ e) {
+    __shared__ double vs[HH_T];
+    const int m = K - k - 1, t = threadIdx.x;
+    const double* x = A + (size_t)k * K + (k + 1);
+    const HHRefl H = hh_reflector(x, norms, nn);
+    int b = blockIdx.x;
+    if (b < nr * nc) {
+        const int c = b / nr, r = (b - c * nr) * HH_T + t, j0 = c * cw, jn = min(cw, m - j0);
+        if (t < jn) vs[t] = j0 + t == 0 ? 1.0 : x[j0 + t] * H.scale;
         __syncthreads();
+        if (r >= m) return;
+        const double* col = A + (size_t)(k + 1 + j0) * K + (k + 1) + r;
+        double acc0 = 0, acc1 = 0;
+        int j = 0;
+        for (; j + 16 <= jn; j += 16) {
+            double v[16];
+#pragma unroll
+            for (int q = 0; q < 16; q++) v[q] = col[(size_t)(j + q) * K];
+#pragma unroll
+            for (int q = 0; q < 16; q += 2) {
+                acc0 += v[q] * vs[j + q];
+                acc1 += v[q + 1] * vs[j + q + 1];
+            }
+        }
+        for (; j < jn; j++) acc0 += col[(size_t)j * K] * vs[j];
+        part[(size_t)c * m + r] = acc0 + acc1;
+        return;
     }
-    const double kap = 0.5 * t * red[0];
-    for (int i = threadIdx.x; i < m; i += blockDim.x) p[i] = t * p[i] - kap * v[i];
-}
-
-
-// ---- blocked reduction (panels of columns, deferred two-sided updates) -------
-// Within a panel the rank-2 updates of its reflectors are kept as the columns
-// of V (reflectors) and W (update vectors), K x nb column-major, zero above
-// their first row; the trailing matrix is updated once per panel.
-
-// Column k (rows k .. K-1) gets the panel's deferred updates from its first i
-// reflectors: A(r, k) -= sum_j V(r, j) W(k, j) + W(r, j) V(k, j).
-__global__ __launch_bounds__(256) void hh_colupd_kernel(double* A, int K, int k, int i, const double* __restrict__ V,
-                                                        const double* __restrict__ W) {
-    const int r = k + blockIdx.x * 256 + threadIdx.x;
-    if (r >= K) return;
-    double acc = 0.0;
-    for (int j = 0; j < i; j++)
-        acc += V[(size_t)j * K + r] * W[(size_t)j * K + k] + W[(size_t)j * K + r] * V[(size_t)j * K + k];
-    A[(size_t)k * K + r] -= acc;
-}
-
-// ab[j] = W(:, j) . v and ab[i + j] = V(:, j) . v over rows k+1 .. K-1 (v in
-// column k of A), j < i; one workgroup per dot, fixed-order reduction.
-__global__ __launch_bounds__(256) void hh_dots_kernel(const double* A, int K, int k, int i, const double* __restrict__ V,
-                                                      const double* __restrict__ W, double* __restrict__ ab) {
-    __shared__ double red[256];
-    const int j = blockIdx.x;
-    const double* x = (j < i ? W + (size_t)j * K : V + (size_t)(j - i) * K);
-    const double* v = A + (size_t)k * K;
-    double acc = 0.0;
-    for (int r = k + 1 + threadIdx.x; r < K; r += 256) acc += x[r] * v[r];
-    red[threadIdx.x] = acc;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+    b -= nr * nc;
+    if (b < 2 * i) {
+        const double* y = (b < i ? W + (size_t)b * K : V + (size_t)(b - i) * K) + (k + 1);
+        double acc = 0.0;
+        for (int r = t; r < m; r += HH_T) acc += y[r] * (r == 0 ? 1.0 : x[r] * H.scale);
+        acc = wave_total(acc);
+        if ((t & 63) == 0) vs[t >> 6] = acc;
         __syncthreads();
+        if (t == 0) ab[b] = (vs[0] + vs[1]) + (vs[2] + vs[3]);
+        return;
     }
-    if (threadIdx.x == 0) ab[j] = red[0];
+    b -= 2 * i;
+    const int r = b * HH_T + t;
+    if (r < m) V[(size_t)i * K + (k + 1) + r] = r == 0 ? 1.0 : x[r] * H.scale;
+    if (b == 0 && t == 0) {
+        tau[k] = H.tau;
+        e[k] = H.beta;
+    }
 }
 
-// p -= V' (W'^T v) + W' (V'^T v): the deferred updates' share of A22 v, p
-// indexed from row k+1.
-__global__ __launch_bounds__(256) void hh_corr_kernel(double* p, int K, int k, int i, const double* __restrict__ V,
-                                                      const double* __restrict__ W, const double* __restrict__ ab) {
-    const int r = k + 1 + blockIdx.x * 256 + threadIdx.x;
-    if (r >= K) return;
+// p = A22 v (the nc chunks' parts in order) - V (W^T v) - W (V^T v), indexed from row
+// k + 1; the partials of p . v; the reflector over column k of A.
+__global__ __launch_bounds__(HH_T) void hh_comb_kernel(double* __restrict__ A, int K, int k, int i,
+                                                       const double* __restrict__ V, const double* __restrict__ W,
+                                                       const double* __restrict__ part, int nc,
+                                                       const double* __restrict__ ab, double* __restrict__ p,
+                                                       double* __restrict__ pv) {
+    __shared__ double red[3][HH_R];
+    const int m = K - k - 1, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = blockIdx.x * HH_R + lane;
+    const double *v = V + (k + 1) + r, *w = W + (k + 1) + r;
     double acc = 0.0;
-    for (int j = 0; j < i; j++) acc += V[(size_t)j * K + r] * ab[j] + W[(size_t)j * K + r] * ab[i + j];
-    p[r - k - 1] -= acc;
-}
-
-// Column i of the panel: V(:, i) = v_k (rows k+1 .. K-1, from A), W(:, i) = w
-// (from p); zero above.
-__global__ __launch_bounds__(256) void hh_store_kernel(const double* A, int K, int k, int i, const double* __restrict__ w,
-                                                       double* __restrict__ V, double* __restrict__ W) {
-    const int r = blockIdx.x * 256 + threadIdx.x;
-    if (r >= K) return;
-    const bool in = r >= k + 1;
-    V[(size_t)i * K + r] = in ? A[(size_t)k * K + r] : 0.0;
-    W[(size_t)i * K + r] = in ? w[r - k - 1] : 0.0;
+    if (r < m) {
+        // this wave's chunks and panel columns, every fourth
+#pragma unroll 8
+        for (int c = wave; c < nc; c += 4) acc += part[(size_t)c * m + r];
+        double cor = 0.0;
+#pragma unroll
+        for (int q = 0; q < TR_NB / 4; q++) {
+            const int j = wave + 4 * q;
+            if (j < i) cor += v[(size_t)j * K] * ab[j] + w[(size_t)j * K] * ab[i + j];
+        }
+        acc -= cor;
+    }
+    if (wave > 0) red[wave - 1][lane] = acc;
+    __syncthreads();
+    if (wave > 0) return;
+    double dot = 0.0;
+    if (r < m) {
+        const double vr = v[(size_t)i * K], pr = (acc + red[0][lane]) + (red[1][lane] + red[2][lane]);
+        p[r] = pr;
+        A[(size_t)k * K + (k + 1) + r] = vr;
+        dot = pr * vr;
+    }
+    dot = wave_total(dot);
+    if (lane == 0) pv[blockIdx.x] = dot;
 }
 
 // Panel of reflectors k0 .. k0 + nb - 1 as a dense K x nb column-major
@@ -714,7 +778,7 @@ static int dense_eigen_top(Dev& D, double* dA, int K, int nev, std::vector<doubl
     std::vector<double> d(K), e(std::max(1, K - 1), 0.0);
     double *dtau = nullptr, *de = nullptr, *dp = nullptr, *dd = nullptr, *dpart = nullptr;
     DevScratch tmp;
-    OPSEC_HIP_TRY(ctx, tmp.alloc(&dpart, (size_t)((K + 255) / 256) * K * 8 + 8));
+    OPSEC_HIP_TRY(ctx, tmp.alloc(&dpart, (size_t)std::max(64, (K + 255) / 256) * K * 8 + 8));
     OPSEC_HIP_TRY(ctx, tmp.alloc(&dtau, (size_t)K * 8 + 8));
     OPSEC_HIP_TRY(ctx, tmp.alloc(&de, (size_t)K * 8 + 8));
     OPSEC_HIP_TRY(ctx, tmp.alloc(&dp, (size_t)std::max(K, nev) * 8 + 8));
@@ -725,30 +789,34 @@ static int dense_eigen_top(Dev& D, double* dA, int K, int nev, std::vector<doubl
     // the column, its reflector formed, and w = tau p - (tau^2/2)(p.v) v from
     // p = A22 v corrected for the deferred updates; after the panel, the
     // trailing matrix A22 -= V W^T + W V^T as two MFMA GEMMs.  The symmetric
-    // matrix-vector product is the only per-column pass over A22.
-    constexpr int TR_NB = 32;
-    double *dVr = nullptr, *dWr = nullptr, *dab = nullptr;
+    // matrix-vector product is the only per-column pass over A22: in chunks of 64
+    // columns while it is small (a 256-column chunk of a 1607 x 1607 matrix left
+    // 49 workgroups, 14 us), of 256 above 4096, where they fill the chip anyway.
+    const int nblk = (K + HH_R - 1) / HH_R;
+    double *dVr = nullptr, *dWr = nullptr, *dab = nullptr, *dred = nullptr;
     OPSEC_HIP_TRY(ctx, tmp.alloc(&dVr, (size_t)K * TR_NB * 8));
     OPSEC_HIP_TRY(ctx, tmp.alloc(&dWr, (size_t)K * TR_NB * 8));
     OPSEC_HIP_TRY(ctx, tmp.alloc(&dab, (size_t)2 * TR_NB * 8));
+    OPSEC_HIP_TRY(ctx, tmp.alloc(&dred, (size_t)2 * nblk * 8));
+    double *dnorm = dred, *dpv = dred + nblk;   // partials of the column norm and of p . v
     for (int k0 = 0; k0 + 2 < K; k0 += TR_NB) {
         const int nbp = std::min(TR_NB, K - 2 - k0);
+        int npv = 0;
         for (int i = 0; i < nbp; i++) {
-            const int k = k0 + i, m = K - k - 1;
-            if (i > 0)
-                hipLaunchKernelGGL(hh_colupd_kernel, dim3((K - k + 255) / 256), dim3(256), 0, D.s, dA, K, k, i, dVr,
-                                   dWr);
-            hipLaunchKernelGGL(hh_vector_kernel, dim3(1), dim3(1024), 0, D.s, dA, K, k, dtau, de);
-            const int nc = (m + 255) / 256;
-            hipLaunchKernelGGL(hh_symv_kernel, dim3(nc, nc), dim3(256), 0, D.s, dA, K, k, dpart);
-            hipLaunchKernelGGL(hh_symv_sum_kernel, dim3(nc), dim3(256), 0, D.s, dpart, nc, m, dp);
-            if (i > 0) {
-                hipLaunchKernelGGL(hh_dots_kernel, dim3(2 * i), dim3(256), 0, D.s, dA, K, k, i, dVr, dWr, dab);
-                hipLaunchKernelGGL(hh_corr_kernel, dim3(nc), dim3(256), 0, D.s, dp, K, k, i, dVr, dWr, dab);
-            }
-            hipLaunchKernelGGL(hh_w_kernel, dim3(1), dim3(1024), 0, D.s, dA, K, k, dtau, dp);
-            hipLaunchKernelGGL(hh_store_kernel, dim3((K + 255) / 256), dim3(256), 0, D.s, dA, K, k, i, dp, dVr, dWr);
+            const int k = k0 + i, m = K - k - 1, nn = (K - k + HH_R - 1) / HH_R, nr = (m + HH_T - 1) / HH_T,
+                      ncb = (m + HH_R - 1) / HH_R;
+            const int cw = m <= 4096 ? 64 : 256, nc = (m + cw - 1) / cw;
+            hipLaunchKernelGGL(hh_col_kernel, dim3(nn), dim3(HH_T), 0, D.s, dA, K, k, i, dVr, dWr, dtau, dp, dpv, npv,
+                               dnorm);
+            hipLaunchKernelGGL(hh_symv_kernel, dim3(nr * nc + 2 * i + nr), dim3(HH_T), 0, D.s, dA, K, k, i, dVr, dWr,
+                               dnorm, nn, nr, nc, cw, dpart, dab, dtau, de);
+            hipLaunchKernelGGL(hh_comb_kernel, dim3(ncb), dim3(HH_T), 0, D.s, dA, K, k, i, dVr, dWr, dpart, nc, dab, dp,
+                               dpv);
+            npv = ncb;
         }
+        const int kl = k0 + nbp - 1;
+        hipLaunchKernelGGL(hh_w_kernel, dim3((K - kl - 1 + HH_T - 1) / HH_T), dim3(HH_T), 0, D.s, K, kl, nbp - 1, dVr,
+                           dWr, dtau, dp, dpv, npv);
         const int r0 = k0 + nbp, m2 = K - r0;
         if (m2 > 0) {
             double* A22 = dA + (size_t)r0 * K + r0;

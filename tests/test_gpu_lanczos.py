@@ -52,6 +52,31 @@ def test_random_symmetric_vs_eigh(ctx, n, nev, block):
     np.testing.assert_allclose(V @ V.T, np.eye(nev), atol=1e-9)
 
 
+# one and a few columns, a panel of 32 columns and one more, blocks of 64 rows and one more, and a matrix
+# large enough for the wide column chunks of the symmetric product
+@pytest.mark.parametrize("n", [2, 3, 33, 34, 35, 65, 66, 130, 257, 4230])
+def test_dense_eigen_panel_edges(ctx, n):
+    """The dense symmetric solver at the edges of its panels and blocks: eigenvalues of a matrix of
+    known spectrum within 10 n eps of the largest (backward error of the tridiagonal reduction),
+    residuals and orthonormality alike."""
+    rng = np.random.default_rng(n)
+    lam = np.sort(rng.uniform(-1, 1, n))[::-1]
+    A = np.diag(lam)
+    for _ in range(3):   # three random reflections of the diagonal matrix
+        u = rng.normal(size=n)
+        u /= np.linalg.norm(u)
+        Au = A @ u
+        A = A - 2 * np.outer(u, Au) - 2 * np.outer(Au, u) + 4 * (u @ Au) * np.outer(u, u)
+    A = 0.5 * (A + A.T)
+    nev = max(1, min(n, (n + 2) // 3))
+    ev, V, nconv = ctx.lanczos_dense(A, nev)
+    tol = 10 * n * 2.0 ** -52
+    assert nconv == nev
+    assert np.abs(ev - lam[:nev]).max() <= tol + 1e-14
+    assert np.abs(A @ V.T - V.T * ev).max() <= tol + 1e-14
+    assert np.abs(V @ V.T - np.eye(nev)).max() <= 1e-9
+
+
 def test_klt_box_multiplets(ctx):
     """KL modes of the periodic 8^3 box: S is 3-level circulant, so its
     spectrum is the real DFT of the generator row, in cubic multiplets."""
