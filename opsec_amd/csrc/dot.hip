@@ -388,7 +388,7 @@ int opsec_count_galaxies(opsec_ctx* ctx, const opsec_galaxy* gals, int64_t ngals
     }
     for (int64_t off = 0; off < ngals; off += CHUNK) {
         const int64_t n = (ngals - off) < CHUNK ? (ngals - off) : CHUNK;
-        OPSEC_HIP_TRY(ctx, hipMemcpyAsync(d->d_gal, gals + off, (size_t)n * 16, hipMemcpyHostToDevice, ctx->stream));
+        OPSEC_HIP_TRY(ctx, stream_copy(ctx, d->d_gal, gals + off, (size_t)n * 16, hipMemcpyHostToDevice));
         hipLaunchKernelGGL(galaxy_keys_kernel, dim3(blocks_for(n, 256)), dim3(256), 0, ctx->stream, d->d_gal, n, g,
                            d->d_map, (uint32_t)ncells, d->d_key[0], d->d_w[0]);
         OPSEC_HIP_TRY(ctx, hipGetLastError());

@@ -447,7 +447,7 @@ int opsec_estimate_run(opsec_ctx* ctx, int nmodes, int nparams, const double* la
     double* dD = nullptr;
     DevScratch tmp;
     OPSEC_HIP_TRY(ctx, tmp.alloc(&dD, bytes));
-    OPSEC_HIP_TRY(ctx, hipMemcpyAsync(dD, D, bytes, hipMemcpyHostToDevice, ctx->stream));
+    OPSEC_HIP_TRY(ctx, stream_copy(ctx, dD, D, bytes, hipMemcpyHostToDevice));
     int rc = run_fisher(ctx, dD, nmodes, nparams, lambda, y, prior, mixing, prec, out);
     hipStreamSynchronize(ctx->stream);
     return rc;

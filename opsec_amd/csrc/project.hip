@@ -2028,7 +2028,7 @@ int opsec_modes_upload(opsec_ctx* ctx, const double* B, int ncells, int nmodes) 
     if ((rc = dev_realloc(ctx, (void**)&ctx->d_B, &capB, bytes))) return rc;
     ps->ldw = nt_pitch<double>(ncells);
     if ((rc = dev_realloc(ctx, (void**)&ps->d_Bw, &ps->cap_Bw, ps->ldw * nmodes * 8))) return rc;
-    OPSEC_HIP_TRY(ctx, hipMemcpyAsync(ctx->d_B, B, bytes, hipMemcpyHostToDevice, ctx->stream));
+    OPSEC_HIP_TRY(ctx, stream_copy(ctx, ctx->d_B, B, bytes, hipMemcpyHostToDevice));
     hipLaunchKernelGGL(scale_rows_kernel<double>, blocks_for(ps->ldw * nmodes), dim3(256), 0, ctx->stream, ctx->d_B,
                        ctx->d_nbar, ncells, nmodes, ps->d_Bw, ps->ldw);
     OPSEC_HIP_TRY(ctx, hipGetLastError());
@@ -2060,9 +2060,8 @@ int opsec_project(opsec_ctx* ctx, int nf, const int* funcs, int prec, double* P_
     if (rc) return rc;
     ctx->proj->funcs.assign(funcs, funcs + nf);
     if (P_packed) {
-        OPSEC_HIP_TRY(ctx, hipMemcpyAsync(P_packed, ctx->proj->d_P, (size_t)nf * packed_size(ctx->nmodes) * 8,
-                                          hipMemcpyDeviceToHost, ctx->stream));
-        OPSEC_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+        OPSEC_HIP_TRY(ctx, stream_copy(ctx, P_packed, ctx->proj->d_P, (size_t)nf * packed_size(ctx->nmodes) * 8,
+                                       hipMemcpyDeviceToHost));
     }
     return OPSEC_OK;
 }
@@ -2170,8 +2169,8 @@ int opsec_project_dense(opsec_ctx* ctx, int n, const double* S, int nmodes, cons
     OPSEC_HIP_TRY(ctx, tmp.alloc(&dS, (size_t)N * N * 8));
     OPSEC_HIP_TRY(ctx, tmp.alloc(&dB, (size_t)N * M * 8));
     OPSEC_HIP_TRY(ctx, tmp.alloc(&dP, (size_t)packed_size(M) * 8));
-    OPSEC_HIP_TRY(ctx, hipMemcpyAsync(dS, S, (size_t)N * N * 8, hipMemcpyHostToDevice, ctx->stream));
-    OPSEC_HIP_TRY(ctx, hipMemcpyAsync(dB, B, (size_t)N * M * 8, hipMemcpyHostToDevice, ctx->stream));
+    OPSEC_HIP_TRY(ctx, stream_copy(ctx, dS, S, (size_t)N * N * 8, hipMemcpyHostToDevice));
+    OPSEC_HIP_TRY(ctx, stream_copy(ctx, dB, B, (size_t)N * M * 8, hipMemcpyHostToDevice));
     if (prec != OPSEC_PREC_BF16X3) {
         int rc = prec == OPSEC_PREC_FP64 ? project_host_nt<double>(ctx, N, dS, M, dB, dP)
                                          : project_host_nt<float>(ctx, N, dS, M, dB, dP);
@@ -2199,10 +2198,8 @@ int opsec_project_dense(opsec_ctx* ctx, int n, const double* S, int nmodes, cons
     int rc = OPSEC_OK;
     if (e != hipSuccess) rc = set_error(ctx, OPSEC_EHIP, "projection launch: %s", hipGetErrorString(e));
     if (!rc) {
-        hipError_t e2 = hipMemcpyAsync(P_packed, dP, (size_t)packed_size(M) * 8, hipMemcpyDeviceToHost, ctx->stream);
-        hipError_t e3 = hipStreamSynchronize(ctx->stream);
-        if (e2 != hipSuccess || e3 != hipSuccess)
-            rc = set_error(ctx, OPSEC_EHIP, "projection copy-back: %s", hipGetErrorString(e2 ? e2 : e3));
+        hipError_t e2 = stream_copy(ctx, P_packed, dP, (size_t)packed_size(M) * 8, hipMemcpyDeviceToHost);
+        if (e2 != hipSuccess) rc = set_error(ctx, OPSEC_EHIP, "projection copy-back: %s", hipGetErrorString(e2));
     }
     return rc;
 }

@@ -2242,9 +2242,8 @@ int opsec_pair_table_get(opsec_ctx* ctx, int f, double* Q) {
     int rc = check_model(ctx, f);
     if (rc) return rc;
     if (!ctx->d_Q || !ctx->Q_valid[f]) return set_error(ctx, OPSEC_ESTATE, "pair table %d not built", f);
-    OPSEC_HIP_TRY(ctx, hipMemcpyAsync(Q, ctx->d_Q + (size_t)f * ctx->nkeys, (size_t)ctx->nkeys * 8,
-                                      hipMemcpyDeviceToHost, ctx->stream));
-    OPSEC_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
+    OPSEC_HIP_TRY(ctx, stream_copy(ctx, Q, ctx->d_Q + (size_t)f * ctx->nkeys, (size_t)ctx->nkeys * 8,
+                                   hipMemcpyDeviceToHost));
     return OPSEC_OK;
 }
 
@@ -2501,9 +2500,13 @@ int opsec_sig_block(opsec_ctx* ctx, const opsec_cell* cells, int ncells, const i
                            (double*)s_out.p, (size_t)lld);
         TRY(hipGetLastError());
         // copy rows back, only the ncols entries of each row (the rest of s is untouched)
-        TRY(hipMemcpy2DAsync(s, (size_t)lld * 8, s_out.p, (size_t)lld * 8, (size_t)ncols * 8, nrows,
-                             hipMemcpyDeviceToHost, st));
-        TRY(hipStreamSynchronize(st));
+        if (lld == ncols) {
+            TRY(stream_copy(ctx, s, s_out.p, (size_t)nrows * ncols * 8, hipMemcpyDeviceToHost));
+        } else {
+            TRY(hipMemcpy2DAsync(s, (size_t)lld * 8, s_out.p, (size_t)lld * 8, (size_t)ncols * 8, nrows,
+                                 hipMemcpyDeviceToHost, st));
+            TRY(hipStreamSynchronize(st));
+        }
 #undef TRY
     }
 done:

@@ -1,0 +1,53 @@
+"""Large host copies staged through pinned buffers: every byte arrives, and
+nothing beside the destination is touched."""
+import threading
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+MB = 1 << 20
+
+
+# under, at and over the least staged sizes (8 MB to the host, 32 MB to the device);
+# full 4 MB chunks with a last partial one, more of them than threads
+@pytest.mark.parametrize("n", [1, 8 * MB - 1, 8 * MB, 8 * MB + 1, 32 * MB - 1, 32 * MB, 32 * MB + 1, 70 * MB + 5])
+def test_round_trip_bytes(ctx, n):
+    src = np.random.default_rng(n).integers(0, 256, n, dtype=np.uint8)
+    p = ctx.dev_alloc(n)
+    try:
+        ctx.h2d(p, src)
+        frame = np.full(n + 130, 7, dtype=np.uint8)   # an odd host address
+        ctx.d2h(frame[65:65 + n], p)
+        assert np.array_equal(frame[65:65 + n], src)
+        assert np.all(frame[:65] == 7) and np.all(frame[65 + n:] == 7)
+        ctx.h2d(p, src[::-1].copy())                   # the buffers again, other bytes
+        back = np.empty(n, dtype=np.uint8)
+        ctx.d2h(back, p)
+        assert np.array_equal(back, src[::-1])
+    finally:
+        ctx.dev_free(p)
+
+
+def test_two_threads(ctx):
+    """Copies of two threads at once: one has the buffers, the other goes by the runtime."""
+    n = 40 * MB + 1
+    rng = np.random.default_rng(5)
+    srcs = [rng.integers(0, 256, n, dtype=np.uint8) for _ in range(2)]
+    outs = [np.zeros(n, dtype=np.uint8) for _ in range(2)]
+    ptrs = [ctx.dev_alloc(n) for _ in range(2)]
+
+    def run(i):
+        ctx.h2d(ptrs[i], srcs[i])
+        ctx.d2h(outs[i], ptrs[i])
+
+    try:
+        th = [threading.Thread(target=run, args=(i,)) for i in range(2)]
+        for t in th:
+            t.start()
+        for t in th:
+            t.join()
+        assert np.array_equal(outs[0], srcs[0]) and np.array_equal(outs[1], srcs[1])
+    finally:
+        for p in ptrs:
+            ctx.dev_free(p)
