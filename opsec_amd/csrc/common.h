@@ -220,6 +220,11 @@ int fisher_scratch_setup(opsec_ctx* ctx);
 // Rows of the packed upper triangle: column j starts at j(j+1)/2.
 inline int64_t packed_size(int64_t m) { return m * (m + 1) / 2; }
 
+// Workgroup barrier for data in LDS: unlike __syncthreads it does not wait for
+// this wave's outstanding accesses to memory (loads of the next tile, stores that
+// no other wave reads).
+__device__ __forceinline__ void lds_barrier() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+
 // Blocking copy ordered on the context's stream.  (hipMemcpy runs on the null
 // stream, which does not order against the context's non-blocking stream, so
 // a kernel queued on the context's stream could overtake it.)  Large copies

@@ -7,11 +7,11 @@
 //   f_n  = sum_k w_k D_n[k] R[k],      R[k] = delta_ij C_i - sum_n p_n D_n[k]
 //   q_n  = sum_k w_k D_n[k] y_i y_j
 // i.e. one Gram product G = X D^T with X = [w D_0 .. w D_{nb-1}, w R, w Y]
-// (nb + 2 rows, padded to 48, or to 64 for nb > 46) and D^T (padded likewise),
+// (nb + 2 rows, padded to a multiple of 16) and D^T (padded likewise),
 // run on MFMA (FP64 16x16x4, or FP32 16x16x4 for the FP32 traces).  Each
 // workgroup writes its partial Gram matrix; a second kernel adds the partials
-// in workgroup order, so F, f and q are the same bits on every run.  The
-// 48 x 48 (64 x 64) result is tiny; the inverse / matrix square root / window
+// in a fixed order, so F, f and q are the same bits on every run.  The
+// result (64 x 64 at most) is tiny; the inverse / matrix square root / window
 // normalisation on nb x nb runs on the host in FP64.
 #include <algorithm>
 #include <cmath>
@@ -24,14 +24,14 @@
 
 namespace opsec {
 
-// NF 16-row fragments per side: the padded Gram size is 16 NF (48 or 64).
-// Packed entries per workgroup iteration (one per thread while loading): 256
-// for FP32 traces at 48, 128 for FP64 at 48, 48 for 64 (LDS stays within
-// 100 KB).
+// NF 16-row fragments per side: the padded Gram size is 16 NF, from nb + 2.
+// Packed entries per workgroup iteration, one per thread while loading: as many
+// as leave two workgroups on a CU for NF <= 2 (67 KB of LDS), one for NF = 3
+// (100 KB) and for 64 rows in FP64.
 template <typename T, int NF>
 struct FShape {
     static constexpr int FG = 16 * NF;
-    static constexpr int KT = NF <= 3 ? (sizeof(T) == 4 ? 256 : 128) : 48;
+    static constexpr int KT = NF == 4 ? 48 : NF == 1 || sizeof(T) == 4 ? 256 : 128;
 };
 constexpr int FG_MAX = 64;
 // Partial Gram matrices: one per workgroup, at most FISHER_MAX_PARTS
@@ -63,6 +63,11 @@ __device__ __forceinline__ int packed_col(long long k) {
     return (int)j;
 }
 
+// Bound by one read of D, then by the MFMA and conversion work between the barriers
+// where LDS leaves one workgroup on a CU.  Padding to 16 NF instead of 48 at least, two
+// workgroups on a CU up to NF = 2 and the loads one tile ahead: 24 parameters, 1000
+// modes (96 MB, 19 us at the rate of a copy) FP64 104 -> 46 us, 40 parameters, 4000
+// modes (2.56 GB, 0.51 ms) FP32 0.91 -> 0.84 ms, 4 parameters, 40 modes 13 -> 6.6 us.
 template <typename T, int NF>
 __global__ __launch_bounds__(256) void fisher_gram_kernel(const double* D, long long K, int nb, const double* lambda,
                                                           const double* y, const double* prior, double* Gpart) {
@@ -89,34 +94,42 @@ __global__ __launch_bounds__(256) void fisher_gram_kernel(const double* D, long 
         if (row >= nb) Dt[row][t] = (T)0;
         if (row >= nb + 2) X[row][t] = (T)0;
     }
-    for (long long k0 = (long long)blockIdx.x * FK_TILE; k0 < K; k0 += (long long)gridDim.x * FK_TILE) {
-        __syncthreads();   // the previous tile's MFMAs are done with X and Dt
-        // one thread per packed entry: its weight, the rows of D (coalesced
-        // along k, loads independent of each other), the residual
-        // R = delta_ij C_i - sum_n p_n D_n in FP64 from the FP64 inputs, and
-        // the scaled rows
-        if (threadIdx.x < FK_TILE) {
-            const int t = threadIdx.x;
-            const long long k = k0 + t;
-            // all FG - 2 row loads are issued first (rows at and beyond nb
-            // load row nb - 1 and count as 0), so one tile costs one memory
-            // latency
-            const long long kc = k < K ? k : K - 1;
-            double v[FG - 2];
+    // Packed entry k0 + t belongs to thread t.  Its mode entries and rows of D (coalesced
+    // along k) are loaded one tile ahead, so that a tile's memory latency lies under the MFMAs of
+    // the tile before; rows from nb on (the last 15 at most) load row nb - 1 and
+    // count as 0.
+    double v[FG - 2], li = 0, lj = 0, yi = 0, yj = 0;
+    bool diag = false;
+    const int t = threadIdx.x;
+    const long long step = (long long)gridDim.x * FK_TILE;
+    auto load = [&](long long kt) {   // uniform row addresses, one 32-bit lane offset
+        const unsigned o = (unsigned)min((long long)t, K - 1 - kt);
+        const double* p = D + kt;
+        const long long k = kt + o;
+        const int j = packed_col(k), i = (int)(k - (long long)j * (j + 1) / 2);
+        diag = i == j;
+        li = lambda[i], lj = lambda[j], yi = y[i], yj = y[j];
 #pragma unroll
-            for (int n = 0; n < FG - 2; n++) v[n] = D[(size_t)min(n, nb - 1) * K + kc];
+        for (int n = 0; n < FG - 2; n++) v[n] = (p + (size_t)(n <= FG - 18 ? n : min(n, nb - 1)) * K)[o];
+    };
+    long long k0 = (long long)blockIdx.x * FK_TILE;
+    if (t < FK_TILE && k0 < K) load(k0);
+    for (; k0 < K; k0 += step) {
+        lds_barrier();   // the previous tile's MFMAs are done with X and Dt
+        // the entry's weight, the residual R = delta_ij C_i - sum_n p_n D_n in
+        // FP64 from the FP64 inputs, and the scaled rows
+        if (t < FK_TILE) {
+            const long long k = k0 + t;
             double w = 0, r = 0, yy = 0;
             if (k < K) {
-                int j = packed_col(k);
-                int i = (int)(k - (long long)j * (j + 1) / 2);
-                double ci = 1.0 + lambda[i], cj = 1.0 + lambda[j];
-                w = (i == j ? 0.5 : 1.0) / (ci * cj);
-                r = (i == j) ? ci : 0.0;
-                yy = y[i] * y[j];
+                const double ci = 1.0 + li, cj = 1.0 + lj;
+                w = (diag ? 0.5 : 1.0) / (ci * cj);
+                r = diag ? ci : 0.0;
+                yy = yi * yj;
             }
 #pragma unroll
             for (int n = 0; n < FG - 2; n++) {
-                const double vn = (n < nb && k < K) ? v[n] : 0.0;
+                const double vn = (n <= FG - 18 || n < nb) && k < K ? v[n] : 0.0;
                 const T vt = (T)vn;
                 Dt[n][t] = vt;
                 X[n][t] = (T)(w * (double)vt);
@@ -124,8 +137,9 @@ __global__ __launch_bounds__(256) void fisher_gram_kernel(const double* D, long 
             }
             X[nb][t] = (T)(w * r);
             X[nb + 1][t] = (T)(w * yy);
+            if (k0 + step < K) load(k0 + step);
         }
-        __syncthreads();
+        lds_barrier();
         // each wave takes FK_TILE / 4 entries = FK_TILE / 16 k-steps of 4
 #pragma unroll
         for (int s = 0; s < FK_TILE / 16; s++) {
@@ -196,13 +210,26 @@ static double* fisher_scratch_ptr(int device) {
     return g_scratch_done[device] ? g_scratch_ptr[device] : nullptr;
 }
 
-// G[e] = sum over the partials in workgroup order (FP64, fixed order).
-__global__ void fisher_sum_parts_kernel(const double* __restrict__ Gpart, int nparts, int FG, double* __restrict__ G) {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= FG * FG) return;
+// G[e] = sum over the partials (FP64, fixed order): 16 threads of a workgroup take
+// nparts / 16 consecutive partials of an element each, then their sums in order.
+// One thread per element over all partials is a chain of their load latencies: 123 us
+// for 512 partials of 48 x 48, 6 us here.
+__global__ __launch_bounds__(256) void fisher_sum_parts_kernel(const double* __restrict__ Gpart, int nparts, int FG,
+                                                               double* __restrict__ G) {
+    __shared__ double part[16][16];
+    const int c = threadIdx.x & 15, g = threadIdx.x >> 4;
+    const int n2 = FG * FG, e = blockIdx.x * 16 + c;   // FG is a multiple of 16
+    const int per = (nparts + 15) / 16, s0 = g * per, s1 = min(nparts, s0 + per);
     double acc = 0.0;
-    for (int s = 0; s < nparts; s++) acc += Gpart[(size_t)s * FG * FG + e];
-    G[e] = acc;
+#pragma unroll 8
+    for (int s = s0; s < s1; s++) acc += Gpart[(size_t)s * n2 + e];
+    part[g][c] = acc;
+    __syncthreads();
+    if (g == 0) {
+        double sum = 0.0;
+        for (int h = 0; h < 16; h++) sum += part[h][c];
+        G[e] = sum;
+    }
 }
 
 // The Gram outputs on the device: F (nb x nb row-major, symmetrised as
@@ -360,13 +387,24 @@ static int post_process(opsec_ctx* ctx, int nb, const std::vector<double>& G, in
     return OPSEC_OK;
 }
 
-// Padded Gram size and packed entries per tile for nb parameters.
-static void gram_shape(int nb, int prec, int* FG, int* KT) {
-    const bool big = nb + 2 > FShape<double, 3>::FG;
-    const bool f64 = prec == OPSEC_PREC_FP64;
-    *FG = big ? FShape<double, 4>::FG : FShape<double, 3>::FG;
-    *KT = f64 ? (big ? FShape<double, 4>::KT : FShape<double, 3>::KT)
-              : (big ? FShape<float, 4>::KT : FShape<float, 3>::KT);
+// 16-row fragments per side, padded Gram size and packed entries per tile for nb
+// parameters.
+template <typename T>
+static int gram_kt(int NF) {
+    return NF == 1 ? FShape<T, 1>::KT : NF == 2 ? FShape<T, 2>::KT : NF == 3 ? FShape<T, 3>::KT : FShape<T, 4>::KT;
+}
+static int gram_shape(int nb, int prec, int* FG, int* KT) {
+    const int NF = (nb + 2 + 15) / 16;
+    *FG = 16 * NF;
+    *KT = prec == OPSEC_PREC_FP64 ? gram_kt<double>(NF) : gram_kt<float>(NF);
+    return NF;
+}
+template <typename T>
+static void launch_gram_kernel(hipStream_t st, int NF, int nparts, const double* dD, long long K, int nb,
+                               const double* d_lambda, const double* d_y, const double* d_prior, double* d_parts) {
+    void (*const kern[4])(const double*, long long, int, const double*, const double*, const double*, double*) = {
+        fisher_gram_kernel<T, 1>, fisher_gram_kernel<T, 2>, fisher_gram_kernel<T, 3>, fisher_gram_kernel<T, 4>};
+    hipLaunchKernelGGL(kern[NF - 1], dim3(nparts), dim3(256), 0, st, dD, K, nb, d_lambda, d_y, d_prior, d_parts);
 }
 
 // Launch the Gram product of the nb packed matrices dD (M modes) into the
@@ -377,22 +415,13 @@ static void launch_gram(opsec_ctx* ctx, const double* dD, int M, int nb, const d
                         const double* d_prior, int prec, int nparts, double* d_parts, double* d_G) {
     const long long K = (long long)M * (M + 1) / 2;
     int FG, KT;
-    gram_shape(nb, prec, &FG, &KT);
-    const bool big = FG > FShape<double, 3>::FG;
-    if (prec == OPSEC_PREC_FP64 && !big)
-        hipLaunchKernelGGL((fisher_gram_kernel<double, 3>), dim3(nparts), dim3(256), 0, ctx->stream, dD, K, nb,
-                           d_lambda, d_y, d_prior, d_parts);
-    else if (prec == OPSEC_PREC_FP64)
-        hipLaunchKernelGGL((fisher_gram_kernel<double, 4>), dim3(nparts), dim3(256), 0, ctx->stream, dD, K, nb,
-                           d_lambda, d_y, d_prior, d_parts);
-    else if (!big)
-        hipLaunchKernelGGL((fisher_gram_kernel<float, 3>), dim3(nparts), dim3(256), 0, ctx->stream, dD, K, nb,
-                           d_lambda, d_y, d_prior, d_parts);
+    const int NF = gram_shape(nb, prec, &FG, &KT);
+    if (prec == OPSEC_PREC_FP64)
+        launch_gram_kernel<double>(ctx->stream, NF, nparts, dD, K, nb, d_lambda, d_y, d_prior, d_parts);
     else
-        hipLaunchKernelGGL((fisher_gram_kernel<float, 4>), dim3(nparts), dim3(256), 0, ctx->stream, dD, K, nb,
-                           d_lambda, d_y, d_prior, d_parts);
-    hipLaunchKernelGGL(fisher_sum_parts_kernel, dim3((FG * FG + 255) / 256), dim3(256), 0, ctx->stream, d_parts,
-                       nparts, FG, d_G);
+        launch_gram_kernel<float>(ctx->stream, NF, nparts, dD, K, nb, d_lambda, d_y, d_prior, d_parts);
+    hipLaunchKernelGGL(fisher_sum_parts_kernel, dim3(FG * FG / 16), dim3(256), 0, ctx->stream, d_parts, nparts, FG,
+                       d_G);
 }
 
 static int check_gram_args(opsec_ctx* ctx, int M, int nb, int prec) {

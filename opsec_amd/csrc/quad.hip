@@ -382,9 +382,6 @@ __device__ __forceinline__ double pair_f64(double x) {
     const unsigned hi = __builtin_amdgcn_mov_dpp((unsigned)(b >> 32), 0xB1, 0xF, 0xF, true);
     return __builtin_bit_cast(double, (unsigned long long)hi << 32 | lo);
 }
-// Workgroup barrier for data in LDS: unlike __syncthreads it does not wait for
-// this wave's outstanding stores to the pool, which only wave 0 reads.
-__device__ __forceinline__ void lds_barrier() { __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 // Order of one wave's own accesses across its lanes (they issue in order).
 __device__ __forceinline__ void wave_order() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); }
 

@@ -191,6 +191,27 @@ def test_estimate_many_bands(ctx, npar, prec, tol):
             ctx.estimate(lam, D2, y, np.append(prior, 1.0), lib.OPSEC_MIX_IDENTITY, prec)
 
 
+# the first and last parameter count of a padded size (nb + 2 to a multiple of 16);
+# packed entries under, at and over one tile (M = 22: 253 entries, 23: 276), and
+# M = 600: more than one tile for each of 512 workgroups of 256 entries.  The
+# chains are 64 tile steps and 48 partials: 1e-10 (FP64) and 1e-5 (FP32, tiles'
+# sums closed in FP64) of the largest element bound them with room
+@pytest.mark.parametrize("prec,tol", [(lib.OPSEC_PREC_FP64, 1e-10), (lib.OPSEC_PREC_FP32, 1e-5)])
+@pytest.mark.parametrize("M,npar", [(1, 1), (22, 14), (23, 15), (150, 30), (150, 31), (600, 14), (600, 30), (600, 31)])
+def test_estimate_padded_sizes(ctx, M, npar, prec, tol):
+    rng = np.random.default_rng(1000 * npar + M)
+    lam = np.sort(rng.uniform(0.05, 5, M))[::-1].copy()
+    diag = np.cumsum(np.arange(1, M + 1)) - 1
+    D = 0.1 * rng.normal(size=(npar, M * (M + 1) // 2))
+    D[:, diag] += rng.uniform(0.5, 1.5, (npar, M))
+    y = np.sqrt(1 + lam) * rng.normal(size=M)
+    prior = rng.uniform(0.5, 2.0, npar)
+    got = ctx.estimate(lam, D, y, prior, lib.OPSEC_MIX_IDENTITY, prec)
+    ref = _orc_estimate(lam, D, y, prior, lib.OPSEC_MIX_IDENTITY)
+    for k in ("F", "q", "f"):
+        np.testing.assert_allclose(got[k], ref[k], rtol=tol, atol=tol * np.abs(ref[k]).max(), err_msg=k)
+
+
 def test_estimate_fp32_traces(ctx):
     rng = np.random.default_rng(5)
     M, npar = 300, 5
