@@ -1285,31 +1285,35 @@ __global__ __launch_bounds__(256) void gm_thread_kernel(XiModelDev m, GMJobs job
     if (threadIdx.x == 0 && blk) atomicAdd(nevals, blk);
 }
 
-// ---- GAUSS: the tensor rule, a node slab per thread -------------------------
+// ---- GAUSS: the tensor rule, node columns per thread ------------------------
 
-// One thread per (integral, a): the b and c sums of x-node a; the a == 0
-// thread of each integral then adds the n slab sums in node order, so the
-// result is the plain a-outer triple sum.  256 / n integrals per workgroup.
-__global__ __launch_bounds__(256) void tent_kernel(XiModelDev m, const GaussJob* jobs, int njobs, TentRule rule,
-                                                   double L, double* Q, size_t qstride) {
-    __shared__ double s_s[64], s_w[64];
-    __shared__ double slab[256];
-    const int n = rule.n;
+// Bound by the evaluations of xi (a divide, a square root and the band's sines each);
+// with few integrals by the chain of a thread's own.  A thread takes the c sums of
+// `bs` columns (a, b .. b + bs - 1) of an integral's n^2; one thread per a then adds
+// the b sums and one the a sum, each in node order, so the result is the plain
+// a-outer triple sum, the same bits for any bs.  864 integrals of 8^3 nodes (one column
+// per thread; a thread per a before): 59 -> 12 us; 1.3 million of 6^3 (6 columns, all
+// of an a, as before): 1.7 ms.
+constexpr int TENT_BS = 8, TENT_THREADS = 512;
+__global__ __launch_bounds__(TENT_THREADS) void tent_kernel(XiModelDev m, const GaussJob* jobs, int njobs,
+                                                             TentRule rule, int per, int bs, double L, double* Q,
+                                                             size_t qstride) {
+    __shared__ double s_s[32], s_w[32];
+    __shared__ double col[TENT_THREADS * TENT_BS], slab[TENT_THREADS];
+    const int n = rule.n, n2 = n * n, groups = n / bs, tpi = n * groups;   // threads per integral
     for (int i = threadIdx.x; i < n; i += blockDim.x) {
         s_s[i] = rule.s[i];
         s_w[i] = rule.w[i];
     }
     __syncthreads();
-    const int per = blockDim.x / n;   // integrals per workgroup
-    const int local = threadIdx.x / n, a = threadIdx.x - local * n;
-    const long long jb = (long long)blockIdx.x * per + local;
-    const bool live = local < per && jb < njobs;
-    if (live) {
-        const GaussJob J = jobs[jb];
+    const long long j0 = (long long)blockIdx.x * per;
+    const int live = (int)min((long long)per, njobs - j0);   // integrals here
+    for (int q = threadIdx.x; q < live * tpi; q += blockDim.x) {   // twice for one integral of over 512
+        const int local = q / tpi, r = q - local * tpi, a = r / groups, b0 = (r - a * groups) * bs;
+        const GaussJob J = jobs[j0 + local];
         const XiDesc xd = m.desc[J.f];
         const double rx = min_image(J.D[0] + s_s[a] * J.h[0], L);
-        double accy = 0;
-        for (int b = 0; b < n; b++) {
+        for (int b = b0; b < b0 + bs; b++) {
             double ry = min_image(J.D[1] + s_s[b] * J.h[1], L);
             double rxy2 = rx * rx + ry * ry;
             double accz = 0;
@@ -1317,22 +1321,28 @@ __global__ __launch_bounds__(256) void tent_kernel(XiModelDev m, const GaussJob*
                 double rz = min_image(J.D[2] + s_s[c] * J.h[2], L);
                 accz += s_w[c] * xi_eval(m, xd, sqrt(rxy2 + rz * rz));
             }
-            accy += s_w[b] * accz;
+            col[local * n2 + a * n + b] = accz;
         }
-        slab[threadIdx.x] = accy;
     }
     __syncthreads();
-    if (live && a == 0) {
+    if (threadIdx.x < live * n) {
+        const int a = threadIdx.x;   // (integral, a)
+        double accy = 0;
+        for (int b = 0; b < n; b++) accy += s_w[b] * col[a * n + b];
+        slab[a] = accy;
+    }
+    __syncthreads();
+    if (threadIdx.x < live) {
         double acc = 0;
-        for (int i = 0; i < n; i++) acc += s_w[i] * slab[threadIdx.x + i];
-        const GaussJob& J = jobs[jb];
+        for (int i = 0; i < n; i++) acc += s_w[i] * slab[threadIdx.x * n + i];
+        const GaussJob& J = jobs[j0 + threadIdx.x];
         Q[(size_t)J.f * qstride + J.key] = acc;
     }
 }
 
-// Near pairs: composite rule.  Each integral is spread over gridDim.y
-// workgroups of 256 threads, one (a, b) node column per thread; a workgroup's
-// tree-reduced partial goes to part[job * gridDim.y + y].
+// Near pairs: composite rule (64 nodes per axis).  Each integral is spread over
+// gridDim.y workgroups of 256 threads, one (a, b) node column per thread; a
+// workgroup's tree-reduced partial goes to part[job * gridDim.y + y].
 __global__ __launch_bounds__(256) void tent_near_kernel(XiModelDev m, const GaussJob* jobs, TentRule rule, double L,
                                                         double* part) {
     __shared__ double s_s[64], s_w[64];
@@ -1376,6 +1386,60 @@ __global__ void tent_near_sum_kernel(const GaussJob* jobs, int njobs, int nsplit
     double acc = 0;
     for (int i = 0; i < nsplit; i++) acc += part[(size_t)j * nsplit + i];
     Q[(size_t)jobs[j].f * qstride + jobs[j].key] = acc;
+}
+
+// The same for few near integrals, where a thread's 64 evaluations in a row are the
+// kernel's time: a wavefront takes NEAR_COLS columns, one node per lane, and one lane
+// per column then adds its 64 values in node order.  The column sums go to
+// colsum[job * n * n + ab]; tent_near_cols_sum_kernel adds them as the workgroup
+// trees and the partials above do, so the bits are the same.  4 integrals: 63 -> 18 us
+// with the sum.  It is taken up to NEAR_COLS_MAX = 128 integrals, about where the
+// other's 16 workgroups each fill the card: calls of 32 integrals 148 -> 128 us, of 128
+// 300 either way.
+constexpr int NEAR_N = 64, NEAR_COLS = 4;
+constexpr size_t NEAR_COLS_MAX = 128;
+__global__ __launch_bounds__(256) void tent_near_cols_kernel(XiModelDev m, const GaussJob* jobs, TentRule rule,
+                                                             double L, double* colsum) {
+    __shared__ double s_w[NEAR_N], val[4 * NEAR_COLS][NEAR_N + 1];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (threadIdx.x < NEAR_N) s_w[lane] = rule.w[lane];
+    const GaussJob J = jobs[blockIdx.x];
+    const XiDesc xd = m.desc[J.f];
+    const int ab0 = blockIdx.y * 4 * NEAR_COLS;
+    const double rz = min_image(J.D[2] + rule.s[lane] * J.h[2], L);
+    for (int k = 0; k < NEAR_COLS; k++) {
+        const int q = wave * NEAR_COLS + k, a = (ab0 + q) / NEAR_N, b = (ab0 + q) % NEAR_N;
+        const double rx = min_image(J.D[0] + rule.s[a] * J.h[0], L);
+        const double ry = min_image(J.D[1] + rule.s[b] * J.h[1], L);
+        const double rxy2 = rx * rx + ry * ry;
+        val[q][lane] = xi_eval(m, xd, sqrt(rxy2 + rz * rz));
+    }
+    __syncthreads();
+    if (threadIdx.x < 4 * NEAR_COLS) {
+        const int q = threadIdx.x, a = (ab0 + q) / NEAR_N, b = (ab0 + q) % NEAR_N;
+        double accz = 0;
+        for (int c = 0; c < NEAR_N; c++) accz += s_w[c] * val[q][c];
+        colsum[(size_t)blockIdx.x * NEAR_N * NEAR_N + ab0 + q] = s_w[a] * s_w[b] * accz;
+    }
+}
+
+__global__ __launch_bounds__(256) void tent_near_cols_sum_kernel(const GaussJob* jobs, const double* colsum, double* Q,
+                                                                 size_t qstride) {
+    constexpr int NS = NEAR_N * NEAR_N / 256;
+    __shared__ double red[NS][256];
+    for (int y = 0; y < NS; y++)
+        red[y][threadIdx.x] = colsum[((size_t)blockIdx.x * NS + y) * 256 + threadIdx.x];
+    __syncthreads();
+    for (int l = 7; l >= 0; l--) {
+        const int w = 1 << l;
+        for (int e = threadIdx.x; e < NS << l; e += 256) red[e >> l][e & (w - 1)] += red[e >> l][(e & (w - 1)) + w];
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        double acc = 0;
+        for (int y = 0; y < NS; y++) acc += red[y][0];
+        Q[(size_t)jobs[blockIdx.x].f * qstride + jobs[blockIdx.x].key] = acc;
+    }
 }
 
 // ---- first-pair search and job construction --------------------------------
@@ -1476,8 +1540,31 @@ static int make_tent_rule(opsec_ctx* ctx, int nodes, TentRule* r) {
     return OPSEC_OK;
 }
 
+// The split of tent_kernel: columns per thread, integrals per workgroup, its threads.
+// As many columns as leave each SIMD twelve wavefronts, four rounds of the three that
+// its registers allow, else one: with less, the last round is too empty (12^3 keys of
+// 8 bands and 8 nodes: 2 columns, 6.7 wavefronts 181 us, 1 column 139 for the call),
+// with one always, the sums and barriers of a workgroup come too often (32^3 keys of 40
+// bands and 6 nodes: 1.83 ms against 1.74).  Then the fullest wavefronts, at most 256
+// threads if they are as full.
+static void tent_split(const opsec_ctx* ctx, int n, size_t njobs, int* per, int* bs, int* threads) {
+    *bs = 1;
+    for (int d = 2; d <= std::min(n, TENT_BS); d++)
+        if (n % d == 0 && njobs * (n * n / d) >= (size_t)12 * 4 * 64 * std::max(1, ctx->num_cus)) *bs = d;
+    const int tpi = n * n / *bs;
+    auto pad = [&](int p) { return (p * tpi + 63) & ~63; };
+    int best = 1;
+    for (int p = 2; p * tpi <= TENT_THREADS; p++) {
+        const int u = p * pad(best), v = best * pad(p);   // the fuller one has more integrals per thread
+        if (u > v || (u == v && pad(p) <= 256)) best = p;
+    }
+    *per = best;
+    *threads = std::min(TENT_THREADS, pad(best));
+}
+
 static void make_near_rule(TentRule* r) {
     const int panels = 4, q = 8;
+    static_assert(2 * 4 * 8 == NEAR_N, "nodes per axis of the near rule");
     double x[8], w[8];
     gauss_legendre(q, x, w);
     int m = panels * q;   // nodes per half
@@ -1797,10 +1884,12 @@ static int run_quadrature(opsec_ctx* ctx, int nf, const int* funcs, const std::v
         }
         const size_t nfar = far.size() * nf, nnear = nearj.size() * nf, nj = nfar + nnear;
         const size_t ntmpl = far.size() + nearj.size();
-        // near partials after the jobs, templates and function list
-        const int nsplit = (nrule.n * nrule.n + 255) / 256;
+        // near partials after the jobs, templates and function list: the columns' where
+        // the workgroups of 256 columns would leave most of the card idle
+        const bool near_cols = nnear <= NEAR_COLS_MAX;
+        const int nsplit = (nrule.n * nrule.n + 255) / 256, nnpart = near_cols ? nrule.n * nrule.n : nsplit;
         const size_t part_off = (sizeof(GaussJob) * (nj + ntmpl) + sizeof(int) * nf + 255) & ~(size_t)255;
-        if ((rc = dev_realloc(ctx, &ctx->d_jobs, &ctx->cap_jobs, part_off + sizeof(double) * nnear * nsplit)))
+        if ((rc = dev_realloc(ctx, &ctx->d_jobs, &ctx->cap_jobs, part_off + sizeof(double) * nnear * nnpart)))
             return rc;
         GaussJob* dj = (GaussJob*)ctx->d_jobs;
         GaussJob* dt = dj + nj;
@@ -1820,12 +1909,20 @@ static int run_quadrature(opsec_ctx* ctx, int nf, const int* funcs, const std::v
             hipLaunchKernelGGL(expand_jobs_kernel, dim3((unsigned)((nnear + 255) / 256)), dim3(256), 0, ctx->stream,
                                dt + far.size(), (int)nearj.size(), dfun, nf, dj + nfar);
         if (nfar) {
-            const size_t per = 256 / rule.n;
-            hipLaunchKernelGGL(tent_kernel, dim3((unsigned)((nfar + per - 1) / per)), dim3(256), 0, ctx->stream, mv,
-                               dj, (int)nfar, rule, ctx->sv.L, dQ, nkeys);
+            int per, bs, threads;
+            tent_split(ctx, rule.n, nfar, &per, &bs, &threads);
+            hipLaunchKernelGGL(tent_kernel, dim3((unsigned)((nfar + per - 1) / per)), dim3(threads), 0, ctx->stream, mv,
+                               dj, (int)nfar, rule, per, bs, ctx->sv.L, dQ, nkeys);
             OPSEC_HIP_TRY(ctx, hipGetLastError());
         }
-        if (nnear) {
+        if (nnear && near_cols) {
+            hipLaunchKernelGGL(tent_near_cols_kernel,
+                               dim3((unsigned)nnear, NEAR_N * NEAR_N / (4 * NEAR_COLS)), dim3(256), 0, ctx->stream, mv,
+                               dj + nfar, nrule, ctx->sv.L, dpart);
+            hipLaunchKernelGGL(tent_near_cols_sum_kernel, dim3((unsigned)nnear), dim3(256), 0, ctx->stream, dj + nfar,
+                               dpart, dQ, nkeys);
+            OPSEC_HIP_TRY(ctx, hipGetLastError());
+        } else if (nnear) {
             hipLaunchKernelGGL(tent_near_kernel, dim3((unsigned)nnear, (unsigned)nsplit), dim3(256), 0, ctx->stream, mv,
                                dj + nfar, nrule, ctx->sv.L, dpart);
             hipLaunchKernelGGL(tent_near_sum_kernel, dim3((unsigned)((nnear + 255) / 256)), dim3(256), 0, ctx->stream,

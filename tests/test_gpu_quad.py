@@ -155,6 +155,35 @@ def test_gauss_sig_block_vs_oracle(c1):
         np.testing.assert_allclose(s, ref, rtol=1e-12, atol=1e-12 * np.abs(ref).max(), err_msg=f"f={f}")
 
 
+# node counts with 1 to 8 columns per thread when 24 bands are done at once (3 of 6, 5 of
+# 10, 7 of 14, 2 of 22, 8 of 24 and 32) and one column for a band alone, which at 24 and 32
+# nodes takes more than a thread per column; 24 bands have 192 near integrals, one has 8
+@pytest.mark.parametrize("nodes", [2, 6, 10, 14, 22, 24, 32])
+def test_gauss_tables_independent_of_split(ctx, nodes):
+    """A band's GAUSS table is the same bits alone and among 24 bands, and is the oracle's."""
+    lo, hi = synth.linear_bands(24, 0.01, 0.3)
+    ctx.model_real(GOLD["pk_k"], GOLD["pk_P"], lo, hi, lib.OPSEC_XI_TABLE)
+    n = 16
+    cells = synth.box_cells(n)
+    sv = lib.survey_box(n)
+    ctx.cells_upload(cells, sv)
+    q = ctx.quad(lib.OPSEC_QUAD_GAUSS, nodes=nodes, near=2)
+    ctx.pair_tables(list(range(1, 25)), q)
+    tables = [ctx.pair_table(f) for f in (1, 13, 24)]
+    orc = O.oracle()
+    r768, tabs = O.oracle_tables(GOLD["pk_k"], GOLD["pk_P"], lo, hi)
+    rows, cols = np.array([0], dtype=np.int32), np.arange(n ** 3, dtype=np.int32)
+    for f, t in zip((1, 13, 24), tables):
+        ctx.pair_tables([f], q)
+        assert np.array_equal(ctx.pair_table(f), t), f
+    xi = O.XiHandle(0, r768, tabs[24])
+    ref = np.zeros((1, n ** 3))
+    orc.orc_sig_block(C.byref(xi.s), cells.ctypes.data, n ** 3, n, n, n, 400.0, O.ptr(rows), 1, O.ptr(cols), n ** 3,
+                      O.ptr(ref), n ** 3, 1, 0, 0, 0, nodes, 2)
+    s = ctx.sig_block(cells, rows, cols, 24, sv, q)
+    np.testing.assert_allclose(s, ref, rtol=1e-12, atol=1e-12 * np.abs(ref).max())
+
+
 def test_pair_tables_and_assembly_vs_reference(c1):
     """Device-resident pair tables and assembly for the full 12^3 matrix vs the reference rows."""
     cells = synth.box_cells(12)
