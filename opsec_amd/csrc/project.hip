@@ -1840,7 +1840,7 @@ static int run_project_toeplitz_nt(opsec_ctx* ctx, int nb, const int* funcs, int
 // Dense FP64 / FP32 projection of the bands funcs[0..nb) in groups: stage 1
 // keeps the group's products C_p = T_p B' (N x M each), so a group holds at most
 // DENSE_GROUP_BYTES of them (all 40 bands of the 32^3 box fit; the 50 bands of
-// the 65536-cell shell at 6000 modes take seven groups).  Within a group stage 1
+// the 65536-cell shell at 6000 modes take four groups).  Within a group stage 1
 // takes the rows of T_p in panels of NT_PANEL_BYTES (several bands per launch
 // where their whole T_p fit).  T_p is symmetric: C_p's row m (mode m, cells
 // contiguous) is row m of B' times the rows of T_p.
