@@ -35,6 +35,13 @@ inline size_t nt_pitch(size_t k) {
     return nt_kpad<T>(k) + nt_bk<T>();
 }
 
+// Position in an operand row of its k-th value, and k of a position, in the serial order
+// of an FP32 product.  Lane group g of an MFMA takes the chunk 4 h + g of a step, so
+// element e of it is MFMA e's: with k = 16 h + 4 e + g there, every MFMA adds four
+// consecutive k, and a product is the chain of fused multiply-adds over k, the bits
+// of any kernel that sums so.  Both operands of a product use the order or neither does.
+__host__ __device__ __forceinline__ int nt_serial(int k) { return (k & ~15) | (k & 3) << 2 | (k >> 2 & 3); }
+
 template <typename T>
 struct NtMma;
 template <>
@@ -68,6 +75,7 @@ struct NtArgs {
     int N;
     int ksteps;            // K / nt_bk
     int nbat, nz;          // batches per band, nbat * bands
+    bool serial = false;   // K in one piece: the operands are in the serial order
     // set by launch_nt_gemm
     int item0 = 0;         // first work item of the launch (item = z * tiles + tile)
     int nsplit = 1;        // split-K launch: its items, each in gridDim.x / nsplit parts
@@ -76,13 +84,14 @@ struct NtArgs {
 
 // Epilogues: base(band, b), then put(base, m, n, M, value).
 template <typename T>
-struct NtRows {              // C[m * ld + n], n < nw (padding columns included)
+struct NtRows {              // C[m * ld + n], n < nw (padding columns included), serial: in that order
     T* p;
     size_t ld, b_stride, q_stride;
     int nw;
+    bool serial = false;
     __device__ __forceinline__ T* base(int q, int b) const { return p + q * q_stride + b * b_stride; }
     __device__ __forceinline__ void put(T* o, int m, int n, int M, T v) const {
-        if (m < M && n < nw) o[(size_t)m * ld + n] = v;
+        if (m < M && n < nw) o[(size_t)m * ld + (serial ? nt_serial(n) : n)] = v;
     }
     static constexpr bool lower = false;
 };
@@ -334,7 +343,7 @@ inline int launch_nt_gemm(opsec_ctx* ctx, NtWork& ws, NtArgs<T> g, const Out& O)
     hipStream_t s = ctx->stream;
     const int nmb = (g.M + NT_BM - 1) / NT_BM, nnb = (g.N + NT_BN - 1) / NT_BN;
     const int total = nt_tiles(nmb, nnb, Out::lower) * g.nz, rest = total % (2 * cus);
-    const int parts = nt_split(rest, g.ksteps, cus), whole = parts > 1 ? total - rest : total;
+    const int parts = g.serial ? 1 : nt_split(rest, g.ksteps, cus), whole = parts > 1 ? total - rest : total;
     g.item0 = 0;
     g.nsplit = 1;
     if (whole > 0) hipLaunchKernelGGL((nt_gemm_kernel<T, Out, false>), dim3(whole), dim3(256), NT_LDS, s, g, O);

@@ -116,13 +116,24 @@ struct ProjState {
 // kernel waiting on table gathers.  Writing and reading a panel costs 16 B per
 // element against 2 M flops.
 
+// FP32 operands may be in nt_gemm.h's serial order (`serial`): column c of a row is then
+// stored at nt_serial(c).  It keeps the sums of a shell's FP32 projection, and of a given
+// matrix's, the plain chains over k, the same bits whatever the number of bands in a call
+// or of CUs.  A box's FP32 sums are not ordered: split over K where that pays, they are
+// nearer to the 64-bit product (a 6686-cell footprint with 777 modes: 6.6e-7 of the norm,
+// 1.5e-6 in the serial order).
+template <typename T>
+static bool serial_sums(const SurveyDev& sv) {
+    return std::is_same<T, float>::value && sv.coordsys == OPSEC_COORD_SPHERICAL;
+}
+
 // out[z][i][c] = Q_f[key(row0 + i, c)], f = funcs[z], i < nrows, c < N; zero for N <= c < Kp.
 // Tile of 8 rows x 512 columns per 256-thread block, two columns per thread; the
 // column coordinates in LDS.
 template <typename T>
 __global__ __launch_bounds__(256) void gen_rows_kernel(const double* __restrict__ Q, size_t qstride,
                                                        const int* __restrict__ funcs, const int* __restrict__ cellidx,
-                                                       PairKey K, int N, int row0, int nrows, int Kp,
+                                                       PairKey K, int N, int row0, int nrows, int Kp, bool serial,
                                                        T* __restrict__ out, size_t ld, size_t zstride) {
     __shared__ int cx[512], cy[512], cz[512];
     const int j0 = blockIdx.x * 512, i0 = blockIdx.y * 8;
@@ -137,6 +148,7 @@ __global__ __launch_bounds__(256) void gen_rows_kernel(const double* __restrict_
     T* o = out + (size_t)blockIdx.z * zstride;
     const int t = 2 * threadIdx.x, j = j0 + t;
     if (j >= Kp) return;
+    const int t0 = serial ? nt_serial(t) : t, t1 = serial ? nt_serial(t + 1) : t + 1;   // the columns stored at j, j + 1
     typedef T pair_t __attribute__((ext_vector_type(2)));
 #pragma unroll
     for (int r = 0; r < 8; r++) {
@@ -145,20 +157,21 @@ __global__ __launch_bounds__(256) void gen_rows_kernel(const double* __restrict_
         const int* ca = cellidx + 3 * (size_t)(row0 + i);
         const int ax = ca[0], ay = ca[1], az = ca[2];
         pair_t v;
-        v[0] = j < N ? (T)q[K(ax, ay, az, cx[t], cy[t], cz[t])] : (T)0;
-        v[1] = j + 1 < N ? (T)q[K(ax, ay, az, cx[t + 1], cy[t + 1], cz[t + 1])] : (T)0;
+        v[0] = j0 + t0 < N ? (T)q[K(ax, ay, az, cx[t0], cy[t0], cz[t0])] : (T)0;
+        v[1] = j0 + t1 < N ? (T)q[K(ax, ay, az, cx[t1], cy[t1], cz[t1])] : (T)0;
         *(pair_t*)(o + (size_t)i * ld + j) = v;
     }
 }
 
 // out[i][c] = X[i * ldx + c] for c < cols, zero for cols <= c < ld.
 template <typename T>
-__global__ void pad_rows_kernel(const double* __restrict__ X, size_t ldx, int rows, int cols, T* __restrict__ out,
-                                size_t ld) {
+__global__ void pad_rows_kernel(const double* __restrict__ X, size_t ldx, int rows, int cols, bool serial,
+                                T* __restrict__ out, size_t ld) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (size_t)rows * ld) return;
-    const size_t r = i / ld, c = i - r * ld;
-    out[i] = c < (size_t)cols ? (T)X[r * ldx + c] : (T)0;
+    const size_t r = i / ld;
+    const int p = (int)(i - r * ld), c = serial ? nt_serial(p) : p;
+    out[i] = c < cols ? (T)X[r * ldx + c] : (T)0;
 }
 
 // ---- split-BF16x3 on pre-split planes --------------------------------------------
@@ -813,11 +826,12 @@ __global__ void sum_parts_kernel(const float* __restrict__ part, int nparts, siz
 
 // B' = diag(w) B with w = sqrt(Nbar), rows padded with zeros to ldw.
 template <typename T>
-__global__ void scale_rows_kernel(const double* B, const double* nbar, int N, int M, T* Bw, size_t ldw) {
+__global__ void scale_rows_kernel(const double* B, const double* nbar, int N, int M, bool serial, T* Bw, size_t ldw) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= ldw * M) return;
-    const size_t n = i / ldw, a = i - n * ldw;
-    Bw[i] = a < (size_t)N ? (T)(B[n * N + a] * sqrt(nbar[a])) : (T)0;
+    const size_t n = i / ldw;
+    const int p = (int)(i - n * ldw), a = serial ? nt_serial(p) : p;
+    Bw[i] = a < N ? (T)(B[n * N + a] * sqrt(nbar[a])) : (T)0;
 }
 
 // ---- Toeplitz projection of box surveys ---------------------------------------------
@@ -1055,11 +1069,11 @@ __global__ __launch_bounds__(256) void idft_kernel(const float* __restrict__ yha
 // B' in grid order: Bg[m][g] = B'[m][gmap[g]] (0 where the grid has no cell and in the padding).
 template <typename T>
 __global__ void grid_b_kernel(const double* __restrict__ Bw, size_t ldw, const int* __restrict__ gmap, int Ng, int M,
-                              T* __restrict__ Bg, size_t ldg) {
+                              bool serial, T* __restrict__ Bg, size_t ldg) {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= (size_t)M * ldg) return;
-    const size_t m = i / ldg, g = i - m * ldg;
-    const int a = g < (size_t)Ng ? gmap[g] : -1;
+    const size_t m = i / ldg;
+    const int p = (int)(i - m * ldg), g = serial ? nt_serial(p) : p, a = g < Ng ? gmap[g] : -1;
     Bg[i] = a >= 0 ? (T)Bw[m * ldw + a] : (T)0;
 }
 
@@ -1071,10 +1085,10 @@ constexpr int TOEP_MAXX = 64;
 template <typename T>
 __global__ __launch_bounds__(256) void bhat64_kernel(const double* __restrict__ Bw, size_t ldw,
                                                      const int* __restrict__ gmap, int n1, int G, int M,
-                                                     const double* __restrict__ trig, T* __restrict__ Bhat, size_t Gp,
-                                                     int nbat) {
-    const int m = blockIdx.y, r = blockIdx.x * 256 + threadIdx.x;
-    if (r >= (int)Gp) return;
+                                                     const double* __restrict__ trig, bool serial,
+                                                     T* __restrict__ Bhat, size_t Gp, int nbat) {
+    const int m = blockIdx.y, p = blockIdx.x * 256 + threadIdx.x, r = serial ? nt_serial(p) : p;
+    if (p >= (int)Gp) return;
     const int L = 2 * n1;
     double v[TOEP_MAXX];
 #pragma unroll
@@ -1090,7 +1104,7 @@ __global__ __launch_bounds__(256) void bhat64_kernel(const double* __restrict__ 
 #pragma unroll
         for (int x = 0; x < TOEP_MAXX; x++)
             if (x < n1) acc += t[(x * k) % L] * v[x];
-        Bhat[((size_t)b * M + m) * Gp + r] = (T)(imag ? -acc : acc);
+        Bhat[((size_t)b * M + m) * Gp + p] = (T)(imag ? -acc : acc);
     }
 }
 
@@ -1112,8 +1126,8 @@ __global__ __launch_bounds__(256) void that_rows_kernel(const double* __restrict
 // are loaded together.
 template <typename T, int NMAX>
 __global__ __launch_bounds__(256) void idft64_kernel(const T* __restrict__ Yhat, int nbat, int G, size_t Gp, int n1,
-                                                     int M, const double* __restrict__ W, T* __restrict__ Y, size_t ldg,
-                                                     int Kg) {
+                                                     int M, const double* __restrict__ W, bool serial,
+                                                     T* __restrict__ Y, size_t ldg, int Kg) {
     extern __shared__ double id64_w[];   // nbat x n1
     const int m = blockIdx.y, r = blockIdx.x * 256 + threadIdx.x;
     Yhat += (size_t)blockIdx.z * nbat * M * Gp;
@@ -1121,7 +1135,7 @@ __global__ __launch_bounds__(256) void idft64_kernel(const T* __restrict__ Yhat,
     for (int i = threadIdx.x; i < nbat * n1; i += 256) id64_w[i] = W[i];
     __syncthreads();
     if (blockIdx.x == 0)
-        for (int g = n1 * G + threadIdx.x; g < Kg; g += 256) Y[g] = (T)0;
+        for (int g = n1 * G + threadIdx.x; g < Kg; g += 256) Y[serial ? nt_serial(g) : g] = (T)0;
     if (r >= G) return;
     double acc[NMAX];
 #pragma unroll
@@ -1141,7 +1155,10 @@ __global__ __launch_bounds__(256) void idft64_kernel(const T* __restrict__ Yhat,
     }
 #pragma unroll
     for (int x = 0; x < NMAX; x++)
-        if (x < n1) Y[(size_t)x * G + r] = (T)acc[x];
+        if (x < n1) {
+            const int g = x * G + r;
+            Y[serial ? nt_serial(g) : g] = (T)acc[x];
+        }
 }
 
 // ---- Toeplitz projection of spherical shells (DFT along phi) -----------------------
@@ -1166,7 +1183,8 @@ __global__ __launch_bounds__(256) void idft64_kernel(const T* __restrict__ Yhat,
 // wave-uniform LDS rows.  NMAX >= Nphi bounds the registers; CB = 128 for NMAX = 64 keeps
 // the block's LDS under 100 KB.  T void: hi / lo BF16 planes
 // [k][Gr][Gp], zero outside G x G (the grid covers Gr x Gp); else out[k][h - row0][c]
-// for the grid's rows h = row0 + blockIdx.y, Gr of them, zero for G <= c < Gp.
+// for the grid's rows h = row0 + blockIdx.y, Gr of them, zero for G <= c < Gp (FP32: in
+// the serial order).
 template <typename T, int NMAX>
 __global__ __launch_bounds__(256) void that_sph_kernel(const double* __restrict__ Q, int G, int nph,
                                                        const double* __restrict__ trig, __bf16* __restrict__ hi,
@@ -1214,7 +1232,7 @@ __global__ __launch_bounds__(256) void that_sph_kernel(const double* __restrict_
         for (int d = 0; d < NMAX; d++)
             if (d < nph) acc += Ck[d] * q[d];
         if ((size_t)c >= Gp) continue;
-        const size_t o = ((size_t)k * Gr + blockIdx.y) * Gp + c;
+        const size_t o = ((size_t)k * Gr + blockIdx.y) * Gp + (std::is_same<T, float>::value ? nt_serial(c) : c);
         if constexpr (std::is_same<T, void>::value) {
             __bf16 x, y;
             split2((float)acc, x, y);
@@ -1689,8 +1707,8 @@ static int panel_rows(int rows, size_t row_bytes) {
 // are contiguous in the output.
 template <typename T>
 static int stage2_nt(opsec_ctx* ctx, NtWork& ws, const T* X, size_t ld, const T* C, size_t cstride, int g, int M, int K,
-                     double* P) {
-    NtArgs<T> A{C, ld, 0, cstride, M, X, ld, 0, 0, M, (int)(nt_kpad<T>(K) / nt_bk<T>()), 1, g};
+                     bool serial, double* P) {
+    NtArgs<T> A{C, ld, 0, cstride, M, X, ld, 0, 0, M, (int)(nt_kpad<T>(K) / nt_bk<T>()), 1, g, serial};
     return launch_nt_gemm<T>(ctx, ws, A, NtPacked{P, (size_t)packed_size(M)});
 }
 
@@ -1711,6 +1729,7 @@ static int run_project_toeplitz_nt(opsec_ctx* ctx, int nb, const int* funcs, int
     if ((rc = toep_check(ctx, tgrid))) return rc;
     if (!tgrid.sph && (sv.n2 >= 65536 || sv.n3 >= 65536))
         return set_error(ctx, OPSEC_EINVAL, "Toeplitz projection: Ny, Nz < 65536");
+    const bool serial = serial_sums<T>(sv);
     const size_t Gp = nt_pitch<T>(G), ldg = nt_pitch<T>(Ng);
     const int Kg = (int)nt_kpad<T>(Ng);
     const int grp = std::min(nb, TOEP64_GROUP);
@@ -1749,9 +1768,10 @@ static int run_project_toeplitz_nt(opsec_ctx* ctx, int nb, const int* funcs, int
         OPSEC_HIP_TRY(ctx, stream_copy(ctx, ps->d_trig64, trig.data(), trig.size() * 8, hipMemcpyHostToDevice));
         OPSEC_HIP_TRY(ctx, stream_copy(ctx, ps->d_W64, W.data(), W.size() * 8, hipMemcpyHostToDevice));
         hipLaunchKernelGGL(grid_b_kernel<T>, blocks_for(ystride), dim3(256), 0, ctx->stream, ps->d_Bw, ps->ldw,
-                           ps->d_gmap64, Ng, M, (T*)tp.Bg, ldg);
+                           ps->d_gmap64, Ng, M, serial, (T*)tp.Bg, ldg);
         hipLaunchKernelGGL(bhat64_kernel<T>, dim3((unsigned)((Gp + 255) / 256), (unsigned)M), dim3(256), 0, ctx->stream,
-                           ps->d_Bw, ps->ldw, ps->d_gmap64, n1, G, M, ps->d_trig64, (T*)tp.Bhat, Gp, nbat);
+                           ps->d_Bw, ps->ldw, ps->d_gmap64, n1, G, M, ps->d_trig64, serial, (T*)tp.Bhat, Gp,
+                           nbat);
         OPSEC_HIP_TRY(ctx, hipGetLastError());
         tp.valid = true;
     }
@@ -1790,17 +1810,17 @@ static int run_project_toeplitz_nt(opsec_ctx* ctx, int nb, const int* funcs, int
                 if (r0 == 0) hipEventRecord(ev[3 * si + 1], ctx->stream);
                 // batch b of band q: Yhat[b] (M x G) = Bhat[b] That_((b+1)/2), columns r0 .. r0 + nr - 1
                 NtArgs<T> A{(const T*)tp.Bhat, Gp, (size_t)M * Gp, 0, M, Tp, Gp, (size_t)nr * Gp, tz, nr,
-                            (int)(nt_kpad<T>(G) / nt_bk<T>()), nbat, nbat * ns};
+                            (int)(nt_kpad<T>(G) / nt_bk<T>()), nbat, nbat * ns, serial};
                 if (!rc) rc = launch_nt_gemm<T>(ctx, ps->ws, A, NtRows<T>{(T*)tp.Yhat + r0, Gp, (size_t)M * Gp, hstride, nr});
             }
             hipLaunchKernelGGL(idft, dim3((unsigned)((G + 255) / 256), (unsigned)M, (unsigned)ns), dim3(256), id_lds,
-                               ctx->stream, (const T*)tp.Yhat, nbat, G, Gp, n1, M, ps->d_W64,
+                               ctx->stream, (const T*)tp.Yhat, nbat, G, Gp, n1, M, ps->d_W64, serial,
                                (T*)tp.Y + (size_t)q0 * ystride, ldg, Kg);
             hipEventRecord(ev[3 * si + 2], ctx->stream);
         }
         hipEventRecord(evg[2 * gi], ctx->stream);
         if (!rc)
-            rc = stage2_nt<T>(ctx, ps->ws, (const T*)tp.Bg, ldg, (const T*)tp.Y, ystride, g, M, Ng,
+            rc = stage2_nt<T>(ctx, ps->ws, (const T*)tp.Bg, ldg, (const T*)tp.Y, ystride, g, M, Ng, serial,
                               (double*)ps->d_P + (size_t)z0 * np);
         hipEventRecord(evg[2 * gi + 1], ctx->stream);
     }
@@ -1850,6 +1870,7 @@ template <typename T>
 static int run_project_dense_nt(opsec_ctx* ctx, int nb, const int* d_funcs, const T* Bw, size_t ldw, int prec) {
     ProjState* ps = ctx->proj;
     const int N = ctx->ncells, M = ctx->nmodes;
+    const bool serial = serial_sums<T>(ctx->sv);
     const size_t per_band = ldw * M;   // stage-1 products use the same padded pitch as B'
     const int grp = (int)std::max<size_t>(1, std::min<size_t>(nb, DENSE_GROUP_BYTES / (per_band * sizeof(T))));
     const int Kp = (int)nt_kpad<T>(N), rows = panel_rows(N, ldw * sizeof(T));
@@ -1873,19 +1894,20 @@ static int run_project_dense_nt(opsec_ctx* ctx, int nb, const int* d_funcs, cons
                 const int nr = std::min(rows, N - r0);
                 hipLaunchKernelGGL(gen_rows_kernel<T>, dim3((unsigned)((Kp + 511) / 512), (unsigned)((nr + 7) / 8), ns),
                                    dim3(256), 0, ctx->stream, ctx->d_Q, (size_t)ctx->nkeys, d_funcs + z0 + q0,
-                                   ctx->d_cellidx, pair_key_of(ctx->sv), N, r0, nr, Kp, Tp, ldw, tband);
-                NtArgs<T> A{Bw, ldw, 0, 0, M, Tp, ldw, 0, tband, nr, Kp / nt_bk<T>(), 1, ns};
+                                   ctx->d_cellidx, pair_key_of(ctx->sv), N, r0, nr, Kp, serial, Tp, ldw,
+                                   tband);
+                NtArgs<T> A{Bw, ldw, 0, 0, M, Tp, ldw, 0, tband, nr, Kp / nt_bk<T>(), 1, ns, serial};
                 // the last panel's tiles also write the padding columns of C (from clamped rows: finite,
                 // and they meet the zero padding of B' in stage 2)
                 if (!rc)
                     rc = launch_nt_gemm<T>(ctx, ps->ws, A,
                                            NtRows<T>{(T*)ps->d_C + (size_t)q0 * per_band + r0, ldw, 0, per_band,
-                                                     r0 + nr < N ? nr : Kp - r0});
+                                                     r0 + nr < N ? nr : Kp - r0, serial});
             }
         }
         hipEventRecord(ev[2 * gi + 1], ctx->stream);
         if (!rc)
-            rc = stage2_nt<T>(ctx, ps->ws, Bw, ldw, (const T*)ps->d_C, per_band, g, M, N,
+            rc = stage2_nt<T>(ctx, ps->ws, Bw, ldw, (const T*)ps->d_C, per_band, g, M, N, serial,
                               (double*)ps->d_P + (size_t)z0 * np);
         hipEventRecord(ev[2 * gi + 2], ctx->stream);
     }
@@ -1926,7 +1948,8 @@ static int run_project(opsec_ctx* ctx, int nb, const int* d_funcs, const int* fu
         int rc;
         if ((rc = dev_realloc(ctx, (void**)&ps->d_Bw32, &ps->cap_Bw32, ld32 * ctx->nmodes * 4))) return rc;
         hipLaunchKernelGGL(scale_rows_kernel<float>, blocks_for(ld32 * ctx->nmodes), dim3(256), 0, ctx->stream,
-                           ctx->d_B, ctx->d_nbar, ctx->ncells, ctx->nmodes, ps->d_Bw32, ld32);
+                           ctx->d_B, ctx->d_nbar, ctx->ncells, ctx->nmodes, serial_sums<float>(ctx->sv), ps->d_Bw32,
+                           ld32);
         OPSEC_HIP_TRY(ctx, hipGetLastError());
         ps->bw32_valid = true;
     }
@@ -1938,6 +1961,7 @@ template <typename T>
 static int project_host_nt(opsec_ctx* ctx, int N, const double* dS, int M, const double* dB, double* dP) {
     const size_t ld = nt_pitch<T>(N);
     const int Kp = (int)nt_kpad<T>(N);
+    const bool serial = std::is_same<T, float>::value;
     struct Work : NtWork {
         ~Work() { dev_free(&p); }
     } ws;
@@ -1946,13 +1970,15 @@ static int project_host_nt(opsec_ctx* ctx, int N, const double* dS, int M, const
     OPSEC_HIP_TRY(ctx, tmp.alloc(&X, ld * N * sizeof(T)));
     OPSEC_HIP_TRY(ctx, tmp.alloc(&Bp, ld * M * sizeof(T)));
     OPSEC_HIP_TRY(ctx, tmp.alloc(&Cp, ld * M * sizeof(T)));
-    hipLaunchKernelGGL(pad_rows_kernel<T>, blocks_for(ld * N), dim3(256), 0, ctx->stream, dS, (size_t)N, N, N, X, ld);
-    hipLaunchKernelGGL(pad_rows_kernel<T>, blocks_for(ld * M), dim3(256), 0, ctx->stream, dB, (size_t)N, M, N, Bp, ld);
+    hipLaunchKernelGGL(pad_rows_kernel<T>, blocks_for(ld * N), dim3(256), 0, ctx->stream, dS, (size_t)N, N, N, serial, X,
+                       ld);
+    hipLaunchKernelGGL(pad_rows_kernel<T>, blocks_for(ld * M), dim3(256), 0, ctx->stream, dB, (size_t)N, M, N, serial, Bp,
+                       ld);
     // C[m][a] = sum_b S[a][b] B[m][b]
-    NtArgs<T> A1{Bp, ld, 0, 0, M, X, ld, 0, 0, N, Kp / nt_bk<T>(), 1, 1};
-    int rc = launch_nt_gemm<T>(ctx, ws, A1, NtRows<T>{Cp, ld, 0, 0, Kp});
+    NtArgs<T> A1{Bp, ld, 0, 0, M, X, ld, 0, 0, N, Kp / nt_bk<T>(), 1, 1, serial};
+    int rc = launch_nt_gemm<T>(ctx, ws, A1, NtRows<T>{Cp, ld, 0, 0, Kp, serial});
     // P[i][j] = sum_a B[i][a] C[j][a], i <= j
-    if (!rc) rc = stage2_nt<T>(ctx, ws, Bp, ld, Cp, 0, 1, M, N, dP);
+    if (!rc) rc = stage2_nt<T>(ctx, ws, Bp, ld, Cp, 0, 1, M, N, serial, dP);
     if (rc) return rc;
     OPSEC_HIP_TRY(ctx, hipGetLastError());
     OPSEC_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
@@ -2030,7 +2056,7 @@ int opsec_modes_upload(opsec_ctx* ctx, const double* B, int ncells, int nmodes) 
     if ((rc = dev_realloc(ctx, (void**)&ps->d_Bw, &ps->cap_Bw, ps->ldw * nmodes * 8))) return rc;
     OPSEC_HIP_TRY(ctx, stream_copy(ctx, ctx->d_B, B, bytes, hipMemcpyHostToDevice));
     hipLaunchKernelGGL(scale_rows_kernel<double>, blocks_for(ps->ldw * nmodes), dim3(256), 0, ctx->stream, ctx->d_B,
-                       ctx->d_nbar, ncells, nmodes, ps->d_Bw, ps->ldw);
+                       ctx->d_nbar, ncells, nmodes, false, ps->d_Bw, ps->ldw);
     OPSEC_HIP_TRY(ctx, hipGetLastError());
     OPSEC_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     ctx->nmodes = nmodes;

@@ -416,3 +416,85 @@ def test_estimate_bit_reproducible(ctx, prec):
         b = ctx.estimate(lam, D, y, prior, lib.OPSEC_MIX_IDENTITY, prec)
         for k in ("F", "q", "f"):
             assert np.array_equal(a[k], b[k]), k
+
+
+def _chain32(A, B):
+    """sum_k A[m][k] B[n][k] of FP32 rows, k by k, each step one fused multiply-add (the
+    80-bit sum of an exact product rounds once more than the hardware's, at its 64th bit)."""
+    acc = np.zeros((A.shape[0], B.shape[0]), dtype=np.float32)
+    A, B = A.astype(np.longdouble), B.astype(np.longdouble)
+    for k in range(A.shape[1]):
+        acc = (acc + A[:, k, None] * B[None, :, k]).astype(np.float32)
+    return acc
+
+
+def _packed_lower(C):
+    return np.concatenate([C[j, :j + 1] for j in range(len(C))]).astype(np.float64)
+
+
+# fewer k than one step, ragged, a K range that a split would cut (10 and 34 steps of 32)
+@pytest.mark.parametrize("n,m", [(5, 3), (45, 20), (130, 129), (315, 24)])
+def test_fp32_product_sums_in_k_order(ctx, n, m):
+    """The FP32 product of a given matrix is the chain of fused multiply-adds over k, to the bit."""
+    rng = np.random.default_rng(n)
+    S, B = rng.normal(size=(n, n)), rng.normal(size=(m, n))
+    b = B.astype(np.float32)
+    C = _chain32(b, S.astype(np.float32))
+    assert np.array_equal(ctx.project_dense(S, B, lib.OPSEC_PREC_FP32), _packed_lower(_chain32(C, b)))
+
+
+@pytest.mark.parametrize("dims,m,drop", [((3, 3, 5), 20, 0.0), ((9, 5, 7), 24, 0.0), ((17, 16, 4), 13, 0.0),
+                                         ((6, 7, 9), 30, 0.2), ((3, 2, 40), 17, 0.0)])
+def test_fp32_shell_sums_in_k_order(ctx, dims, m, drop):
+    """FP32 projections of a shell, dense and Toeplitz: FP32 operands, both products chains of
+    fused multiply-adds over k (the cells, the grid or the arcs, in order), FP64 DFTs rounded to
+    FP32, to the bit whatever the number of bands in the call."""
+    nr, nmu, nphi = dims
+    cells = synth.shell_cells(nr, nmu, nphi)
+    if drop:
+        cells = synth.drop_cells(cells, drop, seed=4)
+    N, G, L = len(cells), nr * nmu, 2 * nphi
+    blo, bhi = synth.linear_bands(3, 0.01, 0.1)
+    ctx.model_real(GOLD["pk_k"], GOLD["pk_P"], blo, bhi, lib.OPSEC_XI_CLOSED)
+    ctx.cells_upload(cells, lib.survey_sph(nr, nmu, nphi))
+    funcs = [1, 2, 3]
+    ctx.pair_tables(funcs, ctx.quad(lib.OPSEC_QUAD_GM))
+    B = np.random.default_rng(m).normal(size=(m, N))
+    ctx.modes_upload(B)
+    Bw = B * np.sqrt(cells["Nbar"])
+    b32 = Bw.astype(np.float32)
+    arc, phi = cells["d1"] * nmu + cells["d2"], cells["d3"]
+    dense, toep = [], []
+    grid = np.zeros((m, nphi, G))
+    grid[:, phi, arc] = Bw
+    x = np.arange(nphi)
+    for f in funcs:
+        Q = ctx.pair_table(f).reshape(G, G, nphi)
+        T = Q[arc[:, None], arc[None, :], np.abs(phi[:, None] - phi[None, :])].astype(np.float32)
+        dense.append(_packed_lower(_chain32(_chain32(b32, T), b32)))
+        Y = np.zeros((m, nphi, G))
+        for bat in range(2 * nphi):
+            k, imag = (bat + 1) // 2, bat > 0 and bat % 2 == 0
+            c, s = np.cos(2 * np.pi * ((x * k) % L) / L), np.sin(2 * np.pi * ((x * k) % L) / L)
+            That = Q @ np.where(x == 0, 1.0, 2 * c)
+            bh = np.einsum("x,mxg->mg", -s if imag else c, grid)
+            yh = _chain32(bh.astype(np.float32), That.astype(np.float32)).astype(np.float64)
+            ck = 1.0 if k in (0, nphi) else 2.0
+            Y += (ck / L) * (-s if imag else c)[None, :, None] * yh[:, None, :]
+        y32, g32 = Y.reshape(m, -1).astype(np.float32), grid.reshape(m, -1).astype(np.float32)
+        toep.append(_packed_lower(_chain32(y32, g32)))
+    got = ctx.project(funcs, lib.OPSEC_PREC_FP32)
+    one = np.concatenate([ctx.project([f], lib.OPSEC_PREC_FP32) for f in funcs])
+    assert np.array_equal(got, dense) and np.array_equal(one, dense)
+    try:
+        ctx.set_projection(lib.OPSEC_PROJ_TOEPLITZ)
+        got = ctx.project(funcs, lib.OPSEC_PREC_FP32)
+        one = np.concatenate([ctx.project([f], lib.OPSEC_PREC_FP32) for f in funcs])
+    finally:
+        ctx.set_projection(lib.OPSEC_PROJ_DENSE)
+    assert np.array_equal(one, got)
+    # the FP64 DFTs' own rounding (about 1e-15) moves an FP32 operand to its neighbour about
+    # once in 10^6; that mode's m of a band's m (m + 1) / 2 entries (at most 1 in 7 here) then differ
+    same = got == np.array(toep)
+    print("Toeplitz FP32", dims, same.size - same.sum(), "of", same.size, "entries differ")
+    assert same.mean() > 0.75
