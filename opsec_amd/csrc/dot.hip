@@ -136,14 +136,18 @@ __global__ void fold_bins_kernel(const uint32_t* __restrict__ key, const float* 
 // on its parity.  So an addition is a map (parity -> increment), such maps
 // compose associatively, and a block of FOLD_BLOCK weights is composed by all
 // threads at once; the sums within it only grow, so if the last is below 2^53
-// all were.  Where that fails (the sum leaves the binade, a weight is negative or
-// not finite, the sum is not positive and normal), the waves before the failing
+// all were.  Weights of 2^51 u and more are not composed: without them a block's
+// increments stay below 2048 x 2^51 = 2^62 and no sum of them wraps.  Where a
+// block fails (the sum leaves the binade, a weight is that large, negative or not
+// finite, the sum is not positive and normal), the waves before the failing
 // one are kept, that wave's weights are added one by one from LDS, and the next
 // block starts behind them.
 // Bound by the composition's latency per block: 5 x 10^5 galaxies of one bin take
 // 425 us, 9.8 ms by one thread (a dependent FP64 addition and its load each).
 constexpr int FOLD_THREADS = 512, FOLD_PER = 4, FOLD_BLOCK = FOLD_THREADS * FOLD_PER;
 constexpr int FOLD_WAVES = FOLD_THREADS / 64, FOLD_WAVE = 64 * FOLD_PER;
+constexpr double FOLD_STEP = 2251799813685248.0;   // 2^51
+static_assert(FOLD_BLOCK <= 2048, "a block's increments, at most 2^51 each, and k < 2^53 stay below 2^63");
 struct FoldMap {
     long long c0, c1;   // increment of an even, of an odd k
     // this addition (or block) first, then b
@@ -198,7 +202,7 @@ __global__ __launch_bounds__(FOLD_THREADS) void fold_long_kernel(const uint32_t*
 #pragma unroll
         for (int j = 0; j < FOLD_PER; j++) {
             const double q = ldexp((double)v[j], 52 - e);   // w / u, exact
-            ok = ok && q >= 0.0 && q < 9007199254740992.0;
+            ok = ok && q >= 0.0 && q < FOLD_STEP;
             const double r = rint(q), d = q - r;
             FoldMap g;
             g.c0 = g.c1 = (long long)(ok ? r : 0.0);

@@ -123,6 +123,36 @@ def test_counts_long_bins_bit_exact(ctx, ngal, kind):
     assert np.array_equal(_bits(got), _bits(ref)), (got[[0, 8]], ref[[0, 8]])
 
 
+UNDER2 = float(np.nextafter(np.float32(2.0), np.float32(0.0)))
+
+
+# running sums no larger than the weights that follow: a starting count, or a small or
+# zero first part, then a block (2048) of weights, one less, one more, and several
+@pytest.mark.parametrize("start,weights", [
+    (1.0, [(2046, 1.0)]), (1.0, [(2047, 1.0)]), (1.0, [(2048, 1.0)]), (1.0, [(6000, 1.0)]),
+    (1.5, [(2048, 1.0)]), (2.0, [(4097, 1.0)]), (1.0, [(2048, UNDER2)]), (1.0, [(4096, UNDER2)]),
+    (1.0, [(2048, 0.5)]), (1.0, [(2048, 0.25)]), (1.0, [(2048, 0.2499999)]), (3.0, [(5000, 1.9)]),
+    (0.0, [(255, 0.0), (2049, 1.0)]), (0.0, [(256, 0.002), (2048, 0.7)]), (0.0, [(255, 0.0), (1, 1.0), (5000, 1.25)]),
+    (0.0, [(1024, 1e-30), (3000, 1.0)]), (1e-300, [(256, 0.0), (2500, 1e-30)])])
+def test_counts_long_bins_large_weights(ctx, start, weights):
+    """A long bin whose weights are about as large as its running sum: the one-by-one sum's bits."""
+    cells = synth.box_cells(2, 0.0, 2.0)
+    ctx.cells_upload(cells, lib.survey_box(2, 0.0, 2.0))
+    w = np.concatenate([np.full(n, v, dtype=np.float32) for n, v in weights])
+    g = np.zeros(len(w), dtype=lib.GALAXY_DTYPE)
+    g["x1"], g["x2"], g["x3"], g["w"] = 0.5, 0.5, 0.5, w
+    ref = start
+    for v in w.astype(np.float64):
+        ref += v
+    counts = np.zeros(9)
+    counts[0] = start
+    got = ctx.count_galaxies(g, counts=counts.copy())
+    assert _bits(got[:1]) == _bits([ref]) and np.all(got[1:] == 0)
+    # the same catalogue in pieces: its first galaxy, then the rest
+    got = ctx.count_galaxies(g[1:], ctx.count_galaxies(g[:1], counts.copy()))
+    assert _bits(got[:1]) == _bits([ref]) and np.all(got[1:] == 0)
+
+
 @pytest.mark.parametrize("n,M,ngal", [(6, 40, 30000), (32, 2000, 2000000)])
 def test_pixel_values_vs_oracle(ctx, n, M, ngal):
     """x bit-exact (IEEE subtract, sqrt and divide); y = B^T x within 1e-13 of
