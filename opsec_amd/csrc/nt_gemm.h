@@ -2,7 +2,8 @@
 //
 // Both operands are rows of T with 16-byte aligned pitches, and K is a whole
 // number of 128-byte steps (nt_kpad); the columns between the real extent and
-// the padded one must be zero in one operand and finite in the other.  Rows
+// the padded one are zero in both operands, so that an infinity or NaN in a row
+// reaches only what its own products reach.  Rows
 // beyond an operand's extent are clamped to its last row and their products
 // dropped in the epilogue, so any M and N are taken.
 #pragma once
@@ -84,14 +85,14 @@ struct NtArgs {
 
 // Epilogues: base(band, b), then put(base, m, n, M, value).
 template <typename T>
-struct NtRows {              // C[m * ld + n], n < nw (padding columns included), serial: in that order
+struct NtRows {              // C[m * ld + n], n < nc, then zeros up to nw; serial: in that order
     T* p;
     size_t ld, b_stride, q_stride;
-    int nw;
+    int nc, nw;
     bool serial = false;
     __device__ __forceinline__ T* base(int q, int b) const { return p + q * q_stride + b * b_stride; }
     __device__ __forceinline__ void put(T* o, int m, int n, int M, T v) const {
-        if (m < M && n < nw) o[(size_t)m * ld + (serial ? nt_serial(n) : n)] = v;
+        if (m < M && n < nw) o[(size_t)m * ld + (serial ? nt_serial(n) : n)] = n < nc ? v : (T)0;
     }
     static constexpr bool lower = false;
 };

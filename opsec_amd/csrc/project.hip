@@ -1811,7 +1811,7 @@ static int run_project_toeplitz_nt(opsec_ctx* ctx, int nb, const int* funcs, int
                 // batch b of band q: Yhat[b] (M x G) = Bhat[b] That_((b+1)/2), columns r0 .. r0 + nr - 1
                 NtArgs<T> A{(const T*)tp.Bhat, Gp, (size_t)M * Gp, 0, M, Tp, Gp, (size_t)nr * Gp, tz, nr,
                             (int)(nt_kpad<T>(G) / nt_bk<T>()), nbat, nbat * ns, serial};
-                if (!rc) rc = launch_nt_gemm<T>(ctx, ps->ws, A, NtRows<T>{(T*)tp.Yhat + r0, Gp, (size_t)M * Gp, hstride, nr});
+                if (!rc) rc = launch_nt_gemm<T>(ctx, ps->ws, A, NtRows<T>{(T*)tp.Yhat + r0, Gp, (size_t)M * Gp, hstride, nr, nr});
             }
             hipLaunchKernelGGL(idft, dim3((unsigned)((G + 255) / 256), (unsigned)M, (unsigned)ns), dim3(256), id_lds,
                                ctx->stream, (const T*)tp.Yhat, nbat, G, Gp, n1, M, ps->d_W64, serial,
@@ -1897,11 +1897,10 @@ static int run_project_dense_nt(opsec_ctx* ctx, int nb, const int* d_funcs, cons
                                    ctx->d_cellidx, pair_key_of(ctx->sv), N, r0, nr, Kp, serial, Tp, ldw,
                                    tband);
                 NtArgs<T> A{Bw, ldw, 0, 0, M, Tp, ldw, 0, tband, nr, Kp / nt_bk<T>(), 1, ns, serial};
-                // the last panel's tiles also write the padding columns of C (from clamped rows: finite,
-                // and they meet the zero padding of B' in stage 2)
+                // the last panel's tiles also write the padding columns of C
                 if (!rc)
                     rc = launch_nt_gemm<T>(ctx, ps->ws, A,
-                                           NtRows<T>{(T*)ps->d_C + (size_t)q0 * per_band + r0, ldw, 0, per_band,
+                                           NtRows<T>{(T*)ps->d_C + (size_t)q0 * per_band + r0, ldw, 0, per_band, nr,
                                                      r0 + nr < N ? nr : Kp - r0, serial});
             }
         }
@@ -1976,7 +1975,7 @@ static int project_host_nt(opsec_ctx* ctx, int N, const double* dS, int M, const
                        ld);
     // C[m][a] = sum_b S[a][b] B[m][b]
     NtArgs<T> A1{Bp, ld, 0, 0, M, X, ld, 0, 0, N, Kp / nt_bk<T>(), 1, 1, serial};
-    int rc = launch_nt_gemm<T>(ctx, ws, A1, NtRows<T>{Cp, ld, 0, 0, Kp, serial});
+    int rc = launch_nt_gemm<T>(ctx, ws, A1, NtRows<T>{Cp, ld, 0, 0, N, Kp, serial});
     // P[i][j] = sum_a B[i][a] C[j][a], i <= j
     if (!rc) rc = stage2_nt<T>(ctx, ws, Bp, ld, Cp, 0, 1, M, N, serial, dP);
     if (rc) return rc;

@@ -498,3 +498,43 @@ def test_fp32_shell_sums_in_k_order(ctx, dims, m, drop):
     same = got == np.array(toep)
     print("Toeplitz FP32", dims, same.size - same.sum(), "of", same.size, "entries differ")
     assert same.mean() > 0.75
+
+
+@pytest.mark.parametrize("n", [1, 17, 45, 128])
+@pytest.mark.parametrize("prec", [lib.OPSEC_PREC_FP64, lib.OPSEC_PREC_FP32])
+def test_project_dense_infinite_entry(ctx, n, prec):
+    """An infinite entry of S in its last row and column: every entry of P is the infinity of
+    its own products' sign, as the plain product has it, and no NaN comes from padding."""
+    rng = np.random.default_rng(n)
+    S, B = np.abs(rand_sym(n, n)), rng.normal(size=(min(n, 5), n))
+    S[-1, -1] = np.inf
+    got = ctx.project_dense(S, B, prec)
+    want = _packed_lower(np.outer(np.sign(B[:, -1]), np.sign(B[:, -1])) * np.inf)
+    assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("proj", [lib.OPSEC_PROJ_DENSE, lib.OPSEC_PROJ_TOEPLITZ])
+@pytest.mark.parametrize("prec", [lib.OPSEC_PREC_FP64, lib.OPSEC_PREC_FP32])
+def test_project_infinite_mode_entry(ctx, prec, proj):
+    """An infinite entry in one mode (27 cells, positive xi): that mode's entries are infinite
+    (the dense product; a DFT along x mixes signs and may leave NaN), all others as without it."""
+    cells = synth.box_cells(3, 0.0, 60.0)
+    ctx.model_test(0, 1.0, 0.02)
+    ctx.cells_upload(cells, lib.survey_box(3, 0.0, 60.0, L=1e9))
+    ctx.pair_tables([0], ctx.quad(lib.OPSEC_QUAD_GAUSS, nodes=4, near=1))
+    B = np.random.default_rng(2).uniform(0.1, 1.0, size=(6, 27))
+    try:
+        ctx.set_projection(proj)
+        ctx.modes_upload(B)
+        ref = ctx.project([0], prec)[0]
+        B[4, 26] = np.inf
+        ctx.modes_upload(B)
+        got = ctx.project([0], prec)[0]
+    finally:
+        ctx.set_projection(lib.OPSEC_PROJ_DENSE)
+    hit = np.array([4 in (i, j) for j in range(6) for i in range(j + 1)])
+    assert np.array_equal(got[~hit], ref[~hit])
+    if proj == lib.OPSEC_PROJ_DENSE:
+        assert np.all(got[hit] == np.inf)
+    else:
+        assert not np.isfinite(got[hit]).any()
