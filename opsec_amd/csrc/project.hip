@@ -167,11 +167,12 @@ __global__ __launch_bounds__(256) void gen_rows_kernel(const double* __restrict_
 template <typename T>
 __global__ void pad_rows_kernel(const double* __restrict__ X, size_t ldx, int rows, int cols, bool serial,
                                 T* __restrict__ out, size_t ld) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)rows * ld) return;
-    const size_t r = i / ld;
-    const int p = (int)(i - r * ld), c = serial ? nt_serial(p) : p;
-    out[i] = c < cols ? (T)X[r * ldx + c] : (T)0;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < (size_t)rows * ld;
+         i += (size_t)gridDim.x * blockDim.x) {
+        const size_t r = i / ld;
+        const int p = (int)(i - r * ld), c = serial ? nt_serial(p) : p;
+        out[i] = c < cols ? (T)X[r * ldx + c] : (T)0;
+    }
 }
 
 // ---- split-BF16x3 on pre-split planes --------------------------------------------
@@ -827,11 +828,11 @@ __global__ void sum_parts_kernel(const float* __restrict__ part, int nparts, siz
 // B' = diag(w) B with w = sqrt(Nbar), rows padded with zeros to ldw.
 template <typename T>
 __global__ void scale_rows_kernel(const double* B, const double* nbar, int N, int M, bool serial, T* Bw, size_t ldw) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= ldw * M) return;
-    const size_t n = i / ldw;
-    const int p = (int)(i - n * ldw), a = serial ? nt_serial(p) : p;
-    Bw[i] = a < N ? (T)(B[n * N + a] * sqrt(nbar[a])) : (T)0;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < ldw * M; i += (size_t)gridDim.x * blockDim.x) {
+        const size_t n = i / ldw;
+        const int p = (int)(i - n * ldw), a = serial ? nt_serial(p) : p;
+        Bw[i] = a < N ? (T)(B[n * N + a] * sqrt(nbar[a])) : (T)0;
+    }
 }
 
 // ---- Toeplitz projection of box surveys ---------------------------------------------
@@ -1070,11 +1071,12 @@ __global__ __launch_bounds__(256) void idft_kernel(const float* __restrict__ yha
 template <typename T>
 __global__ void grid_b_kernel(const double* __restrict__ Bw, size_t ldw, const int* __restrict__ gmap, int Ng, int M,
                               bool serial, T* __restrict__ Bg, size_t ldg) {
-    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (size_t)M * ldg) return;
-    const size_t m = i / ldg;
-    const int p = (int)(i - m * ldg), g = serial ? nt_serial(p) : p, a = g < Ng ? gmap[g] : -1;
-    Bg[i] = a >= 0 ? (T)Bw[m * ldw + a] : (T)0;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < (size_t)M * ldg;
+         i += (size_t)gridDim.x * blockDim.x) {
+        const size_t m = i / ldg;
+        const int p = (int)(i - m * ldg), g = serial ? nt_serial(p) : p, a = g < Ng ? gmap[g] : -1;
+        Bg[i] = a >= 0 ? (T)Bw[m * ldw + a] : (T)0;
+    }
 }
 
 // Bhat[b][m][r] = sum_x cos(2 pi x k / L) B'_x[m][r] (b = 0 or odd) or
@@ -1272,6 +1274,9 @@ static void launch_that_sph(opsec_ctx* ctx, const double* Q, int G, int nph, con
 // ---- host --------------------------------------------------------------------------
 
 static dim3 blocks_for(size_t threads) { return dim3((unsigned)((threads + 255) / 256)); }
+// Blocks of a kernel that strides over n elements: a launch takes fewer than 2^32 threads,
+// and 65536 rows of 65536 columns with their padding are more.
+static dim3 strided_blocks(size_t n) { return blocks_for(std::min<size_t>(n, (size_t)1 << 30)); }
 
 // Split a row-major double matrix (rows x cols, ldx) into a plane pair of
 // rows_p x ld.
@@ -1767,7 +1772,7 @@ static int run_project_toeplitz_nt(opsec_ctx* ctx, int nb, const int* funcs, int
         OPSEC_HIP_TRY(ctx, stream_copy(ctx, ps->d_gmap64, gmap.data(), gmap.size() * 4, hipMemcpyHostToDevice));
         OPSEC_HIP_TRY(ctx, stream_copy(ctx, ps->d_trig64, trig.data(), trig.size() * 8, hipMemcpyHostToDevice));
         OPSEC_HIP_TRY(ctx, stream_copy(ctx, ps->d_W64, W.data(), W.size() * 8, hipMemcpyHostToDevice));
-        hipLaunchKernelGGL(grid_b_kernel<T>, blocks_for(ystride), dim3(256), 0, ctx->stream, ps->d_Bw, ps->ldw,
+        hipLaunchKernelGGL(grid_b_kernel<T>, strided_blocks(ystride), dim3(256), 0, ctx->stream, ps->d_Bw, ps->ldw,
                            ps->d_gmap64, Ng, M, serial, (T*)tp.Bg, ldg);
         hipLaunchKernelGGL(bhat64_kernel<T>, dim3((unsigned)((Gp + 255) / 256), (unsigned)M), dim3(256), 0, ctx->stream,
                            ps->d_Bw, ps->ldw, ps->d_gmap64, n1, G, M, ps->d_trig64, serial, (T*)tp.Bhat, Gp,
@@ -1946,7 +1951,7 @@ static int run_project(opsec_ctx* ctx, int nb, const int* d_funcs, const int* fu
     if (!ps->bw32_valid) {
         int rc;
         if ((rc = dev_realloc(ctx, (void**)&ps->d_Bw32, &ps->cap_Bw32, ld32 * ctx->nmodes * 4))) return rc;
-        hipLaunchKernelGGL(scale_rows_kernel<float>, blocks_for(ld32 * ctx->nmodes), dim3(256), 0, ctx->stream,
+        hipLaunchKernelGGL(scale_rows_kernel<float>, strided_blocks(ld32 * ctx->nmodes), dim3(256), 0, ctx->stream,
                            ctx->d_B, ctx->d_nbar, ctx->ncells, ctx->nmodes, serial_sums<float>(ctx->sv), ps->d_Bw32,
                            ld32);
         OPSEC_HIP_TRY(ctx, hipGetLastError());
@@ -1969,9 +1974,9 @@ static int project_host_nt(opsec_ctx* ctx, int N, const double* dS, int M, const
     OPSEC_HIP_TRY(ctx, tmp.alloc(&X, ld * N * sizeof(T)));
     OPSEC_HIP_TRY(ctx, tmp.alloc(&Bp, ld * M * sizeof(T)));
     OPSEC_HIP_TRY(ctx, tmp.alloc(&Cp, ld * M * sizeof(T)));
-    hipLaunchKernelGGL(pad_rows_kernel<T>, blocks_for(ld * N), dim3(256), 0, ctx->stream, dS, (size_t)N, N, N, serial, X,
+    hipLaunchKernelGGL(pad_rows_kernel<T>, strided_blocks(ld * N), dim3(256), 0, ctx->stream, dS, (size_t)N, N, N, serial, X,
                        ld);
-    hipLaunchKernelGGL(pad_rows_kernel<T>, blocks_for(ld * M), dim3(256), 0, ctx->stream, dB, (size_t)N, M, N, serial, Bp,
+    hipLaunchKernelGGL(pad_rows_kernel<T>, strided_blocks(ld * M), dim3(256), 0, ctx->stream, dB, (size_t)N, M, N, serial, Bp,
                        ld);
     // C[m][a] = sum_b S[a][b] B[m][b]
     NtArgs<T> A1{Bp, ld, 0, 0, M, X, ld, 0, 0, N, Kp / nt_bk<T>(), 1, 1, serial};
@@ -2054,7 +2059,7 @@ int opsec_modes_upload(opsec_ctx* ctx, const double* B, int ncells, int nmodes) 
     ps->ldw = nt_pitch<double>(ncells);
     if ((rc = dev_realloc(ctx, (void**)&ps->d_Bw, &ps->cap_Bw, ps->ldw * nmodes * 8))) return rc;
     OPSEC_HIP_TRY(ctx, stream_copy(ctx, ctx->d_B, B, bytes, hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(scale_rows_kernel<double>, blocks_for(ps->ldw * nmodes), dim3(256), 0, ctx->stream, ctx->d_B,
+    hipLaunchKernelGGL(scale_rows_kernel<double>, strided_blocks(ps->ldw * nmodes), dim3(256), 0, ctx->stream, ctx->d_B,
                        ctx->d_nbar, ncells, nmodes, false, ps->d_Bw, ps->ldw);
     OPSEC_HIP_TRY(ctx, hipGetLastError());
     OPSEC_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));

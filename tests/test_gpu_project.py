@@ -538,3 +538,16 @@ def test_project_infinite_mode_entry(ctx, prec, proj):
         assert np.all(got[hit] == np.inf)
     else:
         assert not np.isfinite(got[hit]).any()
+
+
+@pytest.mark.parametrize("prec", [lib.OPSEC_PREC_FP64, lib.OPSEC_PREC_FP32])
+def test_project_dense_more_elements_than_threads(ctx, prec):
+    """65536 cells: a padded copy of S has more elements than a launch has threads."""
+    n = 65536
+    S = np.zeros((n, n))   # untouched pages
+    B = np.random.default_rng(1).integers(-3, 4, size=(3, n)).astype(np.float64)
+    S[0, 0], S[40000, 123], S[n - 1, n - 1], S[n - 1, 7] = 2.0, 3.0, 5.0, 1.0
+    got = ctx.project_dense(S, B, prec)
+    P = (2 * np.outer(B[:, 0], B[:, 0]) + 3 * np.outer(B[:, 40000], B[:, 123]) + 5 * np.outer(B[:, -1], B[:, -1]) +
+         np.outer(B[:, -1], B[:, 7]))
+    assert np.array_equal(got, _packed(P))
