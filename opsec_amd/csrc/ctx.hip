@@ -16,6 +16,7 @@
 #include <thread>
 
 #include "common.h"
+#include "stage.h"
 #include "xi_dev.h"
 
 namespace opsec {
@@ -327,22 +328,21 @@ static int upload_desc(opsec_ctx* ctx) {
 // eight threads each move chunks through a pinned buffer of their own, the transfers
 // queued on the context's stream: 6.6 ms (41 GB/s), of which 0.25 ms at any size is the
 // start of the threads, hence the least sizes in common.h.  Memory that is pinned
-// already goes directly.  The buffers (32 MB) belong to the context and go with it; the
-// threads live for the call.
-struct HostStage {
-    static constexpr int N = 8;
-    static constexpr size_t BYTES = (size_t)4 << 20;
-    void* buf[N] = {};
-    hipEvent_t ev[N] = {};
-    int n = 0;   // slots made
+// already goes directly, and so does a copy whose slots cannot be made.  The slots (32 MB)
+// belong to the context and go with it; the threads live for the call.
+struct HipStageApi {
+    typedef hipEvent_t event_t;
+    static bool host_alloc(void** p, size_t n) { return hipHostMalloc(p, n, 0) == hipSuccess; }
+    static void host_free(void* p) { (void)hipHostFree(p); }
+    static bool event_create(event_t* e) { return hipEventCreateWithFlags(e, hipEventDisableTiming) == hipSuccess; }
+    static void event_destroy(event_t e) { (void)hipEventDestroy(e); }
+    static void clear_error() { (void)hipGetLastError(); }
 };
+struct HostStage : StageSlots<HipStageApi> {};
 
 void free_stage(opsec_ctx* ctx) {
     if (!ctx->stage) return;
-    for (int i = 0; i < ctx->stage->n; i++) {
-        (void)hipHostFree(ctx->stage->buf[i]);
-        (void)hipEventDestroy(ctx->stage->ev[i]);
-    }
+    ctx->stage->release();
     delete ctx->stage;
     ctx->stage = nullptr;
 }
@@ -355,6 +355,8 @@ static hipError_t plain_copy(opsec_ctx* ctx, void* dst, const void* src, size_t 
 
 hipError_t host_copy(opsec_ctx* ctx, void* dst, const void* src, size_t bytes, hipMemcpyKind kind) {
     const bool up = kind == hipMemcpyHostToDevice;
+    // an error that the caller has still to look at is not ours to clear
+    if (hipPeekAtLastError() != hipSuccess) return plain_copy(ctx, dst, src, bytes, kind);
     hipPointerAttribute_t at;
     if (hipPointerGetAttributes(&at, up ? src : dst) == hipSuccess) {
         if (at.type == hipMemoryTypeHost || at.type == hipMemoryTypeManaged || at.type == hipMemoryTypeDevice)
@@ -367,25 +369,13 @@ hipError_t host_copy(opsec_ctx* ctx, void* dst, const void* src, size_t bytes, h
     // chunks of 512 KB .. 4 MB, about two per thread
     const size_t chunk = std::min(HostStage::BYTES, std::max<size_t>((size_t)512 << 10, (bytes / 16 + 65535) & ~(size_t)65535));
     const size_t nchunks = (bytes + chunk - 1) / chunk;
-    const int want = (int)std::min<size_t>(HostStage::N, nchunks);
     // one copy at a time has the buffers; a second thread's goes through the runtime
     std::unique_lock<std::mutex> lock(ctx->stage_m, std::try_to_lock);
     if (!lock.owns_lock()) return plain_copy(ctx, dst, src, bytes, kind);
     if (!ctx->stage) ctx->stage = new (std::nothrow) HostStage;
     HostStage* S = ctx->stage;
-    while (S && S->n < want) {
-        if (hipHostMalloc(&S->buf[S->n], HostStage::BYTES, 0) != hipSuccess) break;
-        if (hipEventCreateWithFlags(&S->ev[S->n], hipEventDisableTiming) != hipSuccess) {
-            (void)hipHostFree(S->buf[S->n]);
-            break;
-        }
-        S->n++;
-    }
-    const int nt = S ? std::min(S->n, want) : 0;
-    if (nt == 0) {
-        (void)hipGetLastError();
-        return plain_copy(ctx, dst, src, bytes, kind);
-    }
+    if (!S || !S->make()) return plain_copy(ctx, dst, src, bytes, kind);
+    const int nt = (int)std::min<size_t>(HostStage::N, nchunks);
     std::atomic<size_t> next{0};
     std::atomic<int> err{(int)hipSuccess};
     auto work = [&](int w) {
@@ -397,14 +387,14 @@ hipError_t host_copy(opsec_ctx* ctx, void* dst, const void* src, size_t bytes, h
             if (up) {
                 if (!first) e = hipEventSynchronize(S->ev[w]);   // the slot's last transfer has left it
                 if (e != hipSuccess) break;
-                std::memcpy(S->buf[w], (const char*)src + off, n);
-                e = hipMemcpyAsync((char*)dst + off, S->buf[w], n, kind, ctx->stream);
+                std::memcpy(S->slot(w), (const char*)src + off, n);
+                e = hipMemcpyAsync((char*)dst + off, S->slot(w), n, kind, ctx->stream);
                 if (e == hipSuccess) e = hipEventRecord(S->ev[w], ctx->stream);
             } else {
-                e = hipMemcpyAsync(S->buf[w], (const char*)src + off, n, kind, ctx->stream);
+                e = hipMemcpyAsync(S->slot(w), (const char*)src + off, n, kind, ctx->stream);
                 if (e == hipSuccess) e = hipEventRecord(S->ev[w], ctx->stream);
                 if (e == hipSuccess) e = hipEventSynchronize(S->ev[w]);
-                if (e == hipSuccess) std::memcpy((char*)dst + off, S->buf[w], n);
+                if (e == hipSuccess) std::memcpy((char*)dst + off, S->slot(w), n);
             }
         }
         if (e != hipSuccess) err.store((int)e);
