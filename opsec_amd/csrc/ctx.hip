@@ -328,8 +328,9 @@ static int upload_desc(opsec_ctx* ctx) {
 // eight threads each move chunks through a pinned buffer of their own, the transfers
 // queued on the context's stream: 6.6 ms (41 GB/s), of which 0.25 ms at any size is the
 // start of the threads, hence the least sizes in common.h.  Memory that is pinned
-// already goes directly, and so does a copy whose slots cannot be made.  The slots (32 MB)
-// belong to the context and go with it; the threads live for the call.
+// already goes directly, and so does a copy for which no slot can be made.  The slots (32 MB,
+// 0.5 to 2 ms of a context's first large copy) belong to the context and go with it; the
+// threads live for the call.
 struct HipStageApi {
     typedef hipEvent_t event_t;
     static bool host_alloc(void** p, size_t n) { return hipHostMalloc(p, n, 0) == hipSuccess; }
@@ -374,8 +375,8 @@ hipError_t host_copy(opsec_ctx* ctx, void* dst, const void* src, size_t bytes, h
     if (!lock.owns_lock()) return plain_copy(ctx, dst, src, bytes, kind);
     if (!ctx->stage) ctx->stage = new (std::nothrow) HostStage;
     HostStage* S = ctx->stage;
-    if (!S || !S->make()) return plain_copy(ctx, dst, src, bytes, kind);
-    const int nt = (int)std::min<size_t>(HostStage::N, nchunks);
+    const int nt = S ? S->make((int)std::min<size_t>(HostStage::N, nchunks)) : 0;
+    if (nt == 0) return plain_copy(ctx, dst, src, bytes, kind);
     std::atomic<size_t> next{0};
     std::atomic<int> err{(int)hipSuccess};
     auto work = [&](int w) {
@@ -387,14 +388,14 @@ hipError_t host_copy(opsec_ctx* ctx, void* dst, const void* src, size_t bytes, h
             if (up) {
                 if (!first) e = hipEventSynchronize(S->ev[w]);   // the slot's last transfer has left it
                 if (e != hipSuccess) break;
-                std::memcpy(S->slot(w), (const char*)src + off, n);
-                e = hipMemcpyAsync((char*)dst + off, S->slot(w), n, kind, ctx->stream);
+                std::memcpy(S->buf[w], (const char*)src + off, n);
+                e = hipMemcpyAsync((char*)dst + off, S->buf[w], n, kind, ctx->stream);
                 if (e == hipSuccess) e = hipEventRecord(S->ev[w], ctx->stream);
             } else {
-                e = hipMemcpyAsync(S->slot(w), (const char*)src + off, n, kind, ctx->stream);
+                e = hipMemcpyAsync(S->buf[w], (const char*)src + off, n, kind, ctx->stream);
                 if (e == hipSuccess) e = hipEventRecord(S->ev[w], ctx->stream);
                 if (e == hipSuccess) e = hipEventSynchronize(S->ev[w]);
-                if (e == hipSuccess) std::memcpy((char*)dst + off, S->slot(w), n);
+                if (e == hipSuccess) std::memcpy((char*)dst + off, S->buf[w], n);
             }
         }
         if (e != hipSuccess) err.store((int)e);

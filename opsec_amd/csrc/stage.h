@@ -1,4 +1,4 @@
-// Staging slots of large host copies: pinned memory and an event each.  The runtime's
+// Staging slots of large host copies: a pinned buffer and an event each.  The runtime's
 // calls come through Api, so that the set-up and its failures can be checked without a
 // device.
 #pragma once
@@ -11,34 +11,34 @@ template <typename Api>
 struct StageSlots {
     static constexpr int N = 8;
     static constexpr size_t BYTES = (size_t)4 << 20;
-    char* base = nullptr;            // N slots, pinned
+    void* buf[N] = {};
     typename Api::event_t ev[N] = {};
+    int n = 0;   // slots made
 
-    char* slot(int i) const { return base + (size_t)i * BYTES; }
-    // All slots, or none; a failed call's error is taken back, so that no later check reports it
-    // (the copy that wanted the slots goes through the runtime).
-    bool make() {
-        if (base) return true;
-        void* p = nullptr;
-        if (!Api::host_alloc(&p, N * BYTES)) {
-            Api::clear_error();
-            return false;
-        }
-        for (int i = 0; i < N; i++)
-            if (!Api::event_create(&ev[i])) {
+    // At least `want` slots, or as many as could be made; returns min(n, want).  A failed call's
+    // error is taken back, so that no later check reports it: the copy goes on with fewer slots,
+    // or without.
+    int make(int want) {
+        while (n < want) {
+            if (!Api::host_alloc(&buf[n], BYTES)) {
                 Api::clear_error();
-                while (i-- > 0) Api::event_destroy(ev[i]);
-                Api::host_free(p);
-                return false;
+                break;
             }
-        base = (char*)p;
-        return true;
+            if (!Api::event_create(&ev[n])) {
+                Api::clear_error();
+                Api::host_free(buf[n]);
+                break;
+            }
+            n++;
+        }
+        return n < want ? n : want;
     }
     void release() {
-        if (!base) return;
-        for (int i = 0; i < N; i++) Api::event_destroy(ev[i]);
-        Api::host_free(base);
-        base = nullptr;
+        while (n > 0) {
+            n--;
+            Api::host_free(buf[n]);
+            Api::event_destroy(ev[n]);
+        }
     }
 };
 

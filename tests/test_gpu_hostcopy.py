@@ -5,8 +5,20 @@ import threading
 import numpy as np
 import pytest
 
+from opsec_amd import lib
+
 pytestmark = pytest.mark.gpu
 MB = 1 << 20
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    """A context whose slots are made: its first large copy pays for them."""
+    with lib.Context(0) as c:
+        p = c.dev_alloc(128 * MB)
+        c.h2d(p, np.zeros(128 * MB, dtype=np.uint8))
+        c.dev_free(p)
+        yield c
 
 
 # under, at and over the least staged sizes (8 MB to the host, 32 MB to the device);
@@ -51,3 +63,18 @@ def test_two_threads(ctx):
     finally:
         for p in ptrs:
             ctx.dev_free(p)
+
+
+def test_first_copies_of_a_context():
+    """The runtime's copies, the one that makes the slots, and the staged ones after it."""
+    n = 40 * MB + 3
+    rng = np.random.default_rng(6)
+    with lib.Context(0) as c:
+        p = c.dev_alloc(n)
+        for _ in range(5):
+            src = rng.integers(0, 256, n, dtype=np.uint8)
+            c.h2d(p, src)
+            back = np.empty(9 * MB, dtype=np.uint8)
+            c.d2h(back, p)
+            assert np.array_equal(back, src[:9 * MB])
+        c.dev_free(p)

@@ -11,7 +11,8 @@ PROGRAM = r"""
 #include <cstdio>
 #include <cstdlib>
 #include "stage.h"
-// a runtime whose call number `fail` (allocation, then the events) fails and leaves an error
+// a runtime whose call number `fail` (a slot's allocation, its event, the next slot's) fails and
+// leaves an error
 struct Api {
     typedef int event_t;
     static int calls, fail, error, live_mem, live_ev;
@@ -39,15 +40,15 @@ int Api::calls, Api::fail, Api::error, Api::live_mem, Api::live_ev;
 
 int main(int, char** v) {
     Api::fail = std::atoi(v[1]);
+    const int want = std::atoi(v[2]);
     opsec::StageSlots<Api> s;
-    const bool first = s.make();
-    std::printf("%d %d %d %d ", first, Api::error, Api::live_mem, Api::live_ev);
-    const bool again = s.make();   // the failed call has passed
-    const int calls = Api::calls, third = s.make();
-    const int disjoint = s.slot(s.N - 1) + s.BYTES <= s.base + s.N * s.BYTES && s.slot(1) >= s.slot(0) + s.BYTES;
-    std::printf("%d %d %d %d", again, Api::error, third && calls == Api::calls, disjoint);
+    const int got = s.make(want);
+    std::printf("%d %d %d %d ", got, Api::error, Api::live_mem, Api::live_ev);
+    const int again = s.make(s.N), calls = Api::calls;   // the failed call has passed
+    const int fewer = s.make(3);
+    std::printf("%d %d %d %d %d ", again, Api::error, fewer, calls == Api::calls, Api::live_mem);
     s.release();
-    std::printf(" %d %d\n", Api::live_mem, Api::live_ev);
+    std::printf("%d %d\n", Api::live_mem, Api::live_ev);
 }
 """
 
@@ -61,11 +62,14 @@ def prog(tmp_path_factory):
     return str(d / "t")
 
 
-@pytest.mark.parametrize("fail", range(-1, 9))
-def test_no_slots_and_no_error_left(prog, fail):
-    """Whichever call fails (-1: none), there are all slots or none, nothing is held, no error
-    is left behind, and the next call makes the slots."""
-    out = subprocess.run([prog, str(fail)], capture_output=True, text=True, check=True).stdout.split()
-    ok = fail < 0
-    assert out[:4] == (["1", "0", "1", "8"] if ok else ["0", "0", "0", "0"])
-    assert out[4:] == ["1", "0", "1", "1", "0", "0"]
+@pytest.mark.parametrize("want", [1, 5, 8])
+@pytest.mark.parametrize("fail", range(-1, 17))
+def test_failed_slots_leave_no_error(prog, fail, want):
+    """Whichever call fails (each slot's allocation, then its event; -1: none), the slots before
+    it are kept, nothing else is held, no error is left behind, and the next call goes on."""
+    out = [int(x) for x in subprocess.run([prog, str(fail), str(want)], capture_output=True, text=True,
+                                          check=True).stdout.split()]
+    got = want if fail < 0 else min(want, fail // 2)
+    assert out[:4] == [got, 0, got, got]
+    again = 8 if fail < 0 or got < want or fail >= 16 else fail // 2   # it fails on the second call
+    assert out[4:] == [again, 0, 3, int(again >= 3), max(3, again), 0, 0]   # then three are there
