@@ -75,6 +75,13 @@ int opsec_diag_set_gm_bands(int v);
  * holds, up to eight per CU (three per CU for a shell's prior sweep beside its
  * band sweep); v > 0 caps them at v.  The tables are the same bits. */
 int opsec_diag_set_gm_deep_slots(int v);
+/* The region pools the adaptive cubature takes for npending integrals on a device of
+ * `cus` CUs with `fre` bytes free and `held` in the sweep's pools (rerun: of those that
+ * ran out of a first pool), after `failures` failed allocations: out[0] regions per
+ * pool, out[1] pools, out[2] 1 if a pool holds every region the evaluation cap allows.
+ * OPSEC_ENOMEM when nothing smaller is left to try.  Host only. */
+int opsec_diag_gm_pools(int rerun, int npending, int cus, int maxeval, size_t fre, size_t held, int slot_cap,
+                        int failures, int* out);
 
 #ifdef __cplusplus
 }

@@ -157,6 +157,8 @@ int set_error(opsec_ctx* ctx, int code, const char* fmt, ...);
 
 // Allocate (or re-allocate to at least `bytes`) a device buffer owned by ctx.
 int dev_realloc(opsec_ctx* ctx, void** p, size_t* cap, size_t bytes);
+// The same without an error in ctx, for callers that have another way; 0 bytes: freed.
+hipError_t dev_try_realloc(void** p, size_t* cap, size_t bytes);
 void dev_free(void** p);
 
 // Device buffers owned by one call: freed when the scope ends, error returns

@@ -35,20 +35,28 @@ int set_error(opsec_ctx* ctx, int code, const char* fmt, ...) {
     return code;
 }
 
-int dev_realloc(opsec_ctx* ctx, void** p, size_t* cap, size_t bytes) {
-    if (*p && *cap >= bytes) return OPSEC_OK;
+hipError_t dev_try_realloc(void** p, size_t* cap, size_t bytes) {
+    if (*p && bytes > 0 && *cap >= bytes) return hipSuccess;
     if (*p) {
         hipFree(*p);
         *p = nullptr;
         *cap = 0;
     }
-    if (bytes == 0) return OPSEC_OK;
-    hipError_t e = hipMalloc(p, bytes);
-    if (e != hipSuccess) {
+    if (bytes == 0) return hipSuccess;
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) {
+        *cap = bytes;
+    } else {
         *p = nullptr;
-        return set_error(ctx, OPSEC_ENOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
+        (void)hipGetLastError();   // answered here: not for the next launch's check
     }
-    *cap = bytes;
+    return e;
+}
+
+int dev_realloc(opsec_ctx* ctx, void** p, size_t* cap, size_t bytes) {
+    if (*p && *cap >= bytes) return OPSEC_OK;
+    const hipError_t e = dev_try_realloc(p, cap, bytes);
+    if (e != hipSuccess) return set_error(ctx, OPSEC_ENOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
     return OPSEC_OK;
 }
 

@@ -1624,6 +1624,51 @@ constexpr int GM_WAVE_PENDING = 16;
 // the integrals that need more soon get a workgroup of their own instead of holding
 // one wave for 4096 regions (8x8x8 shell's prior: pass 0 28 ms with 4096, 6.8 with 1024).
 constexpr int GM_POOL = 1024;
+// Region pools of a gm_kernel launch: `slots` of `regions` regions; whole: they hold every
+// region the evaluation cap allows.
+struct GMPools {
+    int regions, slots;
+    bool whole;
+};
+constexpr size_t GM_REGION_BYTES = GM_SLOT_DOUBLES * 8 + GM_SLOT_INTS * 4;
+// Whole-cap pools taken at once: 42 integrals at the default cap (48 MB each).  A box's near
+// pairs (27, all of them deep) need 1.3 GB and are spared a first pool and the rerun, 99 -> 92 ms
+// with the 12^3 prior; an 8x8x8 shell's bands (175, a few splits each) would take 8.5 GB, and
+// allocating and freeing that much beside the prior's sweep held up one call in
+// ten by 0.1 to 3 s.
+constexpr size_t GM_WHOLE_BYTES = (size_t)2 << 30;
+// The pools of nrun pending integrals (rerun: those that ran out of a GM_POOL pool), with
+// `fre` bytes of device memory free and `held` in this sweep's pools already.  At first
+// GM_POOL regions, or whole-cap pools when there is at most one per CU and all of them
+// fit GM_WHOLE_BYTES and a quarter of the free memory (a shell's two sweeps may size theirs
+// at the same time).  In a rerun as many whole-cap pools as half the free memory holds.
+// slot_cap > 0 bounds their number.
+static GMPools gm_pools(bool rerun, int nrun, int cus, unsigned maxeval, size_t fre, size_t held, int slot_cap) {
+    const long long cap = maxeval ? (long long)maxeval / GM_NPTS + 2 : (1LL << 20);
+    GMPools g{(int)std::min<long long>(cap, 1LL << 22), std::min(nrun, cus * 8), true};
+    const size_t per_slot = (size_t)g.regions * GM_REGION_BYTES;
+    if (!rerun) {
+        if (nrun > cus || (size_t)nrun > std::max(held, std::min(GM_WHOLE_BYTES, fre / 4)) / per_slot) return GMPools{GM_POOL, g.slots, false};
+    } else {
+        const size_t budget = std::max<size_t>(held, std::max<size_t>((size_t)1 << 30, fre / 2));
+        g.slots = (int)std::max<size_t>(1, std::min<size_t>(g.slots, budget / per_slot));
+    }
+    if (slot_cap > 0) g.slots = std::min(g.slots, slot_cap);
+    return g;
+}
+// What to try when the memory for g is not there (another sweep or program took it):
+// GM_POOL regions each instead of whole-cap pools at first, then half as many; false
+// when one slot was too much.
+static bool gm_pools_fewer(GMPools& g, bool rerun, int nrun, int cus) {
+    if (!rerun && g.whole) {
+        g = GMPools{GM_POOL, std::min(nrun, cus * 8), false};
+        return true;
+    }
+    if (g.slots <= 1) return false;
+    g.slots = (g.slots + 1) / 2;
+    return true;
+}
+
 // Shell tables: the deep sweep beside the shallow one on a second stream (1, the
 // default) or after it (0).
 static int g_gm_overlap = 1;
@@ -1658,10 +1703,8 @@ static int run_gm_device(opsec_ctx* ctx, int nf, const int* funcs, const GMJob* 
     P.coordsys = ctx->sv.coordsys;
     P.L = ctx->sv.L;
     // Pass 0: every job's first region (one thread per job), then the jobs
-    // that need splits with a GM_POOL-region pool per workgroup, or, when there is
-    // at most one per CU, with pools that hold every region the evaluation cap
-    // allows (maxeval / 149 + 2).  Pass 1: jobs that exhausted their pool, with
-    // whole-cap pools.
+    // that need splits with a region pool per workgroup (gm_pools).  Pass 1: jobs
+    // that exhausted a GM_POOL-region pool, with whole-cap pools.
     const size_t njobs_all = npairs * (size_t)nf;
     if (njobs_all > (size_t)INT32_MAX) return set_error(ctx, OPSEC_EINVAL, "too many pair integrals in one call");
     // A shell's sweep of closed-form bands takes its first regions from
@@ -1706,6 +1749,7 @@ static int run_gm_device(opsec_ctx* ctx, int nf, const int* funcs, const GMJob* 
         int* d_ndeep = (int*)((char*)sc.p + 24);
         const int* d_idx = nullptr;
         int nrun = njobs;
+        GMPools pools{0, 0, false};
         GMJobs jobs{(const GMJob*)sj.p, nullptr, 0};   // the rerun's gathered jobs
         int* d_failed_list = (int*)sp.p;               // not the list the jobs are read from
         if (pass == 0) {
@@ -1747,25 +1791,26 @@ static int run_gm_device(opsec_ctx* ctx, int nf, const int* funcs, const GMJob* 
             OPSEC_HIP_TRY(ctx, hipMemcpyAsync(sj.p, sa.p, sizeof(GMJob) * njobs, hipMemcpyDeviceToDevice, stm));
         }
         if (nrun > 0) {
-            const long long cap_regions = P.maxEval ? (long long)P.maxEval / GM_NPTS + 2 : (1LL << 20);
-            const bool deep = pass == 1 || nrun <= ctx->num_cus;
-            P.rmax = deep ? (int)std::min<long long>(cap_regions, 1LL << 22) : GM_POOL;
-            const size_t per_slot = (size_t)P.rmax * (GM_SLOT_DOUBLES * 8 + GM_SLOT_INTS * 4);
-            int nslots = std::min(nrun, ctx->num_cus * 8);
-            if (deep) {
-                // as many workgroups as half the free device memory (and what this sweep
-                // already holds) has pools for
-                size_t fre = 0, tot = 0;
-                if (hipMemGetInfo(&fre, &tot) != hipSuccess) fre = (size_t)16 << 30;
-                const size_t budget = std::max<size_t>(sd.cap + si.cap, std::max<size_t>((size_t)1 << 30, fre / 2));
-                nslots = (int)std::max<size_t>(1, std::min<size_t>(nslots, budget / per_slot));
-                const int cap = g_gm_deep_slots > 0 ? g_gm_deep_slots : deep_cap;
-                if (cap > 0) nslots = std::min(nslots, cap);
+            size_t fre = 0, tot = 0;
+            if ((pass == 1 || nrun <= ctx->num_cus) && hipMemGetInfo(&fre, &tot) != hipSuccess) {
+                (void)hipGetLastError();
+                fre = (size_t)16 << 30;
             }
-            if ((rc = dev_realloc(ctx, &sd.p, &sd.cap, sizeof(double) * GM_SLOT_DOUBLES * (size_t)P.rmax * nslots)))
-                return rc;
-            if ((rc = dev_realloc(ctx, &si.p, &si.cap, sizeof(int) * GM_SLOT_INTS * (size_t)P.rmax * nslots))) return rc;
-            launch_gm(ctx, stm, nslots, mv, jobs, d_idx, nrun, d_counter, (double*)sd.p, (int*)si.p, P,
+            pools = gm_pools(pass == 1, nrun, ctx->num_cus, P.maxEval, fre, sd.cap + si.cap,
+                             g_gm_deep_slots > 0 ? g_gm_deep_slots : deep_cap);
+            hipError_t e = hipSuccess;
+            do {
+                const size_t n = (size_t)pools.regions * pools.slots;
+                e = dev_try_realloc(&sd.p, &sd.cap, sizeof(double) * GM_SLOT_DOUBLES * n);
+                if (e == hipSuccess) e = dev_try_realloc(&si.p, &si.cap, sizeof(int) * GM_SLOT_INTS * n);
+                if (e == hipSuccess) break;
+                (void)dev_try_realloc(&sd.p, &sd.cap, 0);
+            } while (gm_pools_fewer(pools, pass == 1, nrun, ctx->num_cus));
+            if (e != hipSuccess)
+                return set_error(ctx, OPSEC_ENOMEM, "adaptive cubature: no memory for a pool of %d regions: %s",
+                                 pools.regions, hipGetErrorString(e));
+            P.rmax = pools.regions;
+            launch_gm(ctx, stm, pools.slots, mv, jobs, d_idx, nrun, d_counter, (double*)sd.p, (int*)si.p, P,
                       dQ, nkeys, dQerr, (int*)sf.p, d_nev);
             OPSEC_HIP_TRY(ctx, hipGetLastError());
         }
@@ -2652,6 +2697,18 @@ int opsec_diag_set_gm_overlap(int v) {
 
 // Wavefront slots of the deep rerun (0: as many as memory allows, up to eight
 // per CU).
+int opsec_diag_gm_pools(int rerun, int npending, int cus, int maxeval, size_t fre, size_t held, int slot_cap,
+                        int failures, int* out) {
+    if (!out || npending < 1 || cus < 1 || maxeval < 0) return OPSEC_EINVAL;
+    GMPools g = gm_pools(rerun != 0, npending, cus, (unsigned)maxeval, fre, held, slot_cap);
+    for (; failures > 0; failures--)
+        if (!gm_pools_fewer(g, rerun != 0, npending, cus)) return OPSEC_ENOMEM;
+    out[0] = g.regions;
+    out[1] = g.slots;
+    out[2] = g.whole;
+    return OPSEC_OK;
+}
+
 int opsec_diag_set_gm_deep_slots(int v) {
     if (v < 0) return OPSEC_EINVAL;
     g_gm_deep_slots = v;

@@ -154,6 +154,7 @@ _DIAG_SIGS = {
     "opsec_diag_set_gm_overlap": ([_I], _I),
     "opsec_diag_set_gm_bands": ([_I], _I),
     "opsec_diag_set_gm_deep_slots": ([_I], _I),
+    "opsec_diag_gm_pools": ([_I, _I, _I, _I, C.c_size_t, C.c_size_t, _I, _I, _P], _I),
 }
 
 
