@@ -1625,7 +1625,7 @@ constexpr int GM_WAVE_PENDING = 16;
 // one wave for 4096 regions (8x8x8 shell's prior: pass 0 28 ms with 4096, 6.8 with 1024).
 constexpr int GM_POOL = 1024;
 // Region pools of a gm_kernel launch: `slots` of `regions` regions; whole: they hold every
-// region the evaluation cap allows.
+// region the evaluation cap allows, so running out of one is final.
 struct GMPools {
     int regions, slots;
     bool whole;
@@ -1826,7 +1826,7 @@ static int run_gm_device(opsec_ctx* ctx, int nf, const int* funcs, const GMJob* 
         OPSEC_HIP_TRY(ctx, hipMemcpyAsync(&nfail, d_nfail, 4, hipMemcpyDeviceToHost, stm));
         OPSEC_HIP_TRY(ctx, hipStreamSynchronize(stm));
         nev_total += nev;
-        if (nfail > 0 && pass == 1)
+        if (nfail > 0 && pools.whole)
             return set_error(ctx, OPSEC_ECONV, "adaptive cubature exceeded %d regions", P.rmax);
         std::vector<int> failed(nfail);
         if (nfail > 0) {

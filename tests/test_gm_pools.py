@@ -2,6 +2,8 @@
 when the memory is not there.  CPU only: the host rule through its diagnostic."""
 import ctypes as C
 
+import pytest
+
 from opsec_amd import lib
 
 CUS, CAP = 256, 50000000
@@ -44,6 +46,13 @@ def test_rerun_takes_half_the_free_memory_and_the_cap():
     assert pools(1, 5000, free=0)[1] == GB // (WHOLE * REGION)
     assert pools(1, 5000, cap=3 * CUS) == (WHOLE, 3 * CUS, 1)
     assert pools(1, 3, maxeval=2 ** 31 - 1, free=0) == (1 << 22, 1, 1)
+
+
+@pytest.mark.parametrize("maxeval,regions", [(0, 1 << 20), (2 ** 31 - 1, 1 << 22), (CAP, WHOLE)])
+def test_running_out_of_a_whole_pool_is_final(maxeval, regions):
+    """No second sweep with the same pools: `whole` says that the first one decides."""
+    assert pools(0, 3, maxeval=maxeval) == (regions, 3, 1) == pools(1, 3, maxeval=maxeval)
+    assert pools(0, CUS + 1, maxeval=maxeval)[2] == 0
 
 
 def test_smaller_pools_when_the_memory_is_not_there():

@@ -289,3 +289,17 @@ def test_gm_deep_heap_levels(ctx):
     ref = S[0, 0] / cells["Nbar"][0]
     print("deep self pair", got, "error estimate", err, flush=True)
     assert abs(got - ref) <= 1e-12 * abs(ref)
+
+
+def test_gm_running_out_of_regions_is_an_error(ctx):
+    """Without an evaluation cap and with a tolerance out of reach the pool ends the integral, and
+    the next integral is right again."""
+    cells = synth.box_cells(2, 0.0, 40.0)
+    sv = lib.survey_box(2, 0.0, 40.0, L=1e9)
+    ctx.model_test(0, 1.0, 0.3)
+    q = ctx.quad(lib.OPSEC_QUAD_GM, epsrel=0.0, epsabs=0.0, maxeval=0)
+    with pytest.raises(lib.OpsecError, match="exceeded 1048576 regions"):
+        ctx.pair_integral(cells[0], cells[0], 0, sv, q)
+    ok = ctx.quad(lib.OPSEC_QUAD_GM, epsrel=1e-5, maxeval=100000)
+    a = ctx.pair_integral(cells[0], cells[1], 0, sv, ok)
+    assert a == ctx.pair_integral(cells[0], cells[1], 0, sv, ok)
