@@ -1956,9 +1956,14 @@ static int run_quadrature(opsec_ctx* ctx, int nf, const int* funcs, const std::v
         if (nfar) {
             int per, bs, threads;
             tent_split(ctx, rule.n, nfar, &per, &bs, &threads);
-            hipLaunchKernelGGL(tent_kernel, dim3((unsigned)((nfar + per - 1) / per)), dim3(threads), 0, ctx->stream, mv,
-                               dj, (int)nfar, rule, per, bs, ctx->sv.L, dQ, nkeys);
-            OPSEC_HIP_TRY(ctx, hipGetLastError());
+            // a launch takes fewer than 2^32 threads: 16.7 million integrals of 22 nodes per axis
+            const size_t most = (size_t)per * (UINT32_MAX / (unsigned)threads);
+            for (size_t o = 0; o < nfar; o += most) {
+                const size_t n = std::min(most, nfar - o);
+                hipLaunchKernelGGL(tent_kernel, dim3((unsigned)((n + per - 1) / per)), dim3(threads), 0, ctx->stream,
+                                   mv, dj + o, (int)n, rule, per, bs, ctx->sv.L, dQ, nkeys);
+                OPSEC_HIP_TRY(ctx, hipGetLastError());
+            }
         }
         if (nnear && near_cols) {
             hipLaunchKernelGGL(tent_near_cols_kernel,

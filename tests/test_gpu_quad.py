@@ -303,3 +303,22 @@ def test_gm_running_out_of_regions_is_an_error(ctx):
     ok = ctx.quad(lib.OPSEC_QUAD_GM, epsrel=1e-5, maxeval=100000)
     a = ctx.pair_integral(cells[0], cells[1], 0, sv, ok)
     assert a == ctx.pair_integral(cells[0], cells[1], 0, sv, ok)
+
+
+def test_gauss_more_threads_than_a_launch_takes(ctx):
+    """16.8 million integrals of 22 nodes per axis, a workgroup of 256 threads each (two cells of a
+    104 x 100 x 101 grid, 16 bands): the last band's table is the one of that band alone."""
+    n1, n2, n3 = 104, 100, 101
+    cells = synth.box_cells(2, 0.0, 20.0)[[0, 7]].copy()
+    cells["a"] = [0, 1]
+    sv = lib.survey_box(n1, 0.0, 10.0 * n1, L=1e9, ny=n2, nz=n3)
+    sv.max2, sv.max3 = 10.0 * n2, 10.0 * n3
+    lo, hi = synth.linear_bands(16, 0.001, 0.003)
+    ctx.model_real(GOLD["pk_k"], GOLD["pk_P"], lo, hi, lib.OPSEC_XI_CLOSED)
+    ctx.cells_upload(cells, sv)
+    q = ctx.quad(lib.OPSEC_QUAD_GAUSS, nodes=22, near=1)
+    ctx.pair_tables(list(range(1, 17)), q)
+    many = ctx.pair_table(16)
+    ctx.pair_tables([16], q)
+    assert np.array_equal(ctx.pair_table(16), many)
+    assert np.all(np.isfinite(many)) and np.count_nonzero(many) == n1 * n2 * n3
