@@ -177,6 +177,7 @@ struct DevScratch {
         hipError_t e = hipMalloc(&q, bytes);
         *out = e == hipSuccess ? (T*)q : nullptr;
         if (e == hipSuccess) bufs.push_back(q);
+        else (void)hipGetLastError();   // answered by the caller: not for the next launch's check
         return e;
     }
 };

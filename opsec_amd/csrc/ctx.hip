@@ -522,7 +522,10 @@ int opsec_device_info(opsec_ctx* ctx, int* num_cus, char* arch, int arch_len) {
 int opsec_dev_alloc(opsec_ctx* ctx, size_t bytes, void** dptr) {
     if (!ctx || !dptr) return OPSEC_EINVAL;
     hipError_t e = hipMalloc(dptr, bytes);
-    if (e != hipSuccess) return set_error(ctx, OPSEC_ENOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        return set_error(ctx, OPSEC_ENOMEM, "hipMalloc(%zu): %s", bytes, hipGetErrorString(e));
+    }
     ctx->user_bufs.push_back(*dptr);
     return OPSEC_OK;
 }

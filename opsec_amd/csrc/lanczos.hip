@@ -1141,6 +1141,7 @@ static int block_lanczos(opsec_ctx* ctx, const double* S, int N, int nev, double
         rb.T = nullptr;
         if (hipMalloc(&rb.T, (size_t)K * K * 8) != hipSuccess) {
             rb.T = nullptr;
+            (void)hipGetLastError();
             rc = set_error(ctx, OPSEC_ENOMEM, "Ritz workspace");
             break;
         }
@@ -1154,6 +1155,7 @@ static int block_lanczos(opsec_ctx* ctx, const double* S, int N, int nev, double
         const int want = std::min(nev, K);
         if (hipMalloc(&dZ, (size_t)K * want * 8) != hipSuccess) {
             dZ = nullptr;
+            (void)hipGetLastError();
             rc = set_error(ctx, OPSEC_ENOMEM, "Ritz vectors");
             break;
         }

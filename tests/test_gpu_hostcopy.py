@@ -5,7 +5,7 @@ import threading
 import numpy as np
 import pytest
 
-from opsec_amd import lib
+from opsec_amd import lib, synth
 
 pytestmark = pytest.mark.gpu
 MB = 1 << 20
@@ -78,3 +78,22 @@ def test_first_copies_of_a_context():
             c.d2h(back, p)
             assert np.array_equal(back, src[:9 * MB])
         c.dev_free(p)
+
+
+def test_refused_allocation_leaves_the_context_usable():
+    """More memory than there is: the call fails, and the launches of the next ones are not
+    blamed for it, through every path that allocates."""
+    cells = synth.box_cells(2, 0.0, 20.0)
+    sv = lib.survey_box(2, 0.0, 20.0, L=1e9)
+    with lib.Context(0) as c:
+        c.model_test(0, 1.0, 0.1)
+        c.cells_upload(cells, sv)
+        q = c.quad(lib.OPSEC_QUAD_GAUSS, nodes=4, near=1)
+        with pytest.raises(lib.OpsecError):
+            c.dev_alloc(1 << 50)
+        c.pair_tables([0], q)
+        S = c.assemble(0, len(cells))
+        with pytest.raises(lib.OpsecError):   # its buffer on the device; the host's S is never read
+            c.check(c.lib.opsec_project_dense(c.h, 1 << 20, S.ctypes.data, 2, S.ctypes.data, 0, S.ctypes.data))
+        got = c.project_dense(S, np.eye(8), lib.OPSEC_PREC_FP64)
+        assert np.array_equal(got, [S[i, j] for j in range(8) for i in range(j + 1)])
