@@ -41,7 +41,7 @@ struct ProjState {
     size_t cap_P = 0;
     float* d_Ppart = nullptr;    // split-K partials of one band's stage 2 (FP32)
     size_t cap_Ppart = 0;
-    int nb = 0;                  // bands in d_P
+    int nb = 0, M = 0;           // bands in d_P, of M modes
     int prec = 0;
     std::vector<int> funcs;
     float last_ms_stage1 = 0, last_ms_stage2 = 0;
@@ -1278,6 +1278,21 @@ static dim3 blocks_for(size_t threads) { return dim3((unsigned)((threads + 255) 
 // and 65536 rows of 65536 columns with their padding are more.
 static dim3 strided_blocks(size_t n) { return blocks_for(std::min<size_t>(n, (size_t)1 << 30)); }
 
+// Room for the packed results of nb bands.  The last projection's results are gone where its
+// buffer is replaced, and once the caller starts to write (results_begin).
+static int results_room(opsec_ctx* ctx, int nb) {
+    ProjState* ps = ctx->proj;
+    const size_t bytes = (size_t)nb * packed_size(ctx->nmodes) * 8;
+    if (bytes > ps->cap_P) ps->nb = 0;
+    return dev_realloc(ctx, &ps->d_P, &ps->cap_P, bytes);
+}
+static void results_begin(ProjState* ps) { ps->nb = 0; }
+static void results_done(opsec_ctx* ctx, int nb, int prec) {
+    ctx->proj->nb = nb;
+    ctx->proj->M = ctx->nmodes;
+    ctx->proj->prec = prec;
+}
+
 // Split a row-major double matrix (rows x cols, ldx) into a plane pair of
 // rows_p x ld.
 static int split_planes(opsec_ctx* ctx, const double* X, size_t ldx, int rows, int cols, __bf16* planes, int rows_p,
@@ -1400,7 +1415,7 @@ static int run_project_bf16x3(opsec_ctx* ctx, int nb, const int* funcs) {
     if (!gen)
         if ((rc = dev_realloc(ctx, (void**)&ps->d_Sp, &ps->cap_Sp, 2 * Kp * Pp * sizeof(__bf16)))) return rc;
     if ((rc = dev_realloc(ctx, (void**)&ps->d_Cp, &ps->cap_Cp, 2 * Mp * Pp * sizeof(__bf16)))) return rc;
-    if ((rc = dev_realloc(ctx, &ps->d_P, &ps->cap_P, (size_t)nb * packed_size(M) * 8))) return rc;
+    if ((rc = results_room(ctx, nb))) return rc;
     if (g_s2_split > 1 &&
         (rc = dev_realloc(ctx, (void**)&ps->d_Ppart, &ps->cap_Ppart, (size_t)g_s2_split * packed_size(M) * 4)))
         return rc;
@@ -1417,6 +1432,7 @@ static int run_project_bf16x3(opsec_ctx* ctx, int nb, const int* funcs) {
     }
     std::vector<hipEvent_t> ev(4 * (size_t)nb);
     for (auto& e : ev) OPSEC_HIP_TRY(ctx, hipEventCreate(&e));
+    results_begin(ps);
     __bf16* Sh = ps->d_Sp;
     __bf16* Sl = ps->d_Sp + Kp * Pp;
     EpiPlanes toC{ps->d_Cp, ps->d_Cp + Mp * Pp, Pp};
@@ -1481,8 +1497,7 @@ static int run_project_bf16x3(opsec_ctx* ctx, int nb, const int* funcs) {
     ps->last_launches2 = nb;
     ps->last_ms_stage1 = tg + t1;
     ps->last_ms_stage2 = t2;
-    ps->nb = nb;
-    ps->prec = OPSEC_PREC_BF16X3;
+    results_done(ctx, nb, OPSEC_PREC_BF16X3);
     return OPSEC_OK;
 }
 
@@ -1557,7 +1572,7 @@ static int run_project_toeplitz(opsec_ctx* ctx, int nb, const int* funcs) {
     if (!tgrid.sph && (rc = dev_realloc(ctx, (void**)&ps->d_Qhat, &ps->cap_Qhat, (size_t)(n1 + 1) * G * 8)))
         return rc;
     if ((rc = dev_realloc(ctx, (void**)&ps->d_Yhat, &ps->cap_Yhat, (size_t)M * nbat * G * 4))) return rc;
-    if ((rc = dev_realloc(ctx, &ps->d_P, &ps->cap_P, (size_t)nb * packed_size(M) * 8))) return rc;
+    if ((rc = results_room(ctx, nb))) return rc;
     const int s2 = std::max(1, std::min(g_s2_split_toep, (int)(Kg / PK)));
     // stage 2 runs once per group of up to TOEP_GROUP bands: the 136 upper tiles x 4
     // split-K parts of one band fill 2.1 rounds of the CUs, eight bands 17 (against
@@ -1615,6 +1630,7 @@ static int run_project_toeplitz(opsec_ctx* ctx, int nb, const int* funcs) {
     const int ngroups = (nb + grp - 1) / grp;
     std::vector<hipEvent_t> ev(4 * (size_t)nb + 2 * (size_t)ngroups);
     for (auto& e : ev) OPSEC_HIP_TRY(ctx, hipEventCreate(&e));
+    results_begin(ps);
     hipEvent_t* evb = ev.data();
     hipEvent_t* evg = ev.data() + 4 * (size_t)nb;
     float tg = 0, t1 = 0, t2 = 0;
@@ -1686,8 +1702,7 @@ static int run_project_toeplitz(opsec_ctx* ctx, int nb, const int* funcs) {
     ps->last_launches2 = ngroups;
     ps->last_ms_stage1 = tg + t1;
     ps->last_ms_stage2 = t2;
-    ps->nb = nb;
-    ps->prec = OPSEC_PREC_BF16X3;
+    results_done(ctx, nb, OPSEC_PREC_BF16X3);
     return OPSEC_OK;
 }
 
@@ -1749,7 +1764,7 @@ static int run_project_toeplitz_nt(opsec_ctx* ctx, int nb, const int* funcs, int
     if ((rc = dev_realloc(ctx, &tp.Y, &tp.cap_Y, (size_t)grp * ystride * sizeof(T)))) return rc;
     if ((rc = dev_realloc(ctx, &ps->d_T, &ps->cap_T, (size_t)sub * tstride * sizeof(T)))) return rc;
     if (!tgrid.sph && (rc = dev_realloc(ctx, (void**)&ps->d_Qhat, &ps->cap_Qhat, (size_t)(n1 + 1) * G * 8))) return rc;
-    if ((rc = dev_realloc(ctx, &ps->d_P, &ps->cap_P, (size_t)nb * packed_size(M) * 8))) return rc;
+    if ((rc = results_room(ctx, nb))) return rc;
     if (!tp.valid) {
         std::vector<int> gmap;
         if ((rc = toep_gmap(ctx, Ng, gmap))) return rc;
@@ -1788,6 +1803,7 @@ static int run_project_toeplitz_nt(opsec_ctx* ctx, int nb, const int* funcs, int
     // events: per stage-1 launch its start and end, That generated; per group: stage 2
     std::vector<hipEvent_t> ev(3 * (size_t)nsub + 2 * (size_t)ngroups);
     for (auto& e : ev) OPSEC_HIP_TRY(ctx, hipEventCreate(&e));
+    results_begin(ps);
     hipEvent_t* evg = ev.data() + 3 * (size_t)nsub;
     const size_t np = (size_t)packed_size(M);
     T* Tp = (T*)ps->d_T;
@@ -1857,8 +1873,7 @@ static int run_project_toeplitz_nt(opsec_ctx* ctx, int nb, const int* funcs, int
     ps->last_launches2 = ngroups;
     ps->last_ms_stage1 = tg + t1;
     ps->last_ms_stage2 = t2;
-    ps->nb = nb;
-    ps->prec = prec;
+    results_done(ctx, nb, prec);
     return OPSEC_OK;
 }
 
@@ -1884,11 +1899,12 @@ static int run_project_dense_nt(opsec_ctx* ctx, int nb, const int* d_funcs, cons
     int rc;
     if ((rc = dev_realloc(ctx, &ps->d_C, &ps->cap_C, (size_t)grp * per_band * sizeof(T)))) return rc;
     if ((rc = dev_realloc(ctx, &ps->d_T, &ps->cap_T, (size_t)sub * tband * sizeof(T)))) return rc;
-    if ((rc = dev_realloc(ctx, &ps->d_P, &ps->cap_P, (size_t)nb * packed_size(M) * 8))) return rc;
+    if ((rc = results_room(ctx, nb))) return rc;
     const size_t np = (size_t)packed_size(M);
     const int ngroups = (nb + grp - 1) / grp;
     std::vector<hipEvent_t> ev(2 * (size_t)ngroups + 1);
     for (auto& e : ev) OPSEC_HIP_TRY(ctx, hipEventCreate(&e));
+    results_begin(ps);
     hipEventRecord(ev[0], ctx->stream);
     T* Tp = (T*)ps->d_T;
     for (int gi = 0; gi < ngroups; gi++) {
@@ -1932,8 +1948,7 @@ static int run_project_dense_nt(opsec_ctx* ctx, int nb, const int* d_funcs, cons
     if (rc) return rc;
     ps->last_ms_stage1 = t1;
     ps->last_ms_stage2 = t2;
-    ps->nb = nb;
-    ps->prec = prec;
+    results_done(ctx, nb, prec);
     return OPSEC_OK;
 }
 
@@ -1989,15 +2004,19 @@ static int project_host_nt(opsec_ctx* ctx, int N, const double* dS, int M, const
     return OPSEC_OK;
 }
 
-// A new cell set invalidates the uploaded modes and everything derived from them.
-void invalidate_modes(opsec_ctx* ctx) {
+// The uploaded modes and everything derived from them are no longer to be used.
+static void drop_modes(opsec_ctx* ctx) {
     ctx->nmodes = 0;
     if (!ctx->proj) return;
     ctx->proj->bp_valid = false;
     ctx->proj->bw32_valid = false;
     ctx->proj->toep_valid = false;
     for (auto& t : ctx->proj->toep) t.valid = false;
-    ctx->proj->nb = 0;
+}
+// A new cell set takes the last projection's results with them.
+void invalidate_modes(opsec_ctx* ctx) {
+    drop_modes(ctx);
+    if (ctx->proj) ctx->proj->nb = 0;
 }
 
 void free_proj(opsec_ctx* ctx) {
@@ -2053,6 +2072,7 @@ int opsec_modes_upload(opsec_ctx* ctx, const double* B, int ncells, int nmodes) 
     ProjState* ps = ctx->proj;
     size_t bytes = (size_t)ncells * nmodes * 8;
     int rc;
+    drop_modes(ctx);   // until the new ones are there whole: a failed upload leaves none
     dev_free((void**)&ctx->d_B);
     size_t capB = 0;
     if ((rc = dev_realloc(ctx, (void**)&ctx->d_B, &capB, bytes))) return rc;
@@ -2064,10 +2084,6 @@ int opsec_modes_upload(opsec_ctx* ctx, const double* B, int ncells, int nmodes) 
     OPSEC_HIP_TRY(ctx, hipGetLastError());
     OPSEC_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     ctx->nmodes = nmodes;
-    ps->bp_valid = false;
-    ps->bw32_valid = false;
-    ps->toep_valid = false;
-    for (auto& t : ps->toep) t.valid = false;
     return OPSEC_OK;
 }
 
@@ -2237,9 +2253,10 @@ int opsec_project_dense(opsec_ctx* ctx, int n, const double* S, int nmodes, cons
 }  // extern "C"
 
 namespace opsec {
-// Device-resident results of the last opsec_project call (nb packed matrices).
+// Device-resident results of the last opsec_project call (nb packed matrices); none where
+// modes of another number have been uploaded since.
 void* proj_device_results(opsec_ctx* ctx, int* nb, int* M) {
-    if (!ctx->proj || !ctx->proj->d_P || ctx->proj->nb == 0) return nullptr;
+    if (!ctx->proj || !ctx->proj->d_P || ctx->proj->nb == 0 || ctx->proj->M != ctx->nmodes) return nullptr;
     *nb = ctx->proj->nb;
     *M = ctx->nmodes;
     return ctx->proj->d_P;

@@ -551,3 +551,27 @@ def test_project_dense_more_elements_than_threads(ctx, prec):
     P = (2 * np.outer(B[:, 0], B[:, 0]) + 3 * np.outer(B[:, 40000], B[:, 123]) + 5 * np.outer(B[:, -1], B[:, -1]) +
          np.outer(B[:, -1], B[:, 7]))
     assert np.array_equal(got, _packed(P))
+
+
+def test_results_belong_to_their_modes(ctx):
+    """Matrices projected on 8 modes are not read as those of 20 or of 5 (which they are too few
+    for, or mean something else) after a new mode upload; on 8 modes again they are what they were."""
+    cells = synth.box_cells(4, 0.0, 100.0)
+    ctx.model_real(GOLD["pk_k"], GOLD["pk_P"], [0.02, 0.05], [0.05, 0.1], lib.OPSEC_XI_CLOSED)
+    ctx.cells_upload(cells, lib.survey_box(4, 0.0, 100.0))
+    ctx.pair_tables([1, 2], ctx.quad(lib.OPSEC_QUAD_GAUSS, nodes=4, near=1))
+    B = np.linalg.qr(np.random.default_rng(3).normal(size=(64, 20)))[0].T.copy()
+
+    def estimate(m):
+        return ctx.estimate_device(np.linspace(3.0, 1.0, m), np.ones(m), np.ones(2), lib.OPSEC_MIX_IDENTITY)
+
+    ctx.modes_upload(B[:8])
+    ctx.project([1, 2], lib.OPSEC_PREC_FP64, keep_on_device=True)
+    first = estimate(8)
+    for m in (20, 5):
+        ctx.modes_upload(B[:m])
+        with pytest.raises(lib.OpsecError, match="no projection results"):
+            estimate(m)
+    ctx.modes_upload(B[:8])
+    again = estimate(8)
+    assert all(np.array_equal(first[k], again[k]) for k in first)
