@@ -337,26 +337,28 @@ struct NtWork {
 };
 
 // All work items of g on ctx's stream: whole rounds of two workgroups per CU,
-// then the rest, its K range split over the CUs when that pays.
+// then the rest, its K range split over the CUs when that pays and there is memory for the
+// parts.
 template <typename T, typename Out>
-inline int launch_nt_gemm(opsec_ctx* ctx, NtWork& ws, NtArgs<T> g, const Out& O) {
+inline void launch_nt_gemm(opsec_ctx* ctx, NtWork& ws, NtArgs<T> g, const Out& O) {
     const int cus = std::max(1, ctx->num_cus);
     hipStream_t s = ctx->stream;
     const int nmb = (g.M + NT_BM - 1) / NT_BM, nnb = (g.N + NT_BN - 1) / NT_BN;
     const int total = nt_tiles(nmb, nnb, Out::lower) * g.nz, rest = total % (2 * cus);
-    const int parts = g.serial ? 1 : nt_split(rest, g.ksteps, cus), whole = parts > 1 ? total - rest : total;
+    int parts = g.serial ? 1 : nt_split(rest, g.ksteps, cus);
+    if (parts > 1 &&
+        dev_try_realloc(&ws.p, &ws.cap, (size_t)rest * parts * NT_BM * NT_BN * sizeof(T)) != hipSuccess)
+        parts = 1;
+    const int whole = parts > 1 ? total - rest : total;
     g.item0 = 0;
     g.nsplit = 1;
     if (whole > 0) hipLaunchKernelGGL((nt_gemm_kernel<T, Out, false>), dim3(whole), dim3(256), NT_LDS, s, g, O);
-    if (whole == total) return OPSEC_OK;
-    const int rc = dev_realloc(ctx, &ws.p, &ws.cap, (size_t)rest * parts * NT_BM * NT_BN * sizeof(T));
-    if (rc) return rc;
+    if (whole == total) return;
     g.ws = (T*)ws.p;
     g.item0 = whole;
     g.nsplit = rest;
     hipLaunchKernelGGL((nt_gemm_kernel<T, Out, true>), dim3(rest * parts), dim3(256), NT_LDS, s, g, O);
     hipLaunchKernelGGL((nt_fix_kernel<T, Out>), dim3(rest, 4), dim3(256), 0, s, g, parts, O);
-    return OPSEC_OK;
 }
 
 }  // namespace opsec

@@ -1714,10 +1714,10 @@ static int run_project_toeplitz(opsec_ctx* ctx, int nb, const int* funcs) {
 // four rounds of 512 tiles), small next to the stage-1 products themselves.
 constexpr size_t NT_PANEL_BYTES = (size_t)2 << 30;
 
-// Rows of a panel of `row_bytes` each within NT_PANEL_BYTES: all of them, or a
+// Rows of a panel of `row_bytes` each within `panel` bytes: all of them, or a
 // multiple of the tile (at most 32768: the generators' grid).
-static int panel_rows(int rows, size_t row_bytes) {
-    const size_t fit = NT_PANEL_BYTES / row_bytes / NT_BN * NT_BN;
+static int panel_rows(int rows, size_t row_bytes, size_t panel) {
+    const size_t fit = panel / row_bytes / NT_BN * NT_BN;
     return (int)std::min<size_t>(rows, std::max<size_t>(NT_BN, std::min<size_t>(fit, 32768)));
 }
 
@@ -1726,10 +1726,10 @@ static int panel_rows(int rows, size_t row_bytes) {
 // C_p B'^T hold column m of the packed upper triangle as row m, so a tile's rows
 // are contiguous in the output.
 template <typename T>
-static int stage2_nt(opsec_ctx* ctx, NtWork& ws, const T* X, size_t ld, const T* C, size_t cstride, int g, int M, int K,
+static void stage2_nt(opsec_ctx* ctx, NtWork& ws, const T* X, size_t ld, const T* C, size_t cstride, int g, int M, int K,
                      bool serial, double* P) {
     NtArgs<T> A{C, ld, 0, cstride, M, X, ld, 0, 0, M, (int)(nt_kpad<T>(K) / nt_bk<T>()), 1, g, serial};
-    return launch_nt_gemm<T>(ctx, ws, A, NtPacked{P, (size_t)packed_size(M)});
+    launch_nt_gemm<T>(ctx, ws, A, NtPacked{P, (size_t)packed_size(M)});
 }
 
 // Toeplitz projection without operand splitting: FP64 or FP32 MFMA, FP64 DFTs.
@@ -1738,7 +1738,7 @@ static int stage2_nt(opsec_ctx* ctx, NtWork& ws, const T* X, size_t ld, const T*
 // TOEP64_GROUP bands per launch.  Small surveys run stage 1 for several bands
 // per launch as well.
 template <typename T>
-static int run_project_toeplitz_nt(opsec_ctx* ctx, int nb, const int* funcs, int prec) {
+static int run_project_toeplitz_nt(opsec_ctx* ctx, int nb, const int* funcs, int prec, size_t panel) {
     ProjState* ps = ctx->proj;
     ProjState::Toep& tp = ps->toep[std::is_same<T, float>::value];
     const SurveyDev& sv = ctx->sv;
@@ -1756,9 +1756,9 @@ static int run_project_toeplitz_nt(opsec_ctx* ctx, int nb, const int* funcs, int
     const size_t ystride = (size_t)M * ldg, hstride = (size_t)nbat * M * Gp;
     // rows of That_k (all k) per launch; bands per stage-1 launch when all rows fit
     const size_t trow = (size_t)(n1 + 1) * Gp * sizeof(T);
-    const int trows = panel_rows(G, trow);
+    const int trows = panel_rows(G, trow, panel);
     const int sub = trows < G ? 1
-                              : (int)std::max<size_t>(1, std::min<size_t>(grp, NT_PANEL_BYTES / (trow * G + hstride * sizeof(T))));
+                              : (int)std::max<size_t>(1, std::min<size_t>(grp, panel / (trow * G + hstride * sizeof(T))));
     const size_t tstride = (size_t)(n1 + 1) * trows * Gp;
     if ((rc = dev_realloc(ctx, &tp.Yhat, &tp.cap_Yhat, (size_t)sub * hstride * sizeof(T)))) return rc;
     if ((rc = dev_realloc(ctx, &tp.Y, &tp.cap_Y, (size_t)grp * ystride * sizeof(T)))) return rc;
@@ -1832,7 +1832,7 @@ static int run_project_toeplitz_nt(opsec_ctx* ctx, int nb, const int* funcs, int
                 // batch b of band q: Yhat[b] (M x G) = Bhat[b] That_((b+1)/2), columns r0 .. r0 + nr - 1
                 NtArgs<T> A{(const T*)tp.Bhat, Gp, (size_t)M * Gp, 0, M, Tp, Gp, (size_t)nr * Gp, tz, nr,
                             (int)(nt_kpad<T>(G) / nt_bk<T>()), nbat, nbat * ns, serial};
-                if (!rc) rc = launch_nt_gemm<T>(ctx, ps->ws, A, NtRows<T>{(T*)tp.Yhat + r0, Gp, (size_t)M * Gp, hstride, nr, nr});
+                launch_nt_gemm<T>(ctx, ps->ws, A, NtRows<T>{(T*)tp.Yhat + r0, Gp, (size_t)M * Gp, hstride, nr, nr});
             }
             hipLaunchKernelGGL(idft, dim3((unsigned)((G + 255) / 256), (unsigned)M, (unsigned)ns), dim3(256), id_lds,
                                ctx->stream, (const T*)tp.Yhat, nbat, G, Gp, n1, M, ps->d_W64, serial,
@@ -1840,9 +1840,8 @@ static int run_project_toeplitz_nt(opsec_ctx* ctx, int nb, const int* funcs, int
             hipEventRecord(ev[3 * si + 2], ctx->stream);
         }
         hipEventRecord(evg[2 * gi], ctx->stream);
-        if (!rc)
-            rc = stage2_nt<T>(ctx, ps->ws, (const T*)tp.Bg, ldg, (const T*)tp.Y, ystride, g, M, Ng, serial,
-                              (double*)ps->d_P + (size_t)z0 * np);
+        stage2_nt<T>(ctx, ps->ws, (const T*)tp.Bg, ldg, (const T*)tp.Y, ystride, g, M, Ng, serial,
+                     (double*)ps->d_P + (size_t)z0 * np);
         hipEventRecord(evg[2 * gi + 1], ctx->stream);
     }
     hipError_t e = hipGetLastError();
@@ -1881,21 +1880,22 @@ static int run_project_toeplitz_nt(opsec_ctx* ctx, int nb, const int* funcs, int
 // keeps the group's products C_p = T_p B' (N x M each), so a group holds at most
 // DENSE_GROUP_BYTES of them (all 40 bands of the 32^3 box fit; the 50 bands of
 // the 65536-cell shell at 6000 modes take four groups).  Within a group stage 1
-// takes the rows of T_p in panels of NT_PANEL_BYTES (several bands per launch
+// takes the rows of T_p in panels (several bands per launch
 // where their whole T_p fit).  T_p is symmetric: C_p's row m (mode m, cells
 // contiguous) is row m of B' times the rows of T_p.
 constexpr size_t DENSE_GROUP_BYTES = (size_t)48 << 30;
 
 template <typename T>
-static int run_project_dense_nt(opsec_ctx* ctx, int nb, const int* d_funcs, const T* Bw, size_t ldw, int prec) {
+static int run_project_dense_nt(opsec_ctx* ctx, int nb, const int* d_funcs, const T* Bw, size_t ldw, int prec,
+                                size_t panel) {
     ProjState* ps = ctx->proj;
     const int N = ctx->ncells, M = ctx->nmodes;
     const bool serial = serial_sums<T>(ctx->sv);
     const size_t per_band = ldw * M;   // stage-1 products use the same padded pitch as B'
     const int grp = (int)std::max<size_t>(1, std::min<size_t>(nb, DENSE_GROUP_BYTES / (per_band * sizeof(T))));
-    const int Kp = (int)nt_kpad<T>(N), rows = panel_rows(N, ldw * sizeof(T));
+    const int Kp = (int)nt_kpad<T>(N), rows = panel_rows(N, ldw * sizeof(T), panel);
     const size_t tband = (size_t)rows * ldw;
-    const int sub = rows < N ? 1 : (int)std::max<size_t>(1, std::min<size_t>(grp, NT_PANEL_BYTES / (tband * sizeof(T))));
+    const int sub = rows < N ? 1 : (int)std::max<size_t>(1, std::min<size_t>(grp, panel / (tband * sizeof(T))));
     int rc;
     if ((rc = dev_realloc(ctx, &ps->d_C, &ps->cap_C, (size_t)grp * per_band * sizeof(T)))) return rc;
     if ((rc = dev_realloc(ctx, &ps->d_T, &ps->cap_T, (size_t)sub * tband * sizeof(T)))) return rc;
@@ -1919,16 +1919,14 @@ static int run_project_dense_nt(opsec_ctx* ctx, int nb, const int* d_funcs, cons
                                    tband);
                 NtArgs<T> A{Bw, ldw, 0, 0, M, Tp, ldw, 0, tband, nr, Kp / nt_bk<T>(), 1, ns, serial};
                 // the last panel's tiles also write the padding columns of C
-                if (!rc)
-                    rc = launch_nt_gemm<T>(ctx, ps->ws, A,
-                                           NtRows<T>{(T*)ps->d_C + (size_t)q0 * per_band + r0, ldw, 0, per_band, nr,
-                                                     r0 + nr < N ? nr : Kp - r0, serial});
+                launch_nt_gemm<T>(ctx, ps->ws, A,
+                                  NtRows<T>{(T*)ps->d_C + (size_t)q0 * per_band + r0, ldw, 0, per_band, nr,
+                                            r0 + nr < N ? nr : Kp - r0, serial});
             }
         }
         hipEventRecord(ev[2 * gi + 1], ctx->stream);
-        if (!rc)
-            rc = stage2_nt<T>(ctx, ps->ws, Bw, ldw, (const T*)ps->d_C, per_band, g, M, N, serial,
-                              (double*)ps->d_P + (size_t)z0 * np);
+        stage2_nt<T>(ctx, ps->ws, Bw, ldw, (const T*)ps->d_C, per_band, g, M, N, serial,
+                     (double*)ps->d_P + (size_t)z0 * np);
         hipEventRecord(ev[2 * gi + 2], ctx->stream);
     }
     hipError_t e = hipGetLastError();
@@ -1952,16 +1950,17 @@ static int run_project_dense_nt(opsec_ctx* ctx, int nb, const int* d_funcs, cons
     return OPSEC_OK;
 }
 
-// Stage 1 + stage 2 for nb functions (device pair tables), results to d_P.
-static int run_project(opsec_ctx* ctx, int nb, const int* d_funcs, const int* funcs, int prec) {
+// Stage 1 + stage 2 for nb functions (device pair tables), results to d_P, with panels of
+// `panel` bytes.
+static int run_project_panels(opsec_ctx* ctx, int nb, const int* d_funcs, const int* funcs, int prec, size_t panel) {
     ProjState* ps = ctx->proj;
     if (ctx->projection == OPSEC_PROJ_TOEPLITZ) {
         if (prec == OPSEC_PREC_BF16X3) return run_project_toeplitz(ctx, nb, funcs);
-        if (prec == OPSEC_PREC_FP32) return run_project_toeplitz_nt<float>(ctx, nb, funcs, prec);
-        return run_project_toeplitz_nt<double>(ctx, nb, funcs, prec);
+        if (prec == OPSEC_PREC_FP32) return run_project_toeplitz_nt<float>(ctx, nb, funcs, prec, panel);
+        return run_project_toeplitz_nt<double>(ctx, nb, funcs, prec, panel);
     }
     if (prec == OPSEC_PREC_BF16X3) return run_project_bf16x3(ctx, nb, funcs);
-    if (prec == OPSEC_PREC_FP64) return run_project_dense_nt<double>(ctx, nb, d_funcs, ps->d_Bw, ps->ldw, prec);
+    if (prec == OPSEC_PREC_FP64) return run_project_dense_nt<double>(ctx, nb, d_funcs, ps->d_Bw, ps->ldw, prec, panel);
     const size_t ld32 = nt_pitch<float>(ctx->ncells);
     if (!ps->bw32_valid) {
         int rc;
@@ -1972,7 +1971,35 @@ static int run_project(opsec_ctx* ctx, int nb, const int* d_funcs, const int* fu
         OPSEC_HIP_TRY(ctx, hipGetLastError());
         ps->bw32_valid = true;
     }
-    return run_project_dense_nt<float>(ctx, nb, d_funcs, ps->d_Bw32, ld32, prec);
+    return run_project_dense_nt<float>(ctx, nb, d_funcs, ps->d_Bw32, ld32, prec, panel);
+}
+
+// Everything but B' and the results: other projections' operands and work buffers.
+static void free_work(ProjState* ps) {
+    for (void** p : {&ps->d_C, &ps->d_T, &ps->ws.p, (void**)&ps->d_Ppart, (void**)&ps->d_Bp, (void**)&ps->d_Sp,
+                     (void**)&ps->d_Cp, (void**)&ps->d_Qhl, (void**)&ps->d_cpk, (void**)&ps->d_gmap, (void**)&ps->d_Bg,
+                     (void**)&ps->d_Bhat, (void**)&ps->d_That, (void**)&ps->d_Qhat, (void**)&ps->d_Yhat,
+                     (void**)&ps->d_Cg, (void**)&ps->d_trig, (void**)&ps->d_W, (void**)&ps->d_Bw32,
+                     (void**)&ps->d_gmap64, (void**)&ps->d_trig64, (void**)&ps->d_W64})
+        dev_free(p);
+    for (auto& t : ps->toep) {
+        dev_free(&t.Bg);
+        dev_free(&t.Bhat);
+        dev_free(&t.Yhat);
+        dev_free(&t.Y);
+        t.valid = false;
+    }
+    ps->bp_valid = ps->bw32_valid = ps->toep_valid = false;
+}
+
+// Where the memory is not there, once more without the buffers of other projections and with
+// smaller panels (32 MB at last, next to the stage-1 products).
+static int run_project(opsec_ctx* ctx, int nb, const int* d_funcs, const int* funcs, int prec) {
+    for (size_t panel = NT_PANEL_BYTES;; panel /= 4) {
+        const int rc = run_project_panels(ctx, nb, d_funcs, funcs, prec, panel);
+        if (rc != OPSEC_ENOMEM || panel < (size_t)64 << 20) return rc;
+        free_work(ctx->proj);
+    }
 }
 
 // P = B S B^T (packed) of a device matrix S (N x N row-major) and modes B (M x N).
@@ -1986,19 +2013,26 @@ static int project_host_nt(opsec_ctx* ctx, int N, const double* dS, int M, const
     } ws;
     T *X = nullptr, *Bp = nullptr, *Cp = nullptr;
     DevScratch tmp;
-    OPSEC_HIP_TRY(ctx, tmp.alloc(&X, ld * N * sizeof(T)));
     OPSEC_HIP_TRY(ctx, tmp.alloc(&Bp, ld * M * sizeof(T)));
     OPSEC_HIP_TRY(ctx, tmp.alloc(&Cp, ld * M * sizeof(T)));
-    hipLaunchKernelGGL(pad_rows_kernel<T>, strided_blocks(ld * N), dim3(256), 0, ctx->stream, dS, (size_t)N, N, N, serial, X,
-                       ld);
+    // S's padded rows in panels, smaller ones where the memory is not there
+    int rows = panel_rows(N, ld * sizeof(T), NT_PANEL_BYTES);
+    while (tmp.alloc(&X, ld * rows * sizeof(T)) != hipSuccess) {
+        if (rows <= NT_BN) return set_error(ctx, OPSEC_ENOMEM, "projection: no memory for %d rows", rows);
+        rows = (rows / 2 + NT_BN - 1) / NT_BN * NT_BN;
+    }
     hipLaunchKernelGGL(pad_rows_kernel<T>, strided_blocks(ld * M), dim3(256), 0, ctx->stream, dB, (size_t)N, M, N, serial, Bp,
                        ld);
     // C[m][a] = sum_b S[a][b] B[m][b]
-    NtArgs<T> A1{Bp, ld, 0, 0, M, X, ld, 0, 0, N, Kp / nt_bk<T>(), 1, 1, serial};
-    int rc = launch_nt_gemm<T>(ctx, ws, A1, NtRows<T>{Cp, ld, 0, 0, N, Kp, serial});
+    for (int r0 = 0; r0 < N; r0 += rows) {
+        const int nr = std::min(rows, N - r0);
+        hipLaunchKernelGGL(pad_rows_kernel<T>, strided_blocks(ld * nr), dim3(256), 0, ctx->stream, dS + (size_t)r0 * N,
+                           (size_t)N, nr, N, serial, X, ld);
+        NtArgs<T> A1{Bp, ld, 0, 0, M, X, ld, 0, 0, nr, Kp / nt_bk<T>(), 1, 1, serial};
+        launch_nt_gemm<T>(ctx, ws, A1, NtRows<T>{Cp + r0, ld, 0, 0, nr, r0 + nr < N ? nr : Kp - r0, serial});
+    }
     // P[i][j] = sum_a B[i][a] C[j][a], i <= j
-    if (!rc) rc = stage2_nt<T>(ctx, ws, Bp, ld, Cp, 0, 1, M, N, serial, dP);
-    if (rc) return rc;
+    stage2_nt<T>(ctx, ws, Bp, ld, Cp, 0, 1, M, N, serial, dP);
     OPSEC_HIP_TRY(ctx, hipGetLastError());
     OPSEC_HIP_TRY(ctx, hipStreamSynchronize(ctx->stream));
     return OPSEC_OK;
@@ -2021,36 +2055,9 @@ void invalidate_modes(opsec_ctx* ctx) {
 
 void free_proj(opsec_ctx* ctx) {
     if (!ctx->proj) return;
+    free_work(ctx->proj);
     dev_free((void**)&ctx->proj->d_Bw);
-    dev_free(&ctx->proj->d_C);
     dev_free(&ctx->proj->d_P);
-    dev_free((void**)&ctx->proj->d_Bp);
-    dev_free((void**)&ctx->proj->d_Sp);
-    dev_free((void**)&ctx->proj->d_Cp);
-    dev_free((void**)&ctx->proj->d_Qhl);
-    dev_free((void**)&ctx->proj->d_Ppart);
-    dev_free((void**)&ctx->proj->d_cpk);
-    dev_free((void**)&ctx->proj->d_gmap);
-    dev_free((void**)&ctx->proj->d_Bg);
-    dev_free((void**)&ctx->proj->d_Bhat);
-    dev_free((void**)&ctx->proj->d_That);
-    dev_free((void**)&ctx->proj->d_Qhat);
-    dev_free((void**)&ctx->proj->d_Yhat);
-    dev_free((void**)&ctx->proj->d_Cg);
-    dev_free((void**)&ctx->proj->d_trig);
-    dev_free((void**)&ctx->proj->d_W);
-    dev_free((void**)&ctx->proj->d_gmap64);
-    dev_free((void**)&ctx->proj->d_trig64);
-    dev_free((void**)&ctx->proj->d_W64);
-    for (auto& t : ctx->proj->toep) {
-        dev_free(&t.Bg);
-        dev_free(&t.Bhat);
-        dev_free(&t.Yhat);
-        dev_free(&t.Y);
-    }
-    dev_free((void**)&ctx->proj->d_Bw32);
-    dev_free(&ctx->proj->d_T);
-    dev_free(&ctx->proj->ws.p);
     delete ctx->proj;
     ctx->proj = nullptr;
 }

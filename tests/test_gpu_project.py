@@ -575,3 +575,50 @@ def test_results_belong_to_their_modes(ctx):
     ctx.modes_upload(B[:8])
     again = estimate(8)
     assert all(np.array_equal(first[k], again[k]) for k in first)
+
+
+def _fill_device(c, leave):
+    """Allocate the card's memory up to about `leave` bytes (multiples of 64 MB)."""
+    last = []
+    for size in (16 << 30, 4 << 30, 1 << 30, 256 << 20, 64 << 20):
+        while len(last) < 200:
+            try:
+                p = c.dev_alloc(size)
+            except lib.OpsecError:
+                break
+            last.append((size, p))
+    freed = 0
+    for size, p in reversed(last):
+        if freed >= leave:
+            break
+        c.dev_free(p)
+        freed += size
+
+
+@pytest.mark.parametrize("prec,tol", [(lib.OPSEC_PREC_FP64, 1e-12), (lib.OPSEC_PREC_FP32, 2e-5)])
+def test_projection_where_memory_is_short(ctx, prec, tol):
+    """With about 1 GB of the card left the operand panels (2 GB at most) are made smaller, and other
+    projections' buffers given back, instead of the call being refused."""
+    cells = synth.box_cells(96, 0.0, 960.0)
+    cells = cells[cells["d1"] < 4].copy()
+    cells["a"] = np.arange(len(cells))
+    sv = lib.survey_box(96, 0.0, 960.0, L=1e9)
+    sv.n1, sv.max1 = 4, 40.0
+    B = np.random.default_rng(5).normal(size=(24, len(cells)))
+
+    def setup(c):
+        c.model_real(GOLD["pk_k"], GOLD["pk_P"], [0.02], [0.03], lib.OPSEC_XI_CLOSED)
+        c.cells_upload(cells, sv)
+        c.pair_tables([1], c.quad(lib.OPSEC_QUAD_GAUSS, nodes=4, near=1))
+        c.modes_upload(B)
+
+    with lib.Context(0) as c:
+        setup(c)
+        ref = c.project([1], lib.OPSEC_PREC_FP64)[0]
+    with lib.Context(0) as c, lib.Context(0) as filler:
+        setup(c)
+        _fill_device(filler, 1 << 30)
+        for proj in (lib.OPSEC_PROJ_TOEPLITZ, lib.OPSEC_PROJ_DENSE):
+            c.set_projection(proj)
+            got = c.project([1], prec)[0]
+            assert np.abs(got - ref).max() <= tol * np.abs(ref).max()
