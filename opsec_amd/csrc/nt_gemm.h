@@ -83,16 +83,21 @@ struct NtArgs {
     T* ws = nullptr;       // split-K launch: the parts' accumulators
 };
 
-// Epilogues: base(band, b), then put(base, m, n, M, value).
-template <typename T>
-struct NtRows {              // C[m * ld + n], n < nc, then zeros up to nw; serial: in that order
+// Epilogues: base(band, b), then put(base, m, n, M, value), or put_in where inside(m0, n0, M)
+// says that the whole tile is there (with put's tests and their loads for every element a
+// tile of 209 k-steps took 1.8 % longer).
+template <typename T, bool SERIAL>
+struct NtRows {              // C[m * ld + n], n < nc, then zeros up to nw; SERIAL: in that order
     T* p;
     size_t ld, b_stride, q_stride;
     int nc, nw;
-    bool serial = false;
     __device__ __forceinline__ T* base(int q, int b) const { return p + q * q_stride + b * b_stride; }
+    __device__ __forceinline__ bool inside(int m0, int n0, int M) const { return m0 + NT_BM <= M && n0 + NT_BN <= nc; }
+    __device__ __forceinline__ void put_in(T* o, int m, int n, T v) const {
+        o[(size_t)m * ld + (SERIAL ? nt_serial(n) : n)] = v;
+    }
     __device__ __forceinline__ void put(T* o, int m, int n, int M, T v) const {
-        if (m < M && n < nw) o[(size_t)m * ld + (serial ? nt_serial(n) : n)] = n < nc ? v : (T)0;
+        if (m < M && n < nw) o[(size_t)m * ld + (SERIAL ? nt_serial(n) : n)] = n < nc ? v : (T)0;
     }
     static constexpr bool lower = false;
 };
@@ -100,6 +105,10 @@ struct NtPacked {            // P[m (m + 1) / 2 + n] for n <= m: column m of a p
     double* p;
     size_t q_stride;
     __device__ __forceinline__ double* base(int q, int) const { return p + q * q_stride; }
+    __device__ __forceinline__ bool inside(int m0, int n0, int M) const { return m0 + NT_BM <= M && n0 + NT_BN <= m0 + 1; }
+    __device__ __forceinline__ void put_in(double* o, int m, int n, double v) const {
+        o[(size_t)m * (m + 1) / 2 + n] = v;
+    }
     __device__ __forceinline__ void put(double* o, int m, int n, int M, double v) const {
         if (m < M && n <= m) o[(size_t)m * (m + 1) / 2 + n] = v;
     }
@@ -272,13 +281,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
                 for (int r = 0; r < 4; r++) o[((i * 4 + j) * 4 + r) * 256] = acc[i][j][r];
     } else {
         auto* o = O.base(q, b);
+        const bool in = O.inside(m0, n0, g.M);
 #pragma unroll
         for (int i = 0; i < 4; i++)
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int n = n0 + wn + j * 16 + fr;
+            for (int r = 0; r < 4; r++) {
+                const int m = m0 + wm + i * 16 + acc_row<T>(lane, r), n = n0 + wn + fr;
+                if (in) {
 #pragma unroll
-                for (int r = 0; r < 4; r++) O.put(o, m0 + wm + i * 16 + acc_row<T>(lane, r), n, g.M, acc[i][j][r]);
+                    for (int j = 0; j < 4; j++) O.put_in(o, m, n + j * 16, acc[i][j][r]);
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; j++) O.put(o, m, n + j * 16, g.M, acc[i][j][r]);
+                }
             }
     }
 }
@@ -359,6 +374,14 @@ inline void launch_nt_gemm(opsec_ctx* ctx, NtWork& ws, NtArgs<T> g, const Out& O
     g.nsplit = rest;
     hipLaunchKernelGGL((nt_gemm_kernel<T, Out, true>), dim3(rest * parts), dim3(256), NT_LDS, s, g, O);
     hipLaunchKernelGGL((nt_fix_kernel<T, Out>), dim3(rest, 4), dim3(256), 0, s, g, parts, O);
+}
+// The same into rows that are an operand of the next product, in g's order.
+template <typename T>
+inline void launch_nt_gemm_rows(opsec_ctx* ctx, NtWork& ws, const NtArgs<T>& g, T* p, size_t ld, size_t q_stride, int nc,
+                                int nw) {
+    if constexpr (sizeof(T) == 4)
+        if (g.serial) return launch_nt_gemm(ctx, ws, g, NtRows<T, true>{p, ld, 0, q_stride, nc, nw});
+    launch_nt_gemm(ctx, ws, g, NtRows<T, false>{p, ld, 0, q_stride, nc, nw});
 }
 
 }  // namespace opsec

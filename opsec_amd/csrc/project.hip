@@ -130,10 +130,10 @@ static bool serial_sums(const SurveyDev& sv) {
 // out[z][i][c] = Q_f[key(row0 + i, c)], f = funcs[z], i < nrows, c < N; zero for N <= c < Kp.
 // Tile of 8 rows x 512 columns per 256-thread block, two columns per thread; the
 // column coordinates in LDS.
-template <typename T>
+template <typename T, bool SERIAL>
 __global__ __launch_bounds__(256) void gen_rows_kernel(const double* __restrict__ Q, size_t qstride,
                                                        const int* __restrict__ funcs, const int* __restrict__ cellidx,
-                                                       PairKey K, int N, int row0, int nrows, int Kp, bool serial,
+                                                       PairKey K, int N, int row0, int nrows, int Kp,
                                                        T* __restrict__ out, size_t ld, size_t zstride) {
     __shared__ int cx[512], cy[512], cz[512];
     const int j0 = blockIdx.x * 512, i0 = blockIdx.y * 8;
@@ -148,7 +148,7 @@ __global__ __launch_bounds__(256) void gen_rows_kernel(const double* __restrict_
     T* o = out + (size_t)blockIdx.z * zstride;
     const int t = 2 * threadIdx.x, j = j0 + t;
     if (j >= Kp) return;
-    const int t0 = serial ? nt_serial(t) : t, t1 = serial ? nt_serial(t + 1) : t + 1;   // the columns stored at j, j + 1
+    const int t0 = SERIAL ? nt_serial(t) : t, t1 = SERIAL ? nt_serial(t + 1) : t + 1;   // the columns stored at j, j + 1
     typedef T pair_t __attribute__((ext_vector_type(2)));
 #pragma unroll
     for (int r = 0; r < 8; r++) {
@@ -1832,7 +1832,7 @@ static int run_project_toeplitz_nt(opsec_ctx* ctx, int nb, const int* funcs, int
                 // batch b of band q: Yhat[b] (M x G) = Bhat[b] That_((b+1)/2), columns r0 .. r0 + nr - 1
                 NtArgs<T> A{(const T*)tp.Bhat, Gp, (size_t)M * Gp, 0, M, Tp, Gp, (size_t)nr * Gp, tz, nr,
                             (int)(nt_kpad<T>(G) / nt_bk<T>()), nbat, nbat * ns, serial};
-                launch_nt_gemm<T>(ctx, ps->ws, A, NtRows<T>{(T*)tp.Yhat + r0, Gp, (size_t)M * Gp, hstride, nr, nr});
+                launch_nt_gemm<T>(ctx, ps->ws, A, NtRows<T, false>{(T*)tp.Yhat + r0, Gp, (size_t)M * Gp, hstride, nr, nr});
             }
             hipLaunchKernelGGL(idft, dim3((unsigned)((G + 255) / 256), (unsigned)M, (unsigned)ns), dim3(256), id_lds,
                                ctx->stream, (const T*)tp.Yhat, nbat, G, Gp, n1, M, ps->d_W64, serial,
@@ -1907,21 +1907,22 @@ static int run_project_dense_nt(opsec_ctx* ctx, int nb, const int* d_funcs, cons
     results_begin(ps);
     hipEventRecord(ev[0], ctx->stream);
     T* Tp = (T*)ps->d_T;
+    auto gen = gen_rows_kernel<T, false>;
+    if constexpr (std::is_same<T, float>::value)
+        if (serial) gen = gen_rows_kernel<T, true>;
     for (int gi = 0; gi < ngroups; gi++) {
         const int z0 = gi * grp, g = std::min(grp, nb - z0);
         for (int q0 = 0; q0 < g; q0 += sub) {
             const int ns = std::min(sub, g - q0);
             for (int r0 = 0; r0 < N; r0 += rows) {
                 const int nr = std::min(rows, N - r0);
-                hipLaunchKernelGGL(gen_rows_kernel<T>, dim3((unsigned)((Kp + 511) / 512), (unsigned)((nr + 7) / 8), ns),
+                hipLaunchKernelGGL(gen, dim3((unsigned)((Kp + 511) / 512), (unsigned)((nr + 7) / 8), ns),
                                    dim3(256), 0, ctx->stream, ctx->d_Q, (size_t)ctx->nkeys, d_funcs + z0 + q0,
-                                   ctx->d_cellidx, pair_key_of(ctx->sv), N, r0, nr, Kp, serial, Tp, ldw,
-                                   tband);
+                                   ctx->d_cellidx, pair_key_of(ctx->sv), N, r0, nr, Kp, Tp, ldw, tband);
                 NtArgs<T> A{Bw, ldw, 0, 0, M, Tp, ldw, 0, tband, nr, Kp / nt_bk<T>(), 1, ns, serial};
                 // the last panel's tiles also write the padding columns of C
-                launch_nt_gemm<T>(ctx, ps->ws, A,
-                                  NtRows<T>{(T*)ps->d_C + (size_t)q0 * per_band + r0, ldw, 0, per_band, nr,
-                                            r0 + nr < N ? nr : Kp - r0, serial});
+                launch_nt_gemm_rows<T>(ctx, ps->ws, A, (T*)ps->d_C + (size_t)q0 * per_band + r0, ldw, per_band, nr,
+                                       r0 + nr < N ? nr : Kp - r0);
             }
         }
         hipEventRecord(ev[2 * gi + 1], ctx->stream);
@@ -2029,7 +2030,7 @@ static int project_host_nt(opsec_ctx* ctx, int N, const double* dS, int M, const
         hipLaunchKernelGGL(pad_rows_kernel<T>, strided_blocks(ld * nr), dim3(256), 0, ctx->stream, dS + (size_t)r0 * N,
                            (size_t)N, nr, N, serial, X, ld);
         NtArgs<T> A1{Bp, ld, 0, 0, M, X, ld, 0, 0, nr, Kp / nt_bk<T>(), 1, 1, serial};
-        launch_nt_gemm<T>(ctx, ws, A1, NtRows<T>{Cp + r0, ld, 0, 0, nr, r0 + nr < N ? nr : Kp - r0, serial});
+        launch_nt_gemm_rows<T>(ctx, ws, A1, Cp + r0, ld, 0, nr, r0 + nr < N ? nr : Kp - r0);
     }
     // P[i][j] = sum_a B[i][a] C[j][a], i <= j
     stage2_nt<T>(ctx, ws, Bp, ld, Cp, 0, 1, M, N, serial, dP);
