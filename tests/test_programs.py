@@ -92,6 +92,8 @@ def test_modefile_read_by_reference_reader(tmp_path):
     klt output layout; with fewer converged modes the reference's own header
     (n = nconv Ncells, Nmodes from the config, src/klt.cpp:210-225) is
     rejected by its own reader, which is why klt writes all Nmodes vectors."""
+    if not O.ref_available():
+        pytest.skip("reference build not present")
     R = O.ref()
     N, M = 50, 7
     rng = np.random.default_rng(3)
@@ -188,14 +190,15 @@ def test_pipeline_end_to_end_vs_oracle(tmp_path):
     assert eopts["Nmodes"] == str(M) and eopts["Ncells"] == str(N) and int(eopts["nconv"]) == M
     _, (modes,) = formats.read_doubles(tmp_path / "modes.abn")
     B = modes.reshape(M, N)
-    # the reference's own readers accept klt's files (src/sig.cpp:621-697, src/abn.c)
-    got = np.zeros(M * N)
-    nc = C.c_int()
-    assert O.ref().ref_read_modes(str(tmp_path / "modes.abn").encode(), C.byref(nc), O.ptr(got), got.size) == M
-    assert nc.value == N and np.array_equal(got, modes)
-    gl = np.zeros(M)
-    assert O.ref().ref_read_abn_doubles(str(tmp_path / "evals.abn").encode(), O.ptr(gl), M) == M
-    assert np.array_equal(gl, lam)
+    # the reference's own readers accept klt's files (src/sig.cpp:621-697, src/abn.c), where they are built
+    if O.ref_available():
+        got = np.zeros(M * N)
+        nc = C.c_int()
+        assert O.ref().ref_read_modes(str(tmp_path / "modes.abn").encode(), C.byref(nc), O.ptr(got), got.size) == M
+        assert nc.value == N and np.array_equal(got, modes)
+        gl = np.zeros(M)
+        assert O.ref().ref_read_abn_doubles(str(tmp_path / "evals.abn").encode(), O.ptr(gl), M) == M
+        assert np.array_equal(gl, lam)
     # oracle S and its spectrum
     lo, hi = synth.linear_bands(nb, 0.02, 0.14)
     r768, tabs = O.oracle_tables(kP[:, 0], kP[:, 1], lo, hi)
