@@ -119,9 +119,10 @@ struct ProjState {
 // FP32 operands may be in nt_gemm.h's serial order (`serial`): column c of a row is then
 // stored at nt_serial(c).  It keeps the sums of a shell's FP32 projection, and of a given
 // matrix's, the plain chains over k, the same bits whatever the number of bands in a call
-// or of CUs.  A box's FP32 sums are not ordered: split over K where that pays, they are
-// nearer to the 64-bit product (a 6686-cell footprint with 777 modes: 6.6e-7 of the norm,
-// 1.5e-6 in the serial order).
+// or of CUs, and those of results stored earlier.  A box's FP32 sums are not ordered: split
+// over K where that pays, they are nearer to the 64-bit product (a 6686-cell footprint with
+// 777 modes: 6.6e-7 of the norm, 1.4e-6 in the serial order; eight shells, serial, 3e-7 to
+// 9e-7, otherwise 1e-7 to 4e-7).
 template <typename T>
 static bool serial_sums(const SurveyDev& sv) {
     return std::is_same<T, float>::value && sv.coordsys == OPSEC_COORD_SPHERICAL;
