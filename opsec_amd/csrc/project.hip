@@ -122,7 +122,8 @@ struct ProjState {
 // or of CUs, and those of results stored earlier.  A box's FP32 sums are not ordered: split
 // over K where that pays, they are nearer to the 64-bit product (a 6686-cell footprint with
 // 777 modes: 6.6e-7 of the norm, 1.4e-6 in the serial order; eight shells, serial, 3e-7 to
-// 9e-7, otherwise 1e-7 to 4e-7).
+// 9e-7, otherwise 1e-7 to 4e-7) and their last round of tiles is faster: six bands of an
+// 8192-cell shell on 750 modes take 6.7 ms dense and 3.1 Toeplitz, split 6.4 and 2.4.
 template <typename T>
 static bool serial_sums(const SurveyDev& sv) {
     return std::is_same<T, float>::value && sv.coordsys == OPSEC_COORD_SPHERICAL;
