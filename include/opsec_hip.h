@@ -329,7 +329,8 @@ typedef struct opsec_estimate {
 int opsec_estimate_run(opsec_ctx* ctx, int nmodes, int nparams, const double* lambda,
                        const double* D, const double* y, const double* prior, int mixing,
                        int prec, opsec_estimate* out);
-/* Same, with D = the device results of the last opsec_project call. */
+/* Same, with D = the device results of the last opsec_project call (OPSEC_ESTATE
+ * where there are none, or modes of another number were uploaded since). */
 int opsec_estimate_device(opsec_ctx* ctx, const double* lambda, const double* y,
                           const double* prior, int mixing, int prec, opsec_estimate* out);
 
